@@ -125,22 +125,42 @@ __global__ void k_gather_rows(const uint32_t* __restrict__ in, uint64_t pitch, c
   }
 }
 
-// One thread per row, in code order.
-__global__ void k_missing_lists(const uint32_t* __restrict__ x, uint64_t pitch, uint64_t nrows, uint64_t ncodes,
-                                const uint64_t* __restrict__ rp, uint32_t* __restrict__ ix) {
-  const uint64_t r = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-  if (r >= nrows) return;
+// The code-01 entries of every row, in code order: one wave per row, 64 words
+// (1,024 codes) per step, each lane's place from an exclusive scan of the
+// lanes' counts.  Bound by the row reads (N M / 4 bytes).  One thread per row,
+// had every load of a wave on 64 different rows: 6.67 ms per list
+// of 20,011 x 200,003 codes, 1 % missing, against 0.62 ms now.
+__global__ void __launch_bounds__(256) k_missing_lists(const uint32_t* __restrict__ x, uint64_t pitch, uint64_t nrows,
+                                                       uint64_t ncodes, const uint64_t* __restrict__ rp,
+                                                       uint32_t* __restrict__ ix) {
+  const uint64_t r = blockIdx.x * 4ull + threadIdx.x / 64;
+  const int lane = threadIdx.x & 63;
+  if (r >= nrows) return;  // wave-uniform
   const uint32_t* row = x + r * pitch;
   uint64_t o = rp[r];
+  if (o == rp[r + 1]) return;
   const uint64_t nw = (ncodes + 15) / 16;
-  for (uint64_t w = 0; w < nw; ++w) {
-    const uint32_t v = row[w];
-    const uint32_t m = v & ~(v >> 1) & 0x55555555u;
-    if (!m) continue;
-    for (int e = 0; e < 16; ++e) {
-      const uint64_t k = w * 16 + e;
-      if (k < ncodes && ((m >> ipos(e)) & 1u)) ix[o++] = (uint32_t)k;
+  for (uint64_t w0 = 0; w0 < nw; w0 += 64) {
+    const uint64_t w = w0 + lane;
+    uint32_t m = 0;
+    if (w < nw) {
+      const uint32_t v = row[w];
+      m = v & ~(v >> 1) & 0x55555555u;  // bit 2t + 8b: code 4t + b of the word
     }
+    uint32_t bits = 0;  // bit e: code e
+#pragma unroll
+    for (int t = 0; t < 4; ++t) bits |= ((((m >> (2 * t)) & 0x01010101u) * 0x01020408u) >> 24) << (4 * t);
+    if (w < nw && (w + 1) * 16 > ncodes) bits &= (1u << (ncodes - w * 16)) - 1u;  // 1..15 codes left
+    if (!__any(bits != 0)) continue;
+    const uint32_t n = __popc(bits);
+    uint32_t s = n;
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t y = __shfl_up(s, d);
+      if (lane >= d) s += y;
+    }
+    uint64_t p = o + (s - n);
+    for (; bits; bits &= bits - 1) ix[p++] = (uint32_t)(w * 16) + (uint32_t)__builtin_ctz(bits);
+    o += __shfl(s, 63);
   }
 }
 
@@ -257,8 +277,8 @@ void launch_deinterleave(const uint32_t* x, uint64_t pitch, uint64_t nrows, uint
 void launch_missing_lists(const uint32_t* x, uint64_t pitch, uint64_t nrows, uint64_t ncodes, const uint64_t* rp,
                           uint32_t* ix, hipStream_t s) {
   if (!nrows) return;
-  hipLaunchKernelGGL(k_missing_lists, dim3((unsigned)((nrows + 255) / 256)), dim3(256), 0, s, x, pitch, nrows, ncodes,
-                     rp, ix);
+  hipLaunchKernelGGL(k_missing_lists, dim3((unsigned)((nrows + 3) / 4)), dim3(256), 0, s, x, pitch, nrows, ncodes, rp,
+                     ix);
   check_launch("missing_lists");
 }
 

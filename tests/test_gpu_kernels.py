@@ -1,0 +1,80 @@
+"""Single kernels of the device path at the sizes where their tiles, remainders and scans can go wrong."""
+import numpy as np
+import pytest
+
+from pcaone_amd import api
+
+pytestmark = pytest.mark.gpu
+
+CODE_VALUE = np.array([1.0, 0.0, 0.5, 0.0])  # BED2GENO (code 01 missing)
+
+
+def say(msg):
+    print(msg, flush=True)
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = api.Context(0)
+    yield c
+    c.close()
+
+
+def pack(codes):
+    m, n = codes.shape
+    out = np.zeros((m, (n + 3) // 4), dtype=np.uint8)
+    for e in range(4):
+        sub = codes[:, e::4].astype(np.uint8)
+        out[:, : sub.shape[1]] |= sub << (2 * e)
+    return out
+
+
+def random_codes(rng, m, n, miss):
+    codes = rng.choice([0, 2, 3], (m, n))
+    codes[rng.random((m, n)) < miss] = 1
+    return codes
+
+
+def standardized(codes):
+    """The matrix of the products (rows = SNPs) in FP64, centered, scaled, missing entries 0, and the scales."""
+    seen = codes != 1
+    x = CODE_VALUE[codes]
+    cnt = seen.sum(1)
+    F = np.divide(x.sum(1), cnt, out=np.zeros(len(x)), where=cnt > 0)
+    sd = np.sqrt(F * (1 - F))
+    sc = np.where(sd > 1e-9, np.sqrt(2.0) / np.where(sd > 1e-9, sd, 1.0), 1.0)
+    return np.where(seen, (x - F[:, None]) * sc[:, None], 0.0), sc
+
+
+@pytest.mark.parametrize("n,m,miss", [(17, 33, 0.5), (63, 1025, 0.1), (64, 1024, 0.02), (1025, 65, 0.3),
+                                      (2049, 1023, 0.01), (4100, 40, 1.0)])
+def test_missing_lists(ctx, n, m, miss):
+    """Products with missing genotypes in FP64 against the dense matrix: every entry of both lists counts.
+    Rows without a missing entry and rows with nothing else are among them."""
+    say(f"missing lists n={n} m={m} miss={miss}")
+    rng = np.random.default_rng(n + m)
+    codes = random_codes(rng, m, n, miss)
+    codes[0] = rng.choice([0, 2, 3], n)
+    codes[m // 2] = 1
+    codes[:, n // 3] = 1
+    codes[m - 1, n - 1] = 1
+    L = 16
+    omega = rng.standard_normal((n, L))
+    ctx.upload_packed(pack(codes), n)
+    assert ctx.dims() == (n, m, int((codes == 1).sum()))
+    ctx.standardize()
+    ctx.configure("fp64", L)
+    ctx.set_omega(omega)
+    ctx.sketch(0, m, 0)
+    A, sc = standardized(codes)
+    G = A @ omega
+    H = A.T @ G
+    # The device sums sc (v / 4) w, sc (1/2 - F) w and, per missing entry, the latter taken back: each entry
+    # counts at most sc (1/2 + 1/2 + 1/2) |w|, also where the row has nothing but missing entries.  n (m) FP64
+    # sums of such terms, a handful of operations each.
+    u = 8 * 2.0**-53
+    g_terms = 1.5 * sc[:, None] * np.abs(omega).sum(0)
+    g_bound = u * n * g_terms
+    assert (np.abs(ctx.get_g(0, m, L) - G) / g_bound).max() <= 1.0
+    h_bound = u * m * 1.5 * (sc @ np.abs(G)) + 1.5 * (sc @ g_bound)
+    assert (np.abs(ctx.get_h(0, L) - H) / h_bound).max() <= 1.0
