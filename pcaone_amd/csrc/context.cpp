@@ -1062,12 +1062,10 @@ void Context::omega_from(int src, bool flip) {
     launch_apply(X, small_.get(), N, lp, tmp_n_.get(), stream);
     launch_gram(tmp_n_.get(), nullptr, nullptr, N, lp, red_.get(), red_cap_, g2, stream);
     launch_thinq_second(g2, r1, X, L, lp, small_.get(), lstatus_.get(), stream);
-    launch_apply(X, small_.get(), N, lp, omega_c_.get(), stream);
     if (flip) {  // flipOmg (src/RSVD.hpp:80-89) against Omg2
-      double* norms = red_.get() + red_cap_;
-      launch_flip_norms(omega_.get(), omega_c_.get(), N, lp, red_.get(), norms, stream);
-      launch_flip_signs(norms, L, lp, dsign, stream);
+      launch_apply_flip(X, small_.get(), N, L, lp, omega_c_.get(), omega_.get(), red_.get(), dsign, stream);
     } else {
+      launch_apply(X, small_.get(), N, lp, omega_c_.get(), stream);
       dsign = nullptr;
     }
     if (form_colscaled(form_g))
@@ -1095,19 +1093,12 @@ void Context::omega_from(int src, bool flip) {
   for (int i = 0; i < L; ++i)
     for (int j = 0; j < L; ++j) T(i, j) *= s[j];
   set_t(T);
-  launch_apply(X, small_.get(), N, lp, omega_c_.get(), stream);
   double* dsign = nullptr;
   if (flip) {  // flipOmg (src/RSVD.hpp:80-89) against Omg2
-    double* norms = red_.get() + red_cap_;
-    launch_flip_norms(omega_.get(), omega_c_.get(), N, lp, red_.get(), norms, stream);
-    std::vector<double> ab(2 * (size_t)lp);
-    PCAONE_HIP(hipMemcpyAsync(ab.data(), norms, ab.size() * 8, hipMemcpyDeviceToHost, stream));
-    PCAONE_HIP(hipStreamSynchronize(stream));
-    std::vector<double> sign(lp, 1.0);
-    for (int l = 0; l < L; ++l)
-      if (ab[l] > 2.0 * ab[lp + l]) sign[l] = -1.0;
     dsign = small_.get() + 128 * 128;
-    PCAONE_HIP(hipMemcpyAsync(dsign, sign.data(), lp * 8, hipMemcpyHostToDevice, stream));
+    launch_apply_flip(X, small_.get(), N, L, lp, omega_c_.get(), omega_.get(), red_.get(), dsign, stream);
+  } else {
+    launch_apply(X, small_.get(), N, lp, omega_c_.get(), stream);
   }
   if (form_colscaled(form_g))
     launch_col_scales(form_g, omega_c_.get(), N, lp, nullptr, i8max_.get(), i8_scale(0), i8_mul(0), stream);
@@ -1207,7 +1198,7 @@ void Context::omega_householder(bool flip) {
     double* norms = red_.get() + red_cap_;
     launch_flip_norms(omega_.get(), omega_c_.get(), N, lp, red_.get(), norms, stream);
     dsign = small_.get() + 128 * 128;
-    launch_flip_signs(norms, L, lp, dsign, stream);
+    launch_flip_signs(norms, 1, L, lp, dsign, stream);
   }
   if (form_colscaled(form_g))
     launch_col_scales(form_g, omega_c_.get(), N, lp, nullptr, i8max_.get(), i8_scale(0), i8_mul(0), stream);

@@ -89,6 +89,10 @@ void launch_gram(const double* X, const double* T, const double* Y0, uint64_t nr
 uint64_t gram_partial_elems(uint64_t nrows, int lp);
 // Y = X T (rows x lp) for rows [0, nrows); T lp x lp row-major; rows above nrows untouched.
 void launch_apply(const double* X, const double* T, uint64_t nrows, int lp, double* Y, hipStream_t s);
+// The same with flipOmg's column signs of Y against O2 (see launch_flip_signs).
+// partial: 256 x 2 lp scratch.
+void launch_apply_flip(const double* X, const double* T, uint64_t nrows, int n, int lp, double* Y, const double* O2,
+                       double* partial, double* sign, hipStream_t s);
 // flipOmg norms: a[l] = sum_i |O2 - Q|, b[l] = sum_i |O2 + Q|.
 void launch_flip_norms(const double* O2, const double* Q, uint64_t nrows, int lp, double* partial, double* out,
                        hipStream_t s);
@@ -105,9 +109,10 @@ void launch_thinq_first(const double* G1, int n, int lp, double* R1, double* T1,
                         double min_ratio = 0.0);
 void launch_thinq_second(const double* G2, const double* R1, const double* Xtop, int n, int lp, double* T,
                          int* status, hipStream_t s);
-// flipOmg's column signs from the norms of launch_flip_norms: -1 where
-// ab[l] > 2 ab[lp + l] (l < n), else 1 (lp entries).
-void launch_flip_signs(const double* ab, int n, int lp, double* sign, hipStream_t s);
+// flipOmg's column signs from nb partial blocks of the two norms (2 lp values
+// each; launch_flip_norms leaves one): -1 where a[l] > 2 b[l] (l < n), else 1
+// (lp entries).
+void launch_flip_signs(const double* partial, int nb, int n, int lp, double* sign, hipStream_t s);
 // Zero bytes [b0, b0 + n0) and [b1, b1 + n1) of each of `rows` rows of `pitch` bytes.
 void launch_zero_ranges(void* base, uint64_t pitch, uint64_t rows, uint64_t b0, uint64_t n0, uint64_t b1, uint64_t n1,
                         hipStream_t s);

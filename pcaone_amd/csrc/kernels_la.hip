@@ -644,15 +644,27 @@ __global__ void __launch_bounds__(64 * NB) k_gram_mfma(const double* __restrict_
 // FP64-MFMA right multiplication Y = X T for rows [0, nrows): one wave per 16
 // rows computes all NB column blocks; A = X (lane l: X[16i + l%16][k0 + l/16]),
 // B = T (lane l: T[k0 + l/16][16b + l%16]).  T is staged in LDS.
-template <int NB>
+// FLIP: also this block's flipOmg norms of the Y it holds in registers,
+// sum |O2 - Y| and sum |O2 + Y| per column, into partial[block][2 LP].  A pass
+// of their own over O2 and Y, in blocks of 128 threads that walked their rows
+// one after another, took 23-34 us and two reductions behind it per Omega
+// update at N = 10,000-50,000; the norms add 3 us (L = 40, N = 10,000) to 12 us
+// (L = 80, N = 50,000) to the product.
+template <int NB, bool FLIP>
 __global__ void __launch_bounds__(256) k_apply_mfma(const double* __restrict__ X, const double* __restrict__ T,
-                                                    uint64_t nrows, double* __restrict__ Y) {
+                                                    uint64_t nrows, double* __restrict__ Y,
+                                                    const double* __restrict__ O2, double* __restrict__ partial) {
   constexpr int LP = NB * 16;
   extern __shared__ double tl[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int q = lane >> 4, r16 = lane & 15;
   for (int v = tid; v < LP * LP; v += 256) tl[v] = T[v];
   __syncthreads();
+  double fa[FLIP ? NB : 1], fb[FLIP ? NB : 1];
+  if constexpr (FLIP) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) fa[b] = fb[b] = 0.0;
+  }
   const uint64_t nblk = (nrows + 15) / 16;
   for (uint64_t blk = (uint64_t)blockIdx.x * 4 + wave; blk < nblk; blk += (uint64_t)gridDim.x * 4) {
     const uint64_t row = blk * 16 + r16;
@@ -675,8 +687,36 @@ __global__ void __launch_bounds__(256) k_apply_mfma(const double* __restrict__ X
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const uint64_t orow = blk * 16 + q + 4 * r;
-        if (orow < nrows) Y[orow * LP + 16 * b + r16] = acc[b][r];
+        if (orow < nrows) {
+          Y[orow * LP + 16 * b + r16] = acc[b][r];
+          if constexpr (FLIP) {
+            const double o = O2[orow * LP + 16 * b + r16];
+            fa[b] += fabs(o - acc[b][r]);
+            fb[b] += fabs(o + acc[b][r]);
+          }
+        }
       }
+  }
+  if constexpr (FLIP) {
+    __syncthreads();  // T has been read: its LDS takes the waves' sums, [wave][2 LP] (8 LP <= LP LP values)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      fa[b] += __shfl_xor(fa[b], 16);
+      fa[b] += __shfl_xor(fa[b], 32);
+      fb[b] += __shfl_xor(fb[b], 16);
+      fb[b] += __shfl_xor(fb[b], 32);
+      if (q == 0) {
+        tl[wave * 2 * LP + 16 * b + r16] = fa[b];
+        tl[wave * 2 * LP + LP + 16 * b + r16] = fb[b];
+      }
+    }
+    __syncthreads();
+    for (int t = tid; t < 2 * LP; t += 256) {
+      double sum = 0.0;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) sum += tl[w * 2 * LP + t];
+      partial[(uint64_t)blockIdx.x * 2 * LP + t] = sum;
+    }
   }
 }
 
@@ -1338,10 +1378,27 @@ __global__ void __launch_bounds__(kSmallThreads) k_thinq_second(const double* __
 }
 
 // flipOmg's decision (src/RSVD.hpp:80-89): column l flips when
-// sum |Omg2 - Q| > 2 sum |Omg2 + Q| (ab = the two norms, 2 x lp).
-__global__ void k_flip_signs(const double* __restrict__ ab, int n, int lp, double* __restrict__ sign) {
+// sum |Omg2 - Q| > 2 sum |Omg2 + Q|.  partial: nb blocks of the two norms
+// (2 lp values each), summed here by one workgroup.
+__global__ void __launch_bounds__(1024) k_flip_signs(const double* __restrict__ partial, int nb, int n, int lp,
+                                                     double* __restrict__ sign) {
+  __shared__ double red[1024];
+  const int w = 2 * lp, G = 1024 / w;
+  const int col = threadIdx.x % w, g = threadIdx.x / w;
+  double s = 0.0;
+  if (g < G) {
+#pragma unroll 4
+    for (int b = g; b < nb; b += G) s += partial[(uint64_t)b * w + col];
+  }
+  red[threadIdx.x] = s;
+  __syncthreads();
+  if (g == 0) {
+    for (int r = 1; r < G; ++r) s += red[r * w + col];
+    red[col] = s;
+  }
+  __syncthreads();
   const int l = threadIdx.x;
-  if (l < lp) sign[l] = (l < n && ab[l] > 2.0 * ab[lp + l]) ? -1.0 : 1.0;
+  if (l < lp) sign[l] = (l < n && red[l] > 2.0 * red[lp + l]) ? -1.0 : 1.0;
 }
 
 // out[r][l] += sum_z partial[z][r][l] (z in order), l < ncols.
@@ -1631,35 +1688,54 @@ void launch_gram(const double* X, const double* T, const double* Y0, uint64_t nr
   check_launch("gram_sum");
 }
 
-template <int NB>
-static void apply_nb(const double* X, const double* T, uint64_t nrows, double* Y, hipStream_t s) {
+// Blocks of the product with the flipOmg norms: their partials are summed by
+// one workgroup, so no more of them than CUs.
+constexpr uint64_t kFlipBlocks = 256;
+
+template <int NB, bool FLIP>
+static unsigned apply_nb(const double* X, const double* T, uint64_t nrows, double* Y, const double* O2,
+                         double* partial, hipStream_t s) {
   constexpr size_t lds = (size_t)NB * 16 * NB * 16 * sizeof(double);
   static bool attr = false;
   if (!attr) {
-    PCAONE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_apply_mfma<NB>),
+    PCAONE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_apply_mfma<NB, FLIP>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr = true;
   }
   const uint64_t nblk = (nrows + 15) / 16;
-  uint64_t g = (nblk + 3) / 4;
-  if (g > 4096) g = 4096;
-  hipLaunchKernelGGL((k_apply_mfma<NB>), dim3((unsigned)g), dim3(256), lds, s, X, T, nrows, Y);
+  const unsigned g = (unsigned)std::min<uint64_t>((nblk + 3) / 4, FLIP ? kFlipBlocks : 4096);
+  hipLaunchKernelGGL((k_apply_mfma<NB, FLIP>), dim3(g), dim3(256), lds, s, X, T, nrows, Y, O2, partial);
+  return g;
+}
+
+template <bool FLIP>
+static unsigned apply_lp(const double* X, const double* T, uint64_t nrows, int lp, double* Y, const double* O2,
+                         double* partial, hipStream_t s) {
+  require(lp <= 128 && lp % 16 == 0 && lp >= 16, kErrArgument, "apply: bad lp");
+  unsigned g = 0;
+  switch (lp / 16) {
+    case 1: g = apply_nb<1, FLIP>(X, T, nrows, Y, O2, partial, s); break;
+    case 2: g = apply_nb<2, FLIP>(X, T, nrows, Y, O2, partial, s); break;
+    case 3: g = apply_nb<3, FLIP>(X, T, nrows, Y, O2, partial, s); break;
+    case 4: g = apply_nb<4, FLIP>(X, T, nrows, Y, O2, partial, s); break;
+    case 5: g = apply_nb<5, FLIP>(X, T, nrows, Y, O2, partial, s); break;
+    case 6: g = apply_nb<6, FLIP>(X, T, nrows, Y, O2, partial, s); break;
+    case 7: g = apply_nb<7, FLIP>(X, T, nrows, Y, O2, partial, s); break;
+    case 8: g = apply_nb<8, FLIP>(X, T, nrows, Y, O2, partial, s); break;
+  }
+  check_launch("apply_mfma");
+  return g;
 }
 
 void launch_apply(const double* X, const double* T, uint64_t nrows, int lp, double* Y, hipStream_t s) {
+  if (nrows) apply_lp<false>(X, T, nrows, lp, Y, nullptr, nullptr, s);
+}
+
+void launch_apply_flip(const double* X, const double* T, uint64_t nrows, int n, int lp, double* Y, const double* O2,
+                       double* partial, double* sign, hipStream_t s) {
   if (!nrows) return;
-  require(lp <= 128 && lp % 16 == 0 && lp >= 16, kErrArgument, "apply: bad lp");
-  switch (lp / 16) {
-    case 1: apply_nb<1>(X, T, nrows, Y, s); break;
-    case 2: apply_nb<2>(X, T, nrows, Y, s); break;
-    case 3: apply_nb<3>(X, T, nrows, Y, s); break;
-    case 4: apply_nb<4>(X, T, nrows, Y, s); break;
-    case 5: apply_nb<5>(X, T, nrows, Y, s); break;
-    case 6: apply_nb<6>(X, T, nrows, Y, s); break;
-    case 7: apply_nb<7>(X, T, nrows, Y, s); break;
-    case 8: apply_nb<8>(X, T, nrows, Y, s); break;
-  }
-  check_launch("apply_mfma");
+  const unsigned g = apply_lp<true>(X, T, nrows, lp, Y, O2, partial, s);
+  launch_flip_signs(partial, (int)g, n, lp, sign, s);
 }
 
 void launch_flip_norms(const double* O2, const double* Q, uint64_t nrows, int lp, double* partial, double* out,
@@ -1782,8 +1858,8 @@ void launch_thinq_second(const double* G2, const double* R1, const double* Xtop,
   check_launch("thinq_second");
 }
 
-void launch_flip_signs(const double* ab, int n, int lp, double* sign, hipStream_t s) {
-  hipLaunchKernelGGL(k_flip_signs, dim3(1), dim3(128), 0, s, ab, n, lp, sign);
+void launch_flip_signs(const double* partial, int nb, int n, int lp, double* sign, hipStream_t s) {
+  hipLaunchKernelGGL(k_flip_signs, dim3(1), dim3(1024), 0, s, partial, nb, n, lp, sign);
   check_launch("flip_signs");
 }
 

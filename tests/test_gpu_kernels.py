@@ -78,3 +78,37 @@ def test_missing_lists(ctx, n, m, miss):
     assert (np.abs(ctx.get_g(0, m, L) - G) / g_bound).max() <= 1.0
     h_bound = u * m * 1.5 * (sc @ np.abs(G)) + 1.5 * (sc @ g_bound)
     assert (np.abs(ctx.get_h(0, L) - H) / h_bound).max() <= 1.0
+
+
+@pytest.mark.parametrize("n,m,L", [(18, 200, 16), (65, 300, 20), (1023, 1200, 40), (1030, 700, 64), (4097, 500, 80),
+                                   (20011, 300, 33), (130, 400, 100)])
+def test_omega_update(ctx, n, m, L):
+    """Two Omega updates (thin-Q with Householder's column signs, then flipOmg) against LAPACK's Q, seen through
+    the next G = A Omega: L below, at and past the 16-column blocks, N below and past the row blocks."""
+    say(f"omega update n={n} m={m} L={L}")
+    rng = np.random.default_rng(n + L)
+    codes = random_codes(rng, m, n, 0.0)
+    # a planted structure: the columns of successive Q then agree up to their signs
+    for g in range(5):
+        codes[g * m // 6:(g + 1) * m // 6, g * n // 6:(g + 1) * n // 6] = rng.choice([0, 2], (m // 6 + 1, n // 6 + 1))[
+            :(g + 1) * m // 6 - g * m // 6, :(g + 1) * n // 6 - g * n // 6]
+    A, _ = standardized(codes)
+    omega = rng.standard_normal((n, L))
+    ctx.upload_packed(pack(codes), n)
+    ctx.standardize()
+    ctx.configure("fp64", L)
+    ctx.set_omega(omega)
+    ref, amplify = omega, 1.0
+    for _ in range(2):
+        ctx.sketch(0, m, 0)
+        ctx.update_omega(0)
+        H = A.T @ (A @ ref)
+        Q = np.linalg.qr(H)[0]
+        flip = np.abs(ref - Q).sum(0) > 2 * np.abs(ref + Q).sum(0)
+        ref = np.where(flip, -Q, Q)
+        amplify *= 1.0 + np.linalg.cond(H)
+    ctx.sketch(0, m, 0)
+    G = A @ ref
+    # each thin-Q is within a moderate multiple of u cond(H) of the exact one, and the next starts from it
+    err = np.abs(ctx.get_g(0, m, L) - G).max() / np.abs(G).max()
+    assert err <= 1e4 * 2.0**-53 * amplify
