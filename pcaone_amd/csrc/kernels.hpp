@@ -119,7 +119,7 @@ void launch_zero_ranges(void* base, uint64_t pitch, uint64_t rows, uint64_t b0, 
 // flip_UV with V as the base (src/Utils.cpp:118-154) on device-resident
 // V (m x lp) and U (n x lp), row-major: column c < k of both changes sign when
 // V's entry of largest magnitude (the first such) is negative.  partial:
-// 2048 x lp scratch; sign: lp.
+// 2 x 256 x 128 scratch; sign: lp.
 void launch_flip_cols_by_max(double* V, uint64_t m, double* U, uint64_t n, int lp, int k, double* partial,
                              double* sign, hipStream_t s);
 // dst (rows x kp) = first k columns of src (rows x lp) times scale[c] (null = 1), zero padded.

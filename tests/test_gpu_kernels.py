@@ -112,3 +112,21 @@ def test_omega_update(ctx, n, m, L):
     # each thin-Q is within a moderate multiple of u cond(H) of the exact one, and the next starts from it
     err = np.abs(ctx.get_g(0, m, L) - G).max() / np.abs(G).max()
     assert err <= 1e4 * 2.0**-53 * amplify
+
+
+@pytest.mark.parametrize("m,k", [(60, 3), (65, 1), (1000, 10), (16385, 2), (40001, 16)])
+def test_emu_flip_uv(ctx, m, k):
+    """flip_UV with V as the base after every EM iteration: V's entry of largest magnitude is positive in every
+    column, and U went with it (A V points along U)."""
+    say(f"flip_UV m={m} k={k}")
+    n = 90
+    rng = np.random.default_rng(m + k)
+    codes = random_codes(rng, m, n, 0.05)
+    for g in range(k):
+        codes[g::k + 1, g * n // (k + 1):(g + 1) * n // (k + 1)] = rng.choice([0, 2])
+    ctx.upload_packed(pack(codes), n)
+    r = ctx.run(svd=1, k=k, oversamples=10, emu=1, maxiter=2, printv=1, precision="fp64", want_v=True)
+    V, U = r.V, r.U
+    assert np.all(V[np.abs(V).argmax(0), np.arange(k)] > 0)
+    A, _ = standardized(codes)
+    assert np.all(((A.T @ V) * U).sum(0) > 0)
