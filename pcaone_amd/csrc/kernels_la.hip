@@ -1104,308 +1104,376 @@ __global__ void __launch_bounds__(256) k_missing_spmm(MissSpmmArgs a) {
 }
 
 // ---- L x L steps of the thin-Q of H on the device (one workgroup each) ----
-// Register-blocked: 256 threads form a 16 x 16 grid and thread (ty, tx) holds
-// the elements (ty + 16 p, tx + 16 q), p, q < NB = lp / 16, of each L x L
-// matrix in registers.  The elimination steps exchange one row and one
-// column per step through double-buffered LDS vectors, one barrier per step.
-// The elimination order is the host routines' (linalg_host.cpp): right-
-// looking Cholesky, back substitution for R^-1, modified LU for the
-// Householder signs (Ballard et al. 2014); divisions by a step's pivot are
-// multiplications by its reciprocal.
-constexpr int kSmallThreads = 256;
+// Serial chains: n pivots of a Cholesky factorization, n rows of a triangular
+// inverse, n pivots of a modified LU, each a square root or a division long.
+// What bounds them is the latency between one pivot and the next, so a panel
+// of 16 pivots runs inside one wave (lane = matrix column, registers = the
+// panel's 16 rows, readlane in place of LDS and barriers), the inverse gives
+// each column of the result to four lanes of one wave, and the 16-row updates
+// between panels and the products are FP64 MFMAs.  v_mfma_f64_16x16x4 adds its
+// four products to the accumulator one after another in ascending k as fused
+// multiply-adds, so every element sees the operations of the unblocked
+// elimination in the same order, and the results are the same bits.
+// One element per thread of a 16 x 16 grid and a barrier per pivot, as before,
+// against this form, first + second kernel: L = 14 10 + 15 -> 8 + 11 us, L = 20
+// 17 + 29 -> 13 + 19 us, L = 40 48 + 79 -> 22 + 35 us, L = 80 146 + 259 -> 43 + 77 us.
+constexpr int kThinqThreads = 512;
 constexpr int kThinqMaxNB = 5;  // lp <= 80
 
+// LDS pitch of an L x L matrix (rows on 16-byte boundaries, off the bank period).
 template <int NB>
-struct RegMat {
-  double v[NB][NB];
-};
+constexpr int kLP = NB * 16 + 2;
 
-template <int NB>
-__device__ __forceinline__ void rm_zero(RegMat<NB>& m) {
-#pragma unroll
-  for (int p = 0; p < NB; ++p)
-#pragma unroll
-    for (int q = 0; q < NB; ++q) m.v[p][q] = 0.0;
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
 
-// Rows and columns >= n read as zero.
+// Lane S of every group of four lanes, to the whole group.
+template <int S>
+__device__ __forceinline__ double quad_value(double v) {
+  constexpr int ctrl = S * 0x55;
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, ctrl, 0xF, 0xF, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), ctrl, 0xF, 0xF, true);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
+// src (lp x lp in global memory) -> LDS, zero in rows and columns >= n, and
+// below the diagonal blocks when `upper`.
 template <int NB>
-__device__ __forceinline__ void rm_load(RegMat<NB>& m, const double* src, int n, int lp, int ty, int tx) {
-#pragma unroll
-  for (int p = 0; p < NB; ++p)
-#pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int i = ty + 16 * p, k = tx + 16 * q;
-      m.v[p][q] = (i < n && k < n) ? src[i * lp + k] : 0.0;
-    }
+__device__ __forceinline__ void lds_load(double* M, const double* __restrict__ src, int n, bool upper) {
+  constexpr int LP = NB * 16;
+  for (int v = threadIdx.x; v < LP * LP; v += kThinqThreads) {
+    const int i = v / LP, k = v - i * LP;
+    const bool in = i < n && k < n && (!upper || (i >> 4) <= (k >> 4));
+    M[i * kLP<NB> + k] = in ? src[v] : 0.0;
+  }
+}
+
+// acc += sign * A[16 bi ..][k] B[k][16 bj ..] for k in [k0, k1), one 16 x 16
+// block per wave (accumulator register r: row q + 4 r, column r16).
+template <int NB>
+__device__ __forceinline__ f64x4_t block_product(f64x4_t acc, const double* A, const double* B, int bi, int bj, int k0,
+                                                 int k1, int lane) {
+  const int q = lane >> 4, r16 = lane & 15;
+  for (int k = k0; k < k1; k += 4)
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A[(16 * bi + r16) * kLP<NB> + k + q],
+                                               B[(k + q) * kLP<NB> + 16 * bj + r16], acc, 0, 0, 0);
+  return acc;
 }
 
 template <int NB>
-__device__ __forceinline__ void rm_store(const RegMat<NB>& m, double* dst, int lp, int ty, int tx) {
+__device__ __forceinline__ f64x4_t block_load(const double* M, int bi, int bj, int lane) {
+  f64x4_t v;
 #pragma unroll
-  for (int p = 0; p < NB; ++p)
-#pragma unroll
-    for (int q = 0; q < NB; ++q) dst[(ty + 16 * p) * lp + tx + 16 * q] = m.v[p][q];
+  for (int r = 0; r < 4; ++r) v[r] = M[(16 * bi + (lane >> 4) + 4 * r) * kLP<NB> + 16 * bj + (lane & 15)];
+  return v;
 }
 
-// In place: A (n x n, symmetric positive definite, upper triangle used) ->
-// upper R with A = R^T R; rows and columns >= n and the lower triangle end
-// zero.  Returns false (in every thread) on breakdown.  rowbuf: 2 lp.
 template <int NB>
-__device__ bool rb_chol_upper(RegMat<NB>& a, int n, int lp, double* rowbuf, int ty, int tx,
-                              double* min_pivot = nullptr) {
+__device__ __forceinline__ void block_store(double* M, const f64x4_t& v, int bi, int bj, int lane) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) M[(16 * bi + (lane >> 4) + 4 * r) * kLP<NB> + 16 * bj + (lane & 15)] = v[r];
+}
+
+// In place: A (n x n, symmetric positive definite, upper blocks used, zero
+// below the diagonal blocks and past n) -> upper R with A = R^T R, zero
+// elsewhere.  Right-looking.  Returns false (in every thread) on breakdown;
+// *min_pivot (thread 0) receives the smallest pivot.
+template <int NB>
+__device__ bool lds_chol_upper(double* A, int n, double* min_pivot, int* flag) {
+  constexpr int P = kLP<NB>;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int nbn = (n + 15) / 16;
   double dmin = INFINITY;
-  if (ty == 0) {
-#pragma unroll
-    for (int q = 0; q < NB; ++q) rowbuf[tx + 16 * q] = a.v[0][q];
-  }
+  if (tid == 0) *flag = 0;
   __syncthreads();
-  bool ok = true;
-  for (int j = 0; j < n; ++j) {
-    const double* rb = rowbuf + (j & 1) * lp;
-    const double d = rb[j];
-    if (!(d > 0.0) || !isfinite(d)) {  // the same value in every thread
-      ok = false;
-      break;
+  for (int b = 0; b < nbn; ++b) {
+    const int r0 = 16 * b, m = n - r0 - 16;  // m columns right of the panel's own
+    // lanes 0..15: the diagonal block's columns; the others: 48 columns to the right
+    const bool mine = wave < (m > 48 ? 2 : 1);
+    const int col = lane < 16 ? r0 + lane : r0 + 48 * wave + lane;
+    const bool in = mine && col < NB * 16;
+    double a[16];
+    if (mine) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) a[i] = A[(r0 + i) * P + (in ? col : r0)];
     }
-    dmin = fmin(dmin, d);
-    const double rjj = sqrt(d), inv = 1.0 / rjj;
-    double si[NB], sk[NB];
+    __syncthreads();  // wave 0 writes the diagonal block that both waves read
+    if (mine) {
+      bool ok = true;
 #pragma unroll
-    for (int p = 0; p < NB; ++p) si[p] = rb[ty + 16 * p] * inv;
+      for (int j = 0; j < 16; ++j) {
+        if (ok && r0 + j < n) {
+          const double d = lane_value(a[j], j);
+          if (!(d > 0.0) || !isfinite(d)) {  // the same value in every lane
+            ok = false;
+          } else {
+            dmin = fmin(dmin, d);
+            const double rjj = sqrt(d), inv = 1.0 / rjj;
+            const double sj = a[j] * inv;
+            a[j] = lane == j ? rjj : sj;
 #pragma unroll
-    for (int q = 0; q < NB; ++q) sk[q] = rb[tx + 16 * q] * inv;
-#pragma unroll
-    for (int p = 0; p < NB; ++p) {
-      const int i = ty + 16 * p;
-#pragma unroll
-      for (int q = 0; q < NB; ++q) {
-        const int k = tx + 16 * q;
-        if (i > j && k >= i && k < n) a.v[p][q] -= si[p] * sk[q];
-        else if (i == j) a.v[p][q] = k > j ? sk[q] : (k == j ? rjj : 0.0);  // row j of R
-      }
-    }
-    if (j + 1 < n && ty == ((j + 1) & 15)) {  // publish row j + 1 for the next step
-      const int p1 = (j + 1) >> 4;
-#pragma unroll
-      for (int p = 0; p < NB; ++p)
-        if (p == p1) {
-#pragma unroll
-          for (int q = 0; q < NB; ++q) rowbuf[((j + 1) & 1) * lp + tx + 16 * q] = a.v[p][q];
-        }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int p = 0; p < NB; ++p)
-#pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int i = ty + 16 * p, k = tx + 16 * q;
-      if (!ok || k < i || i >= n || k >= n) a.v[p][q] = 0.0;
-    }
-  if (min_pivot) *min_pivot = dmin;
-  return ok;
-}
-
-// X = R^-1 for upper R (n x n, zero outside), by rows from the bottom:
-// X[i][c] = (delta_ic - sum_{k>i} R[i][k] X[k][c]) / R[i][i], the sums
-// accumulated as each row of X is published.  buf: 5 lp (diag, 2 x row, 2 x column).
-template <int NB>
-__device__ void rb_inv_upper(const RegMat<NB>& r, RegMat<NB>& x, int n, int lp, double* buf, int ty, int tx) {
-  double* diag = buf;
-  double* xrow = buf + lp;
-  double* rcol = buf + 3 * lp;
-#pragma unroll
-  for (int p = 0; p < NB; ++p)
-#pragma unroll
-    for (int q = 0; q < NB; ++q)
-      if (ty + 16 * p == tx + 16 * q) diag[ty + 16 * p] = r.v[p][q];
-  rm_zero(x);
-  __syncthreads();
-  for (int i = n - 1; i >= 0; --i) {
-    const int b = i & 1;
-    if (ty == (i & 15)) {
-      const int pi = i >> 4;
-      const double inv = 1.0 / diag[i];
-#pragma unroll
-      for (int p = 0; p < NB; ++p)
-        if (p == pi) {
-#pragma unroll
-          for (int q = 0; q < NB; ++q) {
-            const int c = tx + 16 * q;
-            const double v = (c >= i && c < n) ? ((c == i ? 1.0 : 0.0) - x.v[p][q]) * inv : 0.0;
-            x.v[p][q] = v;
-            xrow[b * lp + c] = v;
+            for (int i = j + 1; i < 16; ++i) a[i] = fma(-lane_value(sj, i), sj, a[i]);
           }
         }
-    }
-    if (tx == (i & 15)) {
-      const int qi = i >> 4;
+      }
+      if (!ok && tid == 0) *flag = 1;
+      if (in && (lane >= 16 || wave == 0)) {
 #pragma unroll
-      for (int q = 0; q < NB; ++q)
-        if (q == qi) {
-#pragma unroll
-          for (int p = 0; p < NB; ++p) rcol[b * lp + ty + 16 * p] = r.v[p][q];
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int p = 0; p < NB; ++p) {
-      if (ty + 16 * p < i) {
-        const double rv = rcol[b * lp + ty + 16 * p];
-#pragma unroll
-        for (int q = 0; q < NB; ++q) x.v[p][q] += rv * xrow[b * lp + tx + 16 * q];
+        for (int i = 0; i < 16; ++i) A[(r0 + i) * P + col] = (lane >= 16 || i <= lane) && r0 + i < n ? a[i] : 0.0;
       }
     }
-  }
-  __syncthreads();  // the buffers are free again
-}
-
-// C = A B over k < n (A, B in LDS, pitch lp, zero outside n x n).
-template <int NB>
-__device__ void rb_matmul(const double* A, const double* B, RegMat<NB>& c, int n, int lp, int ty, int tx) {
-  rm_zero(c);
-  for (int k = 0; k < n; ++k) {
-    double av[NB], bv[NB];
+    __syncthreads();
+    if (*flag) return false;
+    // trailing blocks (bi <= bj): A -= R[panel]^T R[panel]
+    const int t = nbn - b - 1, nt = t * (t + 1) / 2;
+    for (int x = wave; x < nt; x += kThinqThreads / 64) {
+      int i = 0, y = x;
+      while (y >= t - i) y -= t - i, ++i;
+      const int bi = b + 1 + i, bj = bi + y;
+      f64x4_t acc = block_load<NB>(A, bi, bj, lane);
 #pragma unroll
-    for (int p = 0; p < NB; ++p) av[p] = A[(ty + 16 * p) * lp + k];
-#pragma unroll
-    for (int q = 0; q < NB; ++q) bv[q] = B[k * lp + tx + 16 * q];
-#pragma unroll
-    for (int p = 0; p < NB; ++p)
-#pragma unroll
-      for (int q = 0; q < NB; ++q) c.v[p][q] += av[p] * bv[q];
-  }
-}
-
-// Householder diagonal signs of the thin QR whose Q has top block W (n x n,
-// destroyed): modified LU, s_i = -sign(u_ii).  buf: 4 lp.
-template <int NB>
-__device__ void rb_householder_signs(RegMat<NB>& w, int n, int lp, double* buf, double* sgn, int ty, int tx) {
-  double* rowb = buf;
-  double* colb = buf + 2 * lp;
-  for (int i = 0; i < n; ++i) {
-    const int b = i & 1;
-    if (ty == (i & 15) && tx == (i & 15)) {  // the pivot: w[i][i] -= s_i
-      const int pi = i >> 4;
-#pragma unroll
-      for (int p = 0; p < NB; ++p)
-        if (p == pi) {
-          const double si = w.v[p][p] >= 0.0 ? -1.0 : 1.0;
-          w.v[p][p] -= si;
-          sgn[i] = si;
-        }
-    }
-    if (ty == (i & 15)) {
-      const int pi = i >> 4;
-#pragma unroll
-      for (int p = 0; p < NB; ++p)
-        if (p == pi) {
-#pragma unroll
-          for (int q = 0; q < NB; ++q) rowb[b * lp + tx + 16 * q] = w.v[p][q];
-        }
-    }
-    if (tx == (i & 15)) {
-      const int qi = i >> 4;
-#pragma unroll
-      for (int q = 0; q < NB; ++q)
-        if (q == qi) {
-#pragma unroll
-          for (int p = 0; p < NB; ++p) colb[b * lp + ty + 16 * p] = w.v[p][q];
-        }
+      for (int k = 0; k < 16; k += 4) {
+        const double* row = A + (r0 + k + (lane >> 4)) * P + (lane & 15);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-row[16 * bi], row[16 * bj], acc, 0, 0, 0);
+      }
+      block_store<NB>(A, acc, bi, bj, lane);
     }
     __syncthreads();
-    const double inv = 1.0 / rowb[b * lp + i];  // the pivot
-#pragma unroll
-    for (int p = 0; p < NB; ++p) {
-      const int r = ty + 16 * p;
-      if (r > i && r < n) {
-        const double l = colb[b * lp + r] * inv;
-#pragma unroll
-        for (int q = 0; q < NB; ++q) {
-          const int c = tx + 16 * q;
-          if (c > i && c < n) w.v[p][q] -= l * rowb[b * lp + c];
-        }
-      }
-    }
   }
+  if (tid == 0) *min_pivot = dmin;
+  return true;
+}
+
+// X = R^-1 for the upper R in LDS (n x n, zero outside), by rows from the
+// bottom: X[i][c] = (delta_ic - sum_{k > i} R[i][k] X[k][c]) / R[i][i], the sums
+// taken in descending k.  Lane s of four holds the rows 4 m + s of one column
+// c in x[m] (waves 0 .. NB - 1 take 16 columns each; a column's rows below the
+// diagonal stay zero).  rt: scratch of NB 16 x kLP values, which may not
+// overlap R; invd: NB 16 values.  The caller's barrier follows.
+template <int NB>
+__device__ __forceinline__ void lds_inv_upper(const double* R, double* rt, double* invd, int n, double (&x)[4 * NB]) {
+  constexpr int LP = NB * 16, P = kLP<NB>, L4 = LP / 4;
+  // rt[k][s L4 + m] = R[4 m + s][k]: a lane's factors of one k are contiguous
+  for (int v = threadIdx.x; v < LP * LP; v += kThinqThreads) {
+    const int i = v / LP, k = v - i * LP;
+    rt[k * P + (i & 3) * L4 + (i >> 2)] = R[i * P + k];
+  }
+  for (int i = threadIdx.x; i < n; i += kThinqThreads) invd[i] = 1.0 / R[i * P + i];
+#pragma unroll
+  for (int m = 0; m < L4; ++m) x[m] = 0.0;
   __syncthreads();
+  const int wave = threadIdx.x >> 6, c = threadIdx.x >> 2, s = threadIdx.x & 3;
+  if (wave >= NB) return;
+  const int kmax = 16 * wave + 16 < n ? 16 * wave + 16 : n;
+#pragma unroll
+  for (int kk = L4 - 1; kk >= 0; --kk) {
+    auto row = [&]<int S>() {
+      const int k = 4 * kk + S;
+      if (k >= kmax) return;  // the same in the whole wave
+      double v = ((c == k ? 1.0 : 0.0) - x[kk]) * invd[k];
+      v = c >= k && c < n ? v : 0.0;
+      const double xk = quad_value<S>(v);  // lane S holds row k
+      const double* f = rt + k * P + s * L4;
+#pragma unroll
+      for (int m = 0; m < kk; ++m) x[m] = fma(f[m], xk, x[m]);
+      x[kk] = s == S ? xk : (s < S ? fma(f[kk], xk, x[kk]) : x[kk]);
+    };
+    row.template operator()<3>();
+    row.template operator()<2>();
+    row.template operator()<1>();
+    row.template operator()<0>();
+  }
 }
 
-// First pass: R1 = chol(G1), T1 = R1^-1 (lp x lp, zero padded).
+// Householder diagonal signs of the thin QR whose Q has top block W (n x n in
+// LDS, zero past n, destroyed): modified LU, s_i = -sign(u_ii) (Ballard et al.
+// 2014).
 template <int NB>
-__global__ void __launch_bounds__(kSmallThreads) k_thinq_first(const double* __restrict__ G1, int n, int lp,
+__device__ void lds_householder_signs(double* W, int n, double* sgn) {
+  constexpr int P = kLP<NB>, LP = NB * 16;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int nbn = (n + 15) / 16;
+  for (int b = 0; b < nbn; ++b) {
+    const int r0 = 16 * b, m = n - r0 - 16;
+    const int nr = m > 48 ? 2 : (m > 0 ? 1 : 0);  // waves for the rows below; the columns right take as many
+    const int nu = nr > 1 ? nr : 1;
+    double a[16];
+    if (wave < nu) {  // lane = column, registers = the panel's rows
+      const int col = lane < 16 ? r0 + lane : r0 + 48 * wave + lane;
+      const bool in = col < LP;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) a[i] = W[(r0 + i) * P + (in ? col : r0)];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if (r0 + i < n) {
+          const double p = lane_value(a[i], i);
+          const double si = p >= 0.0 ? -1.0 : 1.0, inv = 1.0 / (p - si);
+          if (wave == 0 && lane == i) sgn[r0 + i] = si;
+#pragma unroll
+          for (int r = i + 1; r < 16; ++r) a[r] = fma(-(lane_value(a[r], i) * inv), a[i], a[r]);
+        }
+      }
+      if (in && lane >= 16) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) W[(r0 + i) * P + col] = a[i];
+      }
+    } else if (wave < nu + nr) {  // lane = row, registers = the panel's columns
+      const int row = lane < 16 ? r0 + lane : r0 + 48 * (wave - nu) + lane;
+      const bool in = row < LP;
+#pragma unroll
+      for (int c = 0; c < 16; ++c) a[c] = W[(in ? row : r0) * P + r0 + c];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {  // the rows below exist: the panel is whole
+        const double p = lane_value(a[i], i);
+        const double inv = 1.0 / (p - (p >= 0.0 ? -1.0 : 1.0));
+        const double l = a[i] * inv;
+#pragma unroll
+        for (int c = i + 1; c < 16; ++c) a[c] = fma(-l, lane_value(a[c], i), a[c]);
+        a[i] = l;
+      }
+      if (in && lane >= 16) {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) W[row * P + r0 + c] = a[c];
+      }
+    }
+    __syncthreads();
+    const int t = nbn - b - 1;
+    for (int x = wave; x < t * t; x += kThinqThreads / 64) {
+      const int bi = b + 1 + x / t, bj = b + 1 + x % t;
+      f64x4_t acc = block_load<NB>(W, bi, bj, lane);
+#pragma unroll
+      for (int k = 0; k < 16; k += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-W[(16 * bi + (lane & 15)) * P + r0 + k + (lane >> 4)],
+                                                   W[(r0 + k + (lane >> 4)) * P + 16 * bj + (lane & 15)], acc, 0, 0, 0);
+      block_store<NB>(W, acc, bi, bj, lane);
+    }
+    __syncthreads();
+  }
+}
+
+template <int NB>
+constexpr size_t thinq_lds() {
+  return ((size_t)2 * NB * 16 * kLP<NB> + 3 * NB * 16 + 2) * sizeof(double);
+}
+
+// First pass: R1 = chol(G1), T1 = R1^-1 (lp x lp, zero padded; zero on
+// breakdown).
+template <int NB>
+__global__ void __launch_bounds__(kThinqThreads) k_thinq_first(const double* __restrict__ G1, int n,
                                                                double* __restrict__ R1, double* __restrict__ T1,
                                                                int* __restrict__ status, double min_ratio) {
-  __shared__ double buf[5 * 16 * kThinqMaxNB];
-  __shared__ double dmax_s;
-  const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
-  RegMat<NB> a, x;
-  rm_load(a, G1, n, lp, ty, tx);
-  if (min_ratio > 0.0) {
-    // largest diagonal entry of the Gram (before the factorization overwrites it)
-    if (threadIdx.x == 0) {
-      double m = 0.0;
-      for (int i = 0; i < n; ++i) m = fmax(m, G1[i * lp + i]);
-      dmax_s = m;
-    }
+  constexpr int LP = NB * 16, P = kLP<NB>;
+  extern __shared__ __align__(16) double lm[];
+  double *A = lm, *rt = A + LP * P, *invd = rt + LP * P, *scal = invd + 3 * LP;
+  int* flag = reinterpret_cast<int*>(scal + 1);
+  const int tid = threadIdx.x;
+  lds_load<NB>(A, G1, n, true);
+  // largest diagonal entry of the Gram (before the factorization overwrites it)
+  if (min_ratio > 0.0 && tid < 64) {
+    double mx = 0.0;
+    for (int i = tid; i < n; i += 64) mx = fmax(mx, G1[i * LP + i]);
+    for (int d = 32; d > 0; d >>= 1) mx = fmax(mx, __shfl_xor(mx, d));
+    if (tid == 0) scal[0] = mx;
   }
+  __syncthreads();
   double dmin = 0.0;
-  const bool ok = rb_chol_upper(a, n, lp, buf, ty, tx, &dmin);
-  if (ok) rb_inv_upper(a, x, n, lp, buf, ty, tx);
-  else rm_zero(x);
-  if (!ok && threadIdx.x == 0) *status = 1;
+  const bool ok = lds_chol_upper<NB>(A, n, &dmin, flag);
+  if (!ok) {
+    if (tid == 0) *status = 1;
+    for (int v = tid; v < LP * LP; v += kThinqThreads) R1[v] = T1[v] = 0.0;
+    return;
+  }
   // the host's safety test of this Gram (smallest pivot / largest diagonal),
   // when the caller defers it to the device: a near rank-deficient H is marked
-  if (ok && min_ratio > 0.0 && threadIdx.x == 0 && !(dmin > min_ratio * dmax_s)) *status = 2;
-  rm_store(a, R1, lp, ty, tx);
-  rm_store(x, T1, lp, ty, tx);
+  if (min_ratio > 0.0 && tid == 0 && !(dmin > min_ratio * scal[0])) *status = 2;
+  for (int v = tid; v < LP * LP; v += kThinqThreads) R1[v] = A[v / LP * P + v % LP];
+  double x[4 * NB];
+  lds_inv_upper<NB>(A, rt, invd, n, x);
+  __syncthreads();  // R has been read: A takes X, so that its rows leave whole
+  if (tid < 4 * LP) {
+#pragma unroll
+    for (int m = 0; m < 4 * NB; ++m) A[(4 * m + (tid & 3)) * P + (tid >> 2)] = x[m];
+  }
+  __syncthreads();
+  for (int v = tid; v < LP * LP; v += kThinqThreads) T1[v] = A[v / LP * P + v % LP];
 }
 
 // Second pass: R2 = chol(G2), R^-1 = (R2 R1)^-1, the Householder signs s of
 // Xtop R^-1 (Xtop = the first n rows of the thinned matrix) and
-// T = R^-1 diag(s) (lp x lp, zero padded).  Dynamic LDS: 2 lp x lp matrices.
+// T = R^-1 diag(s) (lp x lp, zero padded; zero on breakdown).
 template <int NB>
-__global__ void __launch_bounds__(kSmallThreads) k_thinq_second(const double* __restrict__ G2,
+__global__ void __launch_bounds__(kThinqThreads) k_thinq_second(const double* __restrict__ G2,
                                                                 const double* __restrict__ R1,
-                                                                const double* __restrict__ Xtop, int n, int lp,
+                                                                const double* __restrict__ Xtop, int n,
                                                                 double* __restrict__ T, int* __restrict__ status) {
-  extern __shared__ __align__(16) unsigned char sm[];
-  __shared__ double buf[5 * 16 * kThinqMaxNB];
-  __shared__ double sgn[16 * kThinqMaxNB];
-  double* MA = reinterpret_cast<double*>(sm);
-  double* MB = MA + lp * lp;
-  const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
-  RegMat<NB> a, x;
-  rm_load(a, G2, n, lp, ty, tx);
-  const bool ok = rb_chol_upper(a, n, lp, buf, ty, tx);  // R2
-  if (ok) {
-    RegMat<NB> t;
-    rm_store(a, MA, lp, ty, tx);
-    rm_load(t, R1, n, lp, ty, tx);
-    rm_store(t, MB, lp, ty, tx);
+  constexpr int LP = NB * 16, P = kLP<NB>, NW = kThinqThreads / 64;
+  extern __shared__ __align__(16) double lm[];
+  double *A = lm, *B = A + LP * P, *invd = B + LP * P, *sgn = invd + LP, *scal = invd + 3 * LP;
+  int* flag = reinterpret_cast<int*>(scal + 1);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  lds_load<NB>(A, G2, n, true);
+  lds_load<NB>(B, R1, n, true);
+  __syncthreads();
+  double dmin;
+  if (!lds_chol_upper<NB>(A, n, &dmin, flag)) {  // R2
+    if (tid == 0) *status = 1;
+    for (int v = tid; v < LP * LP; v += kThinqThreads) T[v] = 0.0;
+    return;
+  }
+  {  // A = R2 R1: the upper blocks
+    constexpr int NT = NB * (NB + 1) / 2, S = (NT + NW - 1) / NW;
+    f64x4_t c[S];
+#pragma unroll
+    for (int u = 0; u < S; ++u) {
+      const int t = wave + NW * u;
+      if (t < NT)
+        c[u] = block_product<NB>(f64x4_t{0, 0, 0, 0}, A, B, sym_block_i(t, NB), sym_block_j(t, NB),
+                                 16 * sym_block_i(t, NB), 16 * sym_block_j(t, NB) + 16, lane);
+    }
     __syncthreads();
-    rb_matmul(MA, MB, a, n, lp, ty, tx);  // R = R2 R1
-    rb_inv_upper(a, x, n, lp, buf, ty, tx);  // R^-1 (ends with a barrier: MA, MB are free)
-    rm_store(x, MB, lp, ty, tx);
-    rm_load(t, Xtop, n, lp, ty, tx);
-    rm_store(t, MA, lp, ty, tx);
-    __syncthreads();
-    rb_matmul(MA, MB, t, n, lp, ty, tx);  // Xtop R^-1
-    rb_householder_signs(t, n, lp, buf, sgn, ty, tx);
-  } else {
-    rm_zero(x);
-    if (threadIdx.x < 16 * NB) sgn[threadIdx.x] = 1.0;
-    if (threadIdx.x == 0) *status = 1;
+#pragma unroll
+    for (int u = 0; u < S; ++u) {
+      const int t = wave + NW * u;
+      if (t < NT) block_store<NB>(A, c[u], sym_block_i(t, NB), sym_block_j(t, NB), lane);
+    }
     __syncthreads();
   }
+  double x[4 * NB];
+  lds_inv_upper<NB>(A, B, invd, n, x);
+  __syncthreads();
+  if (tid < 4 * LP) {  // A = R^-1
 #pragma unroll
-  for (int p = 0; p < NB; ++p)
+    for (int m = 0; m < 4 * NB; ++m) A[(4 * m + (tid & 3)) * P + (tid >> 2)] = x[m];
+  }
+  lds_load<NB>(B, Xtop, n, false);
+  __syncthreads();
+  {  // B = Xtop R^-1 (R^-1 is upper: k up to the block's last column)
+    constexpr int NT = NB * NB, S = (NT + NW - 1) / NW;
+    f64x4_t c[S];
 #pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int c = tx + 16 * q;
-      T[(ty + 16 * p) * lp + c] = c < n ? x.v[p][q] * sgn[c] : 0.0;
+    for (int u = 0; u < S; ++u) {
+      const int t = wave + NW * u;
+      if (t < NT)
+        c[u] = block_product<NB>(f64x4_t{0, 0, 0, 0}, B, A, t / NB, t % NB, 0, 16 * (t % NB) + 16, lane);
     }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < S; ++u) {
+      const int t = wave + NW * u;
+      if (t < NT) block_store<NB>(B, c[u], t / NB, t % NB, lane);
+    }
+    __syncthreads();
+  }
+  lds_householder_signs<NB>(B, n, sgn);
+  for (int v = tid; v < LP * LP; v += kThinqThreads) {
+    const int c = v % LP;
+    T[v] = c < n ? A[v / LP * P + c] * sgn[c] : 0.0;
+  }
 }
 
 // flipOmg's decision (src/RSVD.hpp:80-89): column l flips when
@@ -1852,41 +1920,52 @@ void launch_sum_chunks(const double* partial, uint64_t nz, uint64_t nrows, int n
 
 bool thinq_on_device(int lp) { return lp % 16 == 0 && lp <= 16 * kThinqMaxNB; }
 
+template <int NB>
+void thinq_first_nb(const double* G1, int n, double* R1, double* T1, int* status, double min_ratio, hipStream_t s) {
+  static bool attr = false;
+  if (!attr) {
+    PCAONE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_thinq_first<NB>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)thinq_lds<NB>()));
+    attr = true;
+  }
+  hipLaunchKernelGGL(k_thinq_first<NB>, dim3(1), dim3(kThinqThreads), thinq_lds<NB>(), s, G1, n, R1, T1, status,
+                     min_ratio);
+}
+
 void launch_thinq_first(const double* G1, int n, int lp, double* R1, double* T1, int* status, hipStream_t s,
                         double min_ratio) {
   require(thinq_on_device(lp) && n <= lp, kErrInternal, "thinq: lp too large for the device path");
   switch (lp / 16) {
-    case 1: hipLaunchKernelGGL(k_thinq_first<1>, dim3(1), dim3(kSmallThreads), 0, s, G1, n, lp, R1, T1, status, min_ratio); break;
-    case 2: hipLaunchKernelGGL(k_thinq_first<2>, dim3(1), dim3(kSmallThreads), 0, s, G1, n, lp, R1, T1, status, min_ratio); break;
-    case 3: hipLaunchKernelGGL(k_thinq_first<3>, dim3(1), dim3(kSmallThreads), 0, s, G1, n, lp, R1, T1, status, min_ratio); break;
-    case 4: hipLaunchKernelGGL(k_thinq_first<4>, dim3(1), dim3(kSmallThreads), 0, s, G1, n, lp, R1, T1, status, min_ratio); break;
-    default: hipLaunchKernelGGL(k_thinq_first<5>, dim3(1), dim3(kSmallThreads), 0, s, G1, n, lp, R1, T1, status, min_ratio); break;
+    case 1: thinq_first_nb<1>(G1, n, R1, T1, status, min_ratio, s); break;
+    case 2: thinq_first_nb<2>(G1, n, R1, T1, status, min_ratio, s); break;
+    case 3: thinq_first_nb<3>(G1, n, R1, T1, status, min_ratio, s); break;
+    case 4: thinq_first_nb<4>(G1, n, R1, T1, status, min_ratio, s); break;
+    default: thinq_first_nb<5>(G1, n, R1, T1, status, min_ratio, s); break;
   }
   check_launch("thinq_first");
 }
 
 template <int NB>
-void thinq_second_nb(const double* G2, const double* R1, const double* Xtop, int n, int lp, double* T, int* status,
+void thinq_second_nb(const double* G2, const double* R1, const double* Xtop, int n, double* T, int* status,
                      hipStream_t s) {
-  const size_t lds = (size_t)2 * lp * lp * sizeof(double);
   static bool attr = false;
   if (!attr) {
     PCAONE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_thinq_second<NB>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(2 * 256 * NB * NB * sizeof(double))));
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)thinq_lds<NB>()));
     attr = true;
   }
-  hipLaunchKernelGGL(k_thinq_second<NB>, dim3(1), dim3(kSmallThreads), lds, s, G2, R1, Xtop, n, lp, T, status);
+  hipLaunchKernelGGL(k_thinq_second<NB>, dim3(1), dim3(kThinqThreads), thinq_lds<NB>(), s, G2, R1, Xtop, n, T, status);
 }
 
 void launch_thinq_second(const double* G2, const double* R1, const double* Xtop, int n, int lp, double* T,
                          int* status, hipStream_t s) {
   require(thinq_on_device(lp) && n <= lp, kErrInternal, "thinq: lp too large for the device path");
   switch (lp / 16) {
-    case 1: thinq_second_nb<1>(G2, R1, Xtop, n, lp, T, status, s); break;
-    case 2: thinq_second_nb<2>(G2, R1, Xtop, n, lp, T, status, s); break;
-    case 3: thinq_second_nb<3>(G2, R1, Xtop, n, lp, T, status, s); break;
-    case 4: thinq_second_nb<4>(G2, R1, Xtop, n, lp, T, status, s); break;
-    default: thinq_second_nb<5>(G2, R1, Xtop, n, lp, T, status, s); break;
+    case 1: thinq_second_nb<1>(G2, R1, Xtop, n, T, status, s); break;
+    case 2: thinq_second_nb<2>(G2, R1, Xtop, n, T, status, s); break;
+    case 3: thinq_second_nb<3>(G2, R1, Xtop, n, T, status, s); break;
+    case 4: thinq_second_nb<4>(G2, R1, Xtop, n, T, status, s); break;
+    default: thinq_second_nb<5>(G2, R1, Xtop, n, T, status, s); break;
   }
   check_launch("thinq_second");
 }
