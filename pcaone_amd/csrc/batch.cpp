@@ -492,24 +492,18 @@ void Batch::run(const Param& p, bool want_v, bool use_graph, BatchResult& out) {
   last_k_ = k;
 }
 
-void Batch::get_u(uint32_t c, double* U) const {
+void Batch::get_u(uint32_t c, double* U) {
   require(c < size() && c < stop_epoch_.size(), kErrState, "batch: no result for this cohort");
   const int buf = (stop_epoch_[c] & 1) ? kBufU1 : kBufU0;
-  std::vector<double> h((uint64_t)N_[c] * LP);
-  PCAONE_HIP(hipMemcpyAsync(h.data(), host_coh_[c].mat[buf], h.size() * 8, hipMemcpyDeviceToHost, stream_));
-  PCAONE_HIP(hipStreamSynchronize(stream_));
-  for (int j = 0; j < last_k_; ++j)
-    for (uint64_t i = 0; i < N_[c]; ++i) U[(uint64_t)j * N_[c] + i] = h[i * LP + j];
+  cols_.resize((uint64_t)*std::max_element(N_.begin(), N_.end()) * last_k_);  // one allocation serves every cohort
+  ctx_.download_cols(host_coh_[c].mat[buf], N_[c], LP, last_k_, cols_.get(), U);
 }
 
-void Batch::get_v(uint32_t c, double* V) const {
+void Batch::get_v(uint32_t c, double* V) {
   require(c < size() && c < stop_epoch_.size(), kErrState, "batch: no result for this cohort");
   require(layout_.want_v && host_coh_[c].mat[kBufV], kErrState, "batch: run with loadings first");
-  std::vector<double> h(M_[c] * LP);
-  PCAONE_HIP(hipMemcpyAsync(h.data(), host_coh_[c].mat[kBufV], h.size() * 8, hipMemcpyDeviceToHost, stream_));
-  PCAONE_HIP(hipStreamSynchronize(stream_));
-  for (int j = 0; j < last_k_; ++j)
-    for (uint64_t i = 0; i < M_[c]; ++i) V[(uint64_t)j * M_[c] + i] = h[i * LP + j];
+  cols_.resize(*std::max_element(M_.begin(), M_.end()) * (uint64_t)last_k_);
+  ctx_.download_cols(host_coh_[c].mat[kBufV], M_[c], LP, last_k_, cols_.get(), V);
 }
 
 }  // namespace pcaone

@@ -59,8 +59,8 @@ class Batch {
   // ---- run: every cohort's randomized SVD; results stay on the device
   // until read with get_u / get_v.  use_graph: capture and replay.
   void run(const Param& p, bool want_v, bool use_graph, BatchResult& out);
-  void get_u(uint32_t c, double* U) const;  // N_c x k, column-major
-  void get_v(uint32_t c, double* V) const;  // M_c x k, column-major (run with want_v)
+  void get_u(uint32_t c, double* U);  // N_c x k, column-major
+  void get_v(uint32_t c, double* V);  // M_c x k, column-major (run with want_v)
   const BatchTuning& tuning() const { return tune_; }
   double last_seconds = 0;
 
@@ -87,7 +87,7 @@ class Batch {
              g.wm == o.g.wm && g.waves == o.g.waves && h.wm == o.h.wm && h.waves == o.h.waves;
     }
   } layout_;
-  DevBuf<double> mats_, scf_, vecs_, partial_;
+  DevBuf<double> mats_, scf_, vecs_, partial_, cols_;
   DevBuf<unsigned char> pieces_, part_;
   DevBuf<BatchSmall> small_;
   DevBuf<BatchCohort> coh_;

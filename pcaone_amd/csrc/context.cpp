@@ -2,6 +2,7 @@
 #include "context.hpp"
 
 #include <algorithm>
+#include <bit>
 #include <numeric>
 #include <cmath>
 #include <cstring>
@@ -682,16 +683,40 @@ void Context::stage_in(const double* host, uint64_t count, double* dev) {
 }
 
 void Context::stage_out(const double* dev, uint64_t count, double* host) {
-  pinned_.resize(count * 8);
-  unsigned char* st = pinned_.get();
-  PCAONE_HIP(hipMemcpyAsync(st, dev, count * 8, hipMemcpyDeviceToHost, stream));
-  PCAONE_HIP(hipStreamSynchronize(stream));
-  const int64_t pieces = 16;
+  // device -> two pinned slots -> host: the DMA of one slot runs while the
+  // other is copied out in parallel (the caller's pages are often touched here
+  // for the first time)
+  constexpr uint64_t kSlot = 1ull << 20;  // 8 MB
+  const uint64_t slot = std::min(count, kSlot), n = (count + kSlot - 1) / kSlot;
+  // whole powers of two: a sequence of slightly larger reads does not pin memory anew each time
+  pinned_.resize(std::bit_ceil(std::max<uint64_t>((n > 1 ? 2 : 1) * slot * 8, 256 << 10)));
+  double* st = reinterpret_cast<double*>(pinned_.get());
+  Event done[2];
+  const auto send = [&](uint64_t c) {
+    const uint64_t m = std::min(kSlot, count - c * kSlot);
+    PCAONE_HIP(hipMemcpyAsync(st + (c & 1) * slot, dev + c * kSlot, m * 8, hipMemcpyDeviceToHost, stream));
+    PCAONE_HIP(hipEventRecord(done[c & 1].get(), stream));
+  };
+  if (n) send(0);
+  for (uint64_t c = 0; c < n; ++c) {
+    if (c + 1 < n) send(c + 1);  // its slot was copied out in the step before
+    PCAONE_HIP(hipEventSynchronize(done[c & 1].get()));
+    const uint64_t m = std::min(kSlot, count - c * kSlot);
+    const double* from = st + (c & 1) * slot;
+    double* to = host + c * kSlot;
+    const int64_t pieces = 16;
 #pragma omp parallel for schedule(static)
-  for (int64_t q = 0; q < pieces; ++q) {
-    const uint64_t b0 = count * q / pieces, b1 = count * (q + 1) / pieces;
-    std::memcpy(host + b0, st + b0 * 8, (b1 - b0) * 8);
+    for (int64_t q = 0; q < pieces; ++q) {
+      const uint64_t b0 = m * q / pieces, b1 = m * (q + 1) / pieces;
+      std::memcpy(to + b0, from + b0, (b1 - b0) * 8);
+    }
   }
+}
+
+void Context::download_cols(const double* src, uint64_t rows, int pitch, int k, double* tmp, double* out,
+                            const uint32_t* place) {
+  launch_rows_to_colmajor(src, rows, pitch, k, tmp, stream, place);
+  stage_out(tmp, rows * (uint64_t)k, out);
 }
 
 void Context::set_omega(const double* om) {
@@ -1381,29 +1406,18 @@ void Context::save_prev() {
   PCAONE_HIP(hipMemcpyAsync(upre_.get(), ucur_.get(), (uint64_t)N * lp * 8, hipMemcpyDeviceToDevice, stream));
 }
 
-void Context::download_u(int k, double* U) {
-  launch_rows_to_colmajor(ucur_.get(), N, lp, k, tmp_n_.get(), stream);
-  stage_out(tmp_n_.get(), (uint64_t)N * k, U);
-}
-
-void Context::download_rowmajor(const double* src, uint64_t rows, double* out) {
-  std::vector<double> h(rows * (uint64_t)lp);
-  PCAONE_HIP(hipMemcpyAsync(h.data(), src, h.size() * 8, hipMemcpyDeviceToHost, stream));
-  PCAONE_HIP(hipStreamSynchronize(stream));
-  for (int j = 0; j < L; ++j)
-    for (uint64_t i = 0; i < rows; ++i) out[(uint64_t)j * rows + i] = h[i * lp + j];
-}
+void Context::download_u(int k, double* U) { download_cols(ucur_.get(), N, lp, k, tmp_n_.get(), U); }
 
 void Context::download_g(uint64_t j0, uint64_t j1, double* G) {
   require(L > 0, kErrState, "configure() first");
   require(j0 < j1 && j1 <= M, kErrArgument, "get_g: bad SNP range");
-  download_rowmajor(gt_.get() + j0 * lp, j1 - j0, G);
+  download_cols(gt_.get() + j0 * lp, j1 - j0, lp, L, tmp_m_.get(), G);
 }
 
 void Context::download_h(int which, double* H) {
   require(L > 0, kErrState, "configure() first");
   require(which >= 0 && which <= 2, kErrArgument, "get_h: which must be 0 (H), 1 (H1) or 2 (H2)");
-  download_rowmajor(which == 0 ? H_.get() : (which == 1 ? H1_.get() : H2_.get()), N, H);
+  download_cols(which == 0 ? H_.get() : (which == 1 ? H1_.get() : H2_.get()), N, lp, L, tmp_n_.get(), H);
 }
 
 void Context::residuals_prepare(int k, const double* U, const double* S, const double* V, bool as_read) {
@@ -1467,12 +1481,15 @@ void Context::compute_v(int k) {
   PCAONE_HIP(hipStreamSynchronize(stream));
 }
 
-void Context::download_v(int k, double* V) {
-  std::vector<double> h(M * (uint64_t)lp);
-  PCAONE_HIP(hipMemcpyAsync(h.data(), vbuf_.get(), h.size() * 8, hipMemcpyDeviceToHost, stream));
-  PCAONE_HIP(hipStreamSynchronize(stream));
-  for (uint64_t i = 0; i < M; ++i)
-    for (int j = 0; j < k; ++j) V[(uint64_t)j * M + i] = h[i * lp + j];
+void Context::download_v(int k, double* V) { download_cols(vbuf_.get(), M, lp, k, tmp_m_.get(), V); }
+
+void Context::download_v_original(int k, double* V) {
+  if (perm_identity_) return download_v(k, V);
+  // column i of the device order is SNP perm[i]
+  static_assert(sizeof(int) == sizeof(uint32_t));
+  place_.resize(M);
+  PCAONE_HIP(hipMemcpyAsync(place_.get(), perm.data(), M * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
+  download_cols(vbuf_.get(), M, lp, k, tmp_m_.get(), V, place_.get());
 }
 
 }  // namespace pcaone

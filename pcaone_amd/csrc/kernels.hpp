@@ -170,7 +170,8 @@ void launch_gather_f64(const double* src, const uint32_t* idx, uint64_t n, doubl
 void launch_colmajor_to_rows(const double* src, uint64_t n, int L, int lp, uint64_t rows_pad, double* dst,
                              hipStream_t s);
 // Row-major n x lp -> column-major n x k.
-void launch_rows_to_colmajor(const double* src, uint64_t n, int lp, int k, double* dst, hipStream_t s);
+void launch_rows_to_colmajor(const double* src, uint64_t n, int lp, int k, double* dst, hipStream_t s,
+                             const uint32_t* place = nullptr);
 // Y = X + Z elementwise (n elements).
 void launch_add(const double* X, const double* Z, double* Y, uint64_t n, hipStream_t s);
 // Missing-entry corrections, in two steps.

@@ -141,8 +141,7 @@ void RsvdOpData::fit_with_pi() {
     ctx_.set_impute_device(S.data(), (int)S.size());
     return;
   }
-  require(!U.empty() && !V.empty(), kErrState, "fit_with_pi before the first decomposition");
-  ctx_.set_impute(U.data(), S.data(), V.data(), (int)S.size());
+  fail(kErrInternal, "fit_with_pi: U and V are not on the device");
 }
 
 void RsvdOpData::computeUSV(int p, double tol) {
@@ -173,10 +172,7 @@ void RsvdOpData::computeUSV(int p, double tol) {
           ahead = false;
           S.assign(r.sigma.begin(), r.sigma.begin() + nk);
           ctx_.compute_v(nk);
-          if (need_v_host && !device_uv) {
-            V.resize(rows() * (uint64_t)nk);
-            ctx_.download_v(nk, V.data());
-          }
+          v_ready = true;
           break;
         }
       } else {
@@ -368,17 +364,21 @@ void FancyRsvdOpData::windows_blocks(int pi) {
   seg.flush();
 }
 
-PcaResult run_pca(Context& ctx, const Param& params, RunInfo* info, double* U_out) {
-  if (params.svd == 1 || params.svd == 2) return run_pca_with_halko(ctx, params, info, U_out);
+PcaResult run_pca(Context& ctx, const Param& params, RunInfo* info, double* U_out, double* V_out) {
+  if (params.svd == 1 || params.svd == 2) return run_pca_with_halko(ctx, params, info, U_out, V_out);
   PcaResult r = params.svd == 3 ? run_pca_full(ctx, params, info) : run_pca_arnoldi(ctx, params, info);
   if (U_out && !r.U.empty()) {
     std::memcpy(U_out, r.U.data(), r.U.size() * sizeof(double));
     r.U.clear();
   }
+  if (V_out && !r.V.empty()) {
+    std::memcpy(V_out, r.V.data(), r.V.size() * sizeof(double));
+    r.V.clear();
+  }
   return r;
 }
 
-PcaResult run_pca_with_halko(Context& ctx, const Param& params, RunInfo* info, double* U_out) {
+PcaResult run_pca_with_halko(Context& ctx, const Param& params, RunInfo* info, double* U_out, double* V_out) {
   // src/Halko.cpp:271-345 (genetic input, in-core, no LD output)
   ctx.reset_columns();  // restores the as-read state between runs; not part of the timed work
   BlockPlan plan;
@@ -453,8 +453,6 @@ PcaResult run_pca_with_halko(Context& ctx, const Param& params, RunInfo* info, d
       rsvd->U.resize(N * (uint64_t)k);
       ctx.download_u(k, rsvd->U.data());
     }
-    rsvd->V.resize(M * (uint64_t)k);
-    ctx.download_v(k, rsvd->V.data());
   }
   PcaResult res;
   res.k = k;
@@ -463,11 +461,10 @@ PcaResult run_pca_with_halko(Context& ctx, const Param& params, RunInfo* info, d
   res.S = rsvd->S;
   res.E.resize(res.S.size());
   for (size_t i = 0; i < res.S.size(); ++i) res.E[i] = res.S[i] * res.S[i] / (double)M;  // src/Halko.cpp:339
-  if (rsvd->need_v_host && !rsvd->V.empty()) {
+  if (rsvd->need_v_host && rsvd->v_ready) {
     // loadings in the original SNP order (src/Data.cpp:226-233)
-    res.V.assign(rsvd->V.size(), 0.0);
-    for (int c = 0; c < k; ++c)
-      for (uint64_t i = 0; i < M; ++i) res.V[(uint64_t)c * M + ctx.perm[i]] = rsvd->V[(uint64_t)c * M + i];
+    if (!V_out) res.V.resize(M * (uint64_t)k);
+    ctx.download_v_original(k, V_out ? V_out : res.V.data());
   }
   if (info) info->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   return res;

@@ -86,10 +86,11 @@ class RsvdOpData {
   void initOmg();
 
   bool update = false, standardize = false;
-  std::vector<double> U, S, V;  // N x k, k, M x k (column-major; V in device column order)
+  std::vector<double> U, S;  // N x k (column-major), k
   bool need_v_host = false;
+  bool v_ready = false;      // V (device column order) is in the context
   double* u_out = nullptr;  // when set (and no EMU), U is written there instead of into U
-  bool device_uv = false;   // U and V stay on the device (EM iterations); U, V left empty
+  bool device_uv = false;   // U and V stay on the device (EM iterations); U left empty
   RunInfo* info = nullptr;
 
  protected:
@@ -129,10 +130,13 @@ struct PcaResult {
 };
 
 // U_out (nullable, N x k column-major): receives U directly; res.U is then empty.
-PcaResult run_pca_with_halko(Context& ctx, const Param& params, RunInfo* info, double* U_out = nullptr);
+// V_out (nullable, M x k): the same for V, where the params ask for it.
+PcaResult run_pca_with_halko(Context& ctx, const Param& params, RunInfo* info, double* U_out = nullptr,
+                             double* V_out = nullptr);
 // The PCA the params select (src/Main.cpp:176-217): --svd 0 IRAM, 1/2 the
 // randomized SVD, 3 the exact eigen-decomposition.
-PcaResult run_pca(Context& ctx, const Param& params, RunInfo* info, double* U_out = nullptr);
+PcaResult run_pca(Context& ctx, const Param& params, RunInfo* info, double* U_out = nullptr,
+                  double* V_out = nullptr);
 
 
 }  // namespace pcaone

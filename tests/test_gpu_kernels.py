@@ -130,3 +130,43 @@ def test_emu_flip_uv(ctx, m, k):
     assert np.all(V[np.abs(V).argmax(0), np.arange(k)] > 0)
     A, _ = standardized(codes)
     assert np.all(((A.T @ V) * U).sum(0) > 0)
+
+
+@pytest.mark.parametrize("n,m,L", [(150, 33, 1), (150, 300, 17), (150, 1025, 128), (150, 20001, 128)])
+def test_read_back(ctx, n, m, L):
+    """G and H read back column-major: whole and in windows, below and past the 32-row tiles and the 8 MB slots."""
+    say(f"read back n={n} m={m} L={L}")
+    rng = np.random.default_rng(m + L)
+    codes = random_codes(rng, m, n, 0.0)
+    omega = rng.standard_normal((n, L))
+    ctx.upload_packed(pack(codes), n)
+    ctx.standardize()
+    ctx.configure("fp64", L)
+    ctx.set_omega(omega)
+    ctx.sketch(0, m, 0)
+    A, _ = standardized(codes)
+    G = ctx.get_g(0, m, L)
+    ref = A @ omega
+    assert np.abs(G - ref).max() <= 1e-12 * np.abs(ref).max()  # a placement test: FP64 sums of 150 terms
+    for j0, j1 in [(0, 1), (1, 33), (m // 3, m), (m - 1, m)]:
+        np.testing.assert_array_equal(ctx.get_g(j0, j1, L), G[j0:j1])
+    H = A.T @ ref
+    assert np.abs(ctx.get_h(0, L) - H).max() <= 1e-12 * np.abs(H).max()
+
+
+@pytest.mark.parametrize("svd,m", [(1, 40), (2, 2049)])
+def test_loadings_order(ctx, svd, m):
+    """Loadings come back in the original SNP order, with and without winSVD's shuffle: V S = A U."""
+    say(f"loadings svd={svd} m={m}")
+    n, k = 120, 3
+    rng = np.random.default_rng(m)
+    codes = random_codes(rng, m, n, 0.0)
+    for g in range(3):
+        codes[g::4, g * 30:g * 30 + 30] = 2 * (g % 2)
+    ctx.upload_packed(pack(codes), n)
+    r = ctx.run(svd=svd, k=k, oversamples=10, maxp=30, tol=1e-12, bands=8, precision="fp64", want_v=True)
+    A, _ = standardized(codes)
+    proj = A @ r.U
+    # V is G~'s own left factor: it agrees with A U up to the convergence of the subspace
+    for c in range(k):
+        assert np.dot(r.V[:, c], proj[:, c]) / np.linalg.norm(proj[:, c]) >= 0.999
