@@ -17,6 +17,15 @@ namespace {
 constexpr int LP = kBatchLp;
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
+// Kernels whose rows are independent of each other take an item of up to
+// kBatchRowsPerItem rows in slices of kSliceRows (grid.y): the items of the N
+// rows alone leave most CUs idle (90 items for 32 cohorts of 500-8,000
+// samples).  32 cohorts, L = 20, whole items -> slices: H epilogue 192 -> 22 us,
+// X T 53 -> 15 us, Omega's pieces 83 -> 20 us.  The reductions keep whole items:
+// their order is part of the result.
+constexpr uint32_t kSliceRows = 128;
+constexpr unsigned kSlices = kBatchRowsPerItem / kSliceRows;
+
 template <Form F>
 using piece_t = typename std::conditional<
     F == Form::FP64, double,
@@ -79,7 +88,7 @@ constexpr int tile_pitch(int rows) {
 
 // Omega (signed by the flipOmg signs or not) -> the FP64 copy, the value its
 // pieces sum to and the transposed pieces, in tiles of 64 rows: row-major
-// reads and writes, the pieces transposed through LDS.
+// reads and writes, the pieces transposed through LDS.  grid.y: row slices.
 template <Form F>
 __global__ void __launch_bounds__(256) k_b_make_pieces(BatchArgs a, const RowItem* __restrict__ items, int srcsel,
                                                        int signed_) {
@@ -99,8 +108,9 @@ __global__ void __launch_bounds__(256) k_b_make_pieces(BatchArgs a, const RowIte
   const int l = threadIdx.x % LP, r0 = threadIdx.x / LP;
   const double sgn = (signed_ && l < a.L) ? c.st->colsign[l] : 1.0;
   const double cs = F == Form::F8 ? f8_col_scale(c.st->cmax_g[l]) : 1.0;
-  for (uint32_t t0 = 0; t0 < it.nrows; t0 += TR) {
-    const int nr = (int)min<uint32_t>(TR, it.nrows - t0);
+  const uint32_t s0 = blockIdx.y * kSliceRows, s1 = min<uint32_t>(it.nrows, s0 + kSliceRows);
+  for (uint32_t t0 = s0; t0 < s1; t0 += TR) {
+    const int nr = (int)min<uint32_t>(TR, s1 - t0);
     for (int r = r0; r < TR; r += 256 / LP) {
       w_t pc[3] = {w_t(0), w_t(0), w_t(0)};
       if (r < nr) {
@@ -127,35 +137,44 @@ __global__ void __launch_bounds__(256) k_b_make_pieces(BatchArgs a, const RowIte
 }
 
 // ---------------------------------------------------------------- row reductions
-// partial[item][l] = sum over the item's rows of X[r][l] (colsum) or the two
-// flipOmg norms (width 2 LP).  8 row groups x 32 columns, combined in order.
+// partial[item][l] = sum over the item's rows of X[r][l] (colsum, 8 row groups)
+// or the two flipOmg norms (width 2 LP, 32 row groups; they only decide
+// signs), the groups combined in order.  A thread's loads are issued sixteen at a
+// time ahead of their additions: colsum 37 -> 11 us, norms 59 -> 19 us at 32
+// cohorts of up to 1,024 rows per item.
 template <bool FLIP>
-__global__ void __launch_bounds__(256) k_b_rowsum(BatchArgs a, const RowItem* __restrict__ items,
-                                                  double* __restrict__ partial) {
+__global__ void __launch_bounds__(FLIP ? 1024 : 256) k_b_rowsum(BatchArgs a, const RowItem* __restrict__ items,
+                                                                double* __restrict__ partial) {
+  constexpr int NG = FLIP ? 32 : 8;
   const RowItem it = items[blockIdx.x];
   const BatchCohort& c = a.coh[it.cohort];
   if (c.st->state != 1) return;
-  __shared__ double red[2][8][LP];
+  __shared__ double red[FLIP ? 2 : 1][NG][LP];
   const int l = threadIdx.x & 31, g = threadIdx.x >> 5;
   double s0 = 0.0, s1 = 0.0;
   if constexpr (FLIP) {
-    const double* o2 = c.mat[kBufOmega];
-    const double* q = c.mat[kBufOmegaC];
-    for (uint32_t rr = g; rr < it.nrows; rr += 8) {
-      const uint64_t t = (it.row0 + rr) * LP + l;
-      s0 += fabs(o2[t] - q[t]);
-      s1 += fabs(o2[t] + q[t]);
+    const double* o2 = c.mat[kBufOmega] + it.row0 * LP + l;
+    const double* q = c.mat[kBufOmegaC] + it.row0 * LP + l;
+#pragma unroll 8
+    for (uint32_t rr = g; rr < it.nrows; rr += NG) {
+      const double o = o2[rr * LP], v = q[rr * LP];
+      s0 += fabs(o - v);
+      s1 += fabs(o + v);
     }
+    red[1][g][l] = s1;
   } else {
-    const double* x = c.mat[kBufOmegaR];
-    for (uint32_t rr = g; rr < it.nrows; rr += 8) s0 += x[(it.row0 + rr) * LP + l];
+    const double* x = c.mat[kBufOmegaR] + it.row0 * LP + l;
+#pragma unroll 16
+    for (uint32_t rr = g; rr < it.nrows; rr += NG) s0 += x[rr * LP];
   }
   red[0][g][l] = s0;
-  red[1][g][l] = s1;
   __syncthreads();
   if (threadIdx.x < LP) {
     double t0 = 0.0, t1 = 0.0;
-    for (int q = 0; q < 8; ++q) t0 += red[0][q][l], t1 += red[1][q][l];
+    for (int q = 0; q < NG; ++q) {
+      t0 += red[0][q][l];
+      if constexpr (FLIP) t1 += red[1][q][l];
+    }
     if constexpr (FLIP) {
       partial[(uint64_t)blockIdx.x * 2 * LP + l] = t0;
       partial[(uint64_t)blockIdx.x * 2 * LP + LP + l] = t1;
@@ -166,13 +185,21 @@ __global__ void __launch_bounds__(256) k_b_rowsum(BatchArgs a, const RowItem* __
 }
 
 // Per cohort: dest = sum over its items (in order) of partial[item][0:width].
+// A workgroup takes 32 of the width's values (grid.y): its 32 thread rows
+// fetch 128 items at a time into LDS, the next ones in flight while one
+// thread per value adds the staged ones in item order.  Bound by the loads'
+// latency: one thread per value that loaded and added item after item, one
+// workgroup per cohort, took 64 us on average at 32 cohorts (up to 98 Gram
+// items and 780 epilogue items each), against 6 us.
 enum SumDest : int { kDestColsum = 0, kDestBvec, kDestGramA, kDestGramH, kDestAb };
 enum ItemList : int { kListM = 0, kListN, kListE };
+constexpr int kSumItems = 128;
 
-__global__ void __launch_bounds__(256) k_b_sum_items(BatchArgs a, const double* __restrict__ partial, int width,
-                                                     int list, int dest, int state_req) {
+__global__ void __launch_bounds__(1024) k_b_sum_items(BatchArgs a, const double* __restrict__ partial, int width,
+                                                      int list, int dest, int state_req) {
   const BatchCohort& c = a.coh[blockIdx.x];
   if (c.st->state != state_req) return;
+  __shared__ double st[kSumItems][32];
   const uint32_t b = list == kListM ? c.m_begin : (list == kListN ? c.n_begin : c.e_begin);
   const uint32_t e = list == kListM ? c.m_end : (list == kListN ? c.n_end : c.e_end);
   double* out = dest == kDestColsum ? c.colsum
@@ -180,11 +207,39 @@ __global__ void __launch_bounds__(256) k_b_sum_items(BatchArgs a, const double* 
                 : dest == kDestGramA ? c.st->gram_a
                 : dest == kDestGramH ? c.st->gram_h
                                      : c.st->ab;
-  for (int v = threadIdx.x; v < width; v += 256) {
-    double s = 0.0;
-    for (uint32_t i = b; i < e; ++i) s += partial[(uint64_t)i * width + v];
-    out[v] = s;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int v = blockIdx.y * 32 + tx;  // width is a multiple of 32
+  constexpr int U = kSumItems / 32;
+  double r[U];
+  auto fetch = [&](uint32_t i0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t i = i0 + 32 * u + ty;
+      r[u] = i < e ? partial[(uint64_t)i * width + v] : 0.0;
+    }
+  };
+  fetch(b);
+  double s = 0.0;
+  for (uint32_t i0 = b; i0 < e; i0 += kSumItems) {
+    __syncthreads();  // the previous items have been added
+#pragma unroll
+    for (int u = 0; u < U; ++u) st[32 * u + ty][tx] = r[u];
+    __syncthreads();
+    fetch(i0 + kSumItems);
+    if (ty == 0) {
+      const int n = (int)min<uint32_t>(kSumItems, e - i0);
+      int k = 0;
+      for (; k + 8 <= n; k += 8) {
+        double x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = st[k + u][tx];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += x[u];
+      }
+      for (; k < n; ++k) s += st[k][tx];
+    }
   }
+  if (ty == 0) out[v] = s;
 }
 
 // ---------------------------------------------------------------- epilogues
@@ -344,7 +399,8 @@ __global__ void k_b_zero_cmax(BatchArgs a, int h_side) {
   (h_side ? c.st->cmax_h : c.st->cmax_g)[threadIdx.x] = 0ull;
 }
 
-// H = y / 4 + b over the item's rows, 4 adjacent elements per thread.
+// H = y / 4 + b over the item's rows, 4 adjacent elements per thread; grid.y:
+// row slices.  Four chunks are loaded ahead of their additions (in chunk order).
 template <class PT>
 __global__ void __launch_bounds__(256) k_b_epi_h(BatchArgs a, const RowItem* __restrict__ items) {
   const RowItem it = items[blockIdx.x];
@@ -352,7 +408,9 @@ __global__ void __launch_bounds__(256) k_b_epi_h(BatchArgs a, const RowItem* __r
   if (c.st->state != 1) return;
   const PT* part = static_cast<const PT*>(c.part);
   double* h = c.mat[kBufH];
-  const int n4 = (int)it.nrows * (LP / 4);
+  const int v0 = blockIdx.y * kSliceRows * (LP / 4);
+  const int n4 = min((int)it.nrows * (LP / 4), v0 + (int)kSliceRows * (LP / 4));
+  if (v0 >= n4) return;
   const int l0 = 4 * (threadIdx.x % (LP / 4));  // the same columns on every pass (256 is a multiple of LP / 4)
   double b[4];
 #pragma unroll
@@ -363,9 +421,10 @@ __global__ void __launch_bounds__(256) k_b_epi_h(BatchArgs a, const RowItem* __r
 #pragma unroll
     for (int q = 0; q < 4; ++q) m[q] = 0.25 * f8_col_scale(c.st->cmax_h[l0 + q]);
   }
-  for (int v = threadIdx.x; v < n4; v += 256) {
+  for (int v = v0 + threadIdx.x; v < n4; v += 256) {
     const uint64_t t = it.row0 * LP + 4 * (uint64_t)v;
     double y[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
     for (uint64_t ch = 0; ch < c.nch_h; ++ch) add4(part + ch * c.ychunk_h + t, y);
     *reinterpret_cast<double2*>(h + t) = double2{m[0] * y[0] + b[0], m[1] * y[1] + b[1]};
     *reinterpret_cast<double2*>(h + t + 2) = double2{m[2] * y[2] + b[2], m[3] * y[3] + b[3]};
@@ -375,12 +434,14 @@ __global__ void __launch_bounds__(256) k_b_epi_h(BatchArgs a, const RowItem* __r
 // ---------------------------------------------------------------- Gram and apply
 constexpr int kTileRows = 32;
 
-// partial[item] = X^T Y over the item's rows (LP x LP), FP64 MFMA; wave wv
-// owns output rows 16 wv .. 16 wv + 15.
+// partial[item] = X^T Y over the item's rows (LP x LP), FP64 MFMA; wave wv owns
+// the 16 x 16 output block (wv / 2, wv % 2).  Bound by the serial chain of an
+// item's MFMAs where the items are few: two waves with two blocks each took 46 us
+// per launch on average at 32 cohorts, against 40 us.
 template <bool CROSS>
-__global__ void __launch_bounds__(128) k_b_gram(BatchArgs a, const RowItem* __restrict__ items, int xsel, int ysel,
+__global__ void __launch_bounds__(256) k_b_gram(BatchArgs a, const RowItem* __restrict__ items, int xsel, int ysel,
                                                 int state_req, double* __restrict__ partial) {
-  constexpr int NB = LP / 16;
+  static_assert(LP == 32, "four 16 x 16 blocks on four waves");
   const RowItem it = items[blockIdx.x];
   const BatchCohort& c = a.coh[it.cohort];
   if (c.st->state != state_req) return;
@@ -390,20 +451,18 @@ __global__ void __launch_bounds__(128) k_b_gram(BatchArgs a, const RowItem* __re
   const double* Y = CROSS ? c.mat[ysel] : X;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int q = lane >> 4, r16 = lane & 15;
-  f64x4_t acc[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) acc[b] = f64x4_t{0, 0, 0, 0};
+  const int ci = 16 * (wv >> 1) + r16, cj = 16 * (wv & 1) + r16;
+  f64x4_t acc{0, 0, 0, 0};
   const uint64_t re = it.row0 + it.nrows;
   // The next row tile is loaded into registers while the current one is
   // multiplied; rows past the item's end read as zero.
-  constexpr int PER = kTileRows * LP / (64 * NB);
-  static_assert(PER * 64 * NB == kTileRows * LP, "whole tiles per thread");
+  constexpr int PER = kTileRows * LP / 256;
   double px[PER], py[CROSS ? PER : 1];
   auto fetch = [&](uint64_t r0) {
     const uint64_t nr = re - r0 < (uint64_t)kTileRows ? re - r0 : kTileRows;
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
-      const int v = tid + e * 64 * NB;
+      const int v = tid + e * 256;
       const bool in = (uint64_t)(v / LP) < nr;
       px[e] = in ? X[r0 * LP + v] : 0.0;
       if constexpr (CROSS) py[e] = in ? Y[r0 * LP + v] : 0.0;
@@ -414,33 +473,26 @@ __global__ void __launch_bounds__(128) k_b_gram(BatchArgs a, const RowItem* __re
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
-      xs[tid + e * 64 * NB] = px[e];
-      if constexpr (CROSS) ys[tid + e * 64 * NB] = py[e];
+      xs[tid + e * 256] = px[e];
+      if constexpr (CROSS) ys[tid + e * 256] = py[e];
     }
     __syncthreads();
     if (r0 + kTileRows < re) fetch(r0 + kTileRows);
     const double* yt = CROSS ? ys : xs;
 #pragma unroll
-    for (int k0 = 0; k0 < kTileRows; k0 += 4) {
-      const double av = xs[(k0 + q) * LP + 16 * wv + r16];
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const double bv = yt[(k0 + q) * LP + 16 * b + r16];
-        acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[b], 0, 0, 0);
-      }
-    }
+    for (int k0 = 0; k0 < kTileRows; k0 += 4)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(xs[(k0 + q) * LP + ci], yt[(k0 + q) * LP + cj], acc, 0, 0, 0);
   }
   double* o = partial + (uint64_t)blockIdx.x * LP * LP;
 #pragma unroll
-  for (int b = 0; b < NB; ++b)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o[(16 * wv + q + 4 * r) * LP + 16 * b + r16] = acc[b][r];
+  for (int r = 0; r < 4; ++r) o[(16 * (wv >> 1) + q + 4 * r) * LP + cj] = acc[r];
 }
 
 // Y = X T for the item's rows, T = t (tsel 0) or tv (tsel 1) of the cohort.
 // Thread (row slot rs, column pair cp) keeps columns 2 cp, 2 cp + 1 of T in
 // registers; X arrives in tiles of 64 rows staged in LDS with coalesced
-// loads, and each output sums its 32 products in column order.
+// loads, and each output sums its 32 products in column order.  grid.y: row
+// slices.
 static_assert(sizeof(BatchSmall) % 16 == 0 && offsetof(BatchSmall, t) % 16 == 0 && offsetof(BatchSmall, tv) % 16 == 0,
               "the transforms are read as 16-byte pairs");
 
@@ -448,8 +500,9 @@ __global__ void __launch_bounds__(256) k_b_apply(BatchArgs a, const RowItem* __r
                                                  int tsel, int state_req) {
   constexpr int TR = 64;
   const RowItem it = items[blockIdx.x];
+  const uint32_t s0 = blockIdx.y * kSliceRows, s1 = min<uint32_t>(it.nrows, s0 + kSliceRows);
   const BatchCohort& c = a.coh[it.cohort];
-  if (c.st->state != state_req) return;
+  if (s0 >= s1 || c.st->state != state_req) return;
   __shared__ double2 xs[TR * LP / 2];
   const double* src = tsel ? c.st->tv : c.st->t;
   const int cp = threadIdx.x & 15, rs = threadIdx.x >> 4;
@@ -462,8 +515,8 @@ __global__ void __launch_bounds__(256) k_b_apply(BatchArgs a, const RowItem* __r
   }
   const double* X = c.mat[xsel];
   double* Y = c.mat[ysel];
-  for (uint32_t r0 = 0; r0 < it.nrows; r0 += TR) {
-    const int nr = (int)min<uint32_t>(TR, it.nrows - r0);
+  for (uint32_t r0 = s0; r0 < s1; r0 += TR) {
+    const int nr = (int)min<uint32_t>(TR, s1 - r0);
     const double2* xg = reinterpret_cast<const double2*>(X + (it.row0 + r0) * LP);
     __syncthreads();  // the previous tile has been read
     for (int v = threadIdx.x; v < nr * LP / 2; v += 256) xs[v] = xg[v];
@@ -837,12 +890,12 @@ void launch_batch_make_pieces(const BatchArgs& a, const RowItem* items_n, uint32
   if (!nitems) return;
   const int sg = signed_ ? 1 : 0;
   switch ((Form)a.form) {
-    case Form::FP64: hipLaunchKernelGGL(k_b_make_pieces<Form::FP64>, dim3(nitems), dim3(256), 0, s, a, items_n, src, sg); break;
-    case Form::FP32: hipLaunchKernelGGL(k_b_make_pieces<Form::FP32>, dim3(nitems), dim3(256), 0, s, a, items_n, src, sg); break;
-    case Form::BF16: hipLaunchKernelGGL(k_b_make_pieces<Form::BF16>, dim3(nitems), dim3(256), 0, s, a, items_n, src, sg); break;
-    case Form::BF16X1: hipLaunchKernelGGL(k_b_make_pieces<Form::BF16X1>, dim3(nitems), dim3(256), 0, s, a, items_n, src, sg); break;
-    case Form::FP16: hipLaunchKernelGGL(k_b_make_pieces<Form::FP16>, dim3(nitems), dim3(256), 0, s, a, items_n, src, sg); break;
-    case Form::F8: hipLaunchKernelGGL(k_b_make_pieces<Form::F8>, dim3(nitems), dim3(256), 0, s, a, items_n, src, sg); break;
+    case Form::FP64: hipLaunchKernelGGL(k_b_make_pieces<Form::FP64>, dim3(nitems, kSlices), dim3(256), 0, s, a, items_n, src, sg); break;
+    case Form::FP32: hipLaunchKernelGGL(k_b_make_pieces<Form::FP32>, dim3(nitems, kSlices), dim3(256), 0, s, a, items_n, src, sg); break;
+    case Form::BF16: hipLaunchKernelGGL(k_b_make_pieces<Form::BF16>, dim3(nitems, kSlices), dim3(256), 0, s, a, items_n, src, sg); break;
+    case Form::BF16X1: hipLaunchKernelGGL(k_b_make_pieces<Form::BF16X1>, dim3(nitems, kSlices), dim3(256), 0, s, a, items_n, src, sg); break;
+    case Form::FP16: hipLaunchKernelGGL(k_b_make_pieces<Form::FP16>, dim3(nitems, kSlices), dim3(256), 0, s, a, items_n, src, sg); break;
+    case Form::F8: hipLaunchKernelGGL(k_b_make_pieces<Form::F8>, dim3(nitems, kSlices), dim3(256), 0, s, a, items_n, src, sg); break;
     case Form::I8: fail(kErrArgument, "batch: no int8 form");
   }
   check_launch("batch_make_pieces");
@@ -859,7 +912,7 @@ void launch_batch_colsum(const BatchArgs& a, const RowItem* items_n, uint32_t ni
                          hipStream_t s) {
   if (!nitems) return;
   hipLaunchKernelGGL(k_b_rowsum<false>, dim3(nitems), dim3(256), 0, s, a, items_n, partial);
-  hipLaunchKernelGGL(k_b_sum_items, dim3(nblocks(a.ncoh)), dim3(256), 0, s, a, partial, LP, (int)kListN,
+  hipLaunchKernelGGL(k_b_sum_items, dim3(nblocks(a.ncoh), LP / 32), dim3(1024), 0, s, a, partial, LP, (int)kListN,
                      (int)kDestColsum, 1);
   check_launch("batch_colsum");
 }
@@ -867,8 +920,8 @@ void launch_batch_colsum(const BatchArgs& a, const RowItem* items_n, uint32_t ni
 void launch_batch_flip(const BatchArgs& a, const RowItem* items_n, uint32_t nitems, double* partial,
                        hipStream_t s) {
   if (!nitems) return;
-  hipLaunchKernelGGL(k_b_rowsum<true>, dim3(nitems), dim3(256), 0, s, a, items_n, partial);
-  hipLaunchKernelGGL(k_b_sum_items, dim3(nblocks(a.ncoh)), dim3(256), 0, s, a, partial, 2 * LP, (int)kListN,
+  hipLaunchKernelGGL(k_b_rowsum<true>, dim3(nitems), dim3(1024), 0, s, a, items_n, partial);
+  hipLaunchKernelGGL(k_b_sum_items, dim3(nblocks(a.ncoh), 2 * LP / 32), dim3(1024), 0, s, a, partial, 2 * LP, (int)kListN,
                      (int)kDestAb, 1);
   check_launch("batch_flip");
 }
@@ -890,7 +943,7 @@ void launch_batch_epi_g(const BatchArgs& a, const RowItem* items_e, uint32_t nit
       break;
     case Form::I8: fail(kErrArgument, "batch: no int8 form");
   }
-  hipLaunchKernelGGL(k_b_sum_items, dim3(nblocks(a.ncoh)), dim3(256), 0, s, a, partial, LP, (int)kListE,
+  hipLaunchKernelGGL(k_b_sum_items, dim3(nblocks(a.ncoh), LP / 32), dim3(1024), 0, s, a, partial, LP, (int)kListE,
                      (int)kDestBvec, 1);
   check_launch("batch_epi_g");
 }
@@ -898,9 +951,9 @@ void launch_batch_epi_g(const BatchArgs& a, const RowItem* items_e, uint32_t nit
 void launch_batch_epi_h(const BatchArgs& a, const RowItem* items_n, uint32_t nitems, hipStream_t s) {
   if (!nitems) return;
   if ((Form)a.form == Form::FP64)
-    hipLaunchKernelGGL(k_b_epi_h<double>, dim3(nitems), dim3(256), 0, s, a, items_n);
+    hipLaunchKernelGGL(k_b_epi_h<double>, dim3(nitems, kSlices), dim3(256), 0, s, a, items_n);
   else
-    hipLaunchKernelGGL(k_b_epi_h<float>, dim3(nitems), dim3(256), 0, s, a, items_n);
+    hipLaunchKernelGGL(k_b_epi_h<float>, dim3(nitems, kSlices), dim3(256), 0, s, a, items_n);
   check_launch("batch_epi_h");
 }
 
@@ -908,10 +961,10 @@ void launch_batch_gram(const BatchArgs& a, const RowItem* items, uint32_t nitems
                        int dest, int state_req, double* partial, hipStream_t s) {
   if (!nitems) return;
   if (ysel < 0)
-    hipLaunchKernelGGL(k_b_gram<false>, dim3(nitems), dim3(128), 0, s, a, items, xsel, xsel, state_req, partial);
+    hipLaunchKernelGGL(k_b_gram<false>, dim3(nitems), dim3(256), 0, s, a, items, xsel, xsel, state_req, partial);
   else
-    hipLaunchKernelGGL(k_b_gram<true>, dim3(nitems), dim3(128), 0, s, a, items, xsel, ysel, state_req, partial);
-  hipLaunchKernelGGL(k_b_sum_items, dim3(nblocks(a.ncoh)), dim3(256), 0, s, a, partial, LP * LP,
+    hipLaunchKernelGGL(k_b_gram<true>, dim3(nitems), dim3(256), 0, s, a, items, xsel, ysel, state_req, partial);
+  hipLaunchKernelGGL(k_b_sum_items, dim3(nblocks(a.ncoh), LP * LP / 32), dim3(1024), 0, s, a, partial, LP * LP,
                      m_rows ? (int)kListM : (int)kListN, dest == 0 ? (int)kDestGramA : (int)kDestGramH, state_req);
   check_launch("batch_gram");
 }
@@ -919,7 +972,7 @@ void launch_batch_gram(const BatchArgs& a, const RowItem* items, uint32_t nitems
 void launch_batch_apply(const BatchArgs& a, const RowItem* items, uint32_t nitems, int xsel, int ysel, int tsel,
                         int state_req, hipStream_t s) {
   if (!nitems) return;
-  hipLaunchKernelGGL(k_b_apply, dim3(nitems), dim3(256), 0, s, a, items, xsel, ysel, tsel, state_req);
+  hipLaunchKernelGGL(k_b_apply, dim3(nitems, kSlices), dim3(256), 0, s, a, items, xsel, ysel, tsel, state_req);
   check_launch("batch_apply");
 }
 

@@ -170,3 +170,30 @@ def test_loadings_order(ctx, svd, m):
     # V is G~'s own left factor: it agrees with A U up to the convergence of the subspace
     for c in range(k):
         assert np.dot(r.V[:, c], proj[:, c]) / np.linalg.norm(proj[:, c]) >= 0.999
+
+
+@pytest.mark.parametrize("form,tol", [("fp64", 1e-10), ("fp8", 1e-4)])
+def test_batch_row_slices(ctx, form, tol):
+    """Cohorts whose rows fall on and beside the batched kernels' slices (128), items (1,024) and sums of 128
+    items, against the single-matrix FP64 runs."""
+    dims = [(20, 127), (127, 128), (128, 129), (129, 1023), (1024, 1024), (1025, 16385), (2049, 40), (4100, 300)]
+    say(f"batch row slices {form}")
+    rng = np.random.default_rng(5)
+    cohorts = []
+    for n, m in dims:
+        codes = random_codes(rng, m, n, 0.0)
+        codes[: m // 3, : n // 3] = 0
+        codes[m // 2:, n // 2:] = 3
+        cohorts.append((pack(codes), n))
+    k = 3
+    kw = dict(svd=1, k=k, oversamples=10, maxp=5, tol=0.0)
+    ctx.batch_upload(cohorts)
+    r = ctx.batch_run(precision=form, kchunk_g=4096, kchunk_h=8192, **kw)
+    assert np.all(r["status"] == 0)
+    for c, (rows, n) in enumerate(cohorts):
+        ctx.upload_packed(rows, n)
+        one = ctx.run(precision="fp64", **kw)
+        np.testing.assert_allclose(r["S"][c], one.S, rtol=tol)
+        U = ctx.batch_get_u(c)
+        # the two structured components, which the passes have converged
+        assert np.all(np.abs((U * one.U).sum(0))[:2] >= 1 - tol)
