@@ -10,12 +10,12 @@
 #include "batch_kernels.hpp"
 #include "bf16.hpp"
 #include "device.hpp"
+#include "small_la.hpp"
 
 namespace pcaone {
 namespace {
 
 constexpr int LP = kBatchLp;
-typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
 // Kernels whose rows are independent of each other take an item of up to
 // kBatchRowsPerItem rows in slices of kSliceRows (grid.y): the items of the N
@@ -543,112 +543,137 @@ __global__ void k_b_active(BatchArgs a, int* __restrict__ active) {
 }
 
 // ---------------------------------------------------------------- L x L steps
-// Matrices in LDS, n x n in the top-left of LP x LP row-major storage.  Every
-// helper is called by all threads of the workgroup and ends synchronized.
+// One workgroup per cohort, matrices in LDS with rows of P values, zero outside
+// n x n.  Serial chains of square roots and divisions bound them: the Cholesky
+// factors run in one wave per 16 pivots (small_la.hpp), the inverses one column
+// per lane, the products as MFMAs (the same sums in the same order as a loop
+// over k), the Jacobi rotations from two reciprocal roots.  32 cohorts, L = 20:
+// 91 us per launch over all modes as loops over LDS with a thread-0 part in every
+// pivot, sweep and stop test, against 34 us.
 constexpr int kSmallThreads = 256;
+constexpr int SNB = LP / 16;
+constexpr int P = kLP<SNB>;
 
-__device__ void sm_zero(double* A) {
-  for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) A[v] = 0.0;
+// C = op(A) B with op = transpose when TA; one 16 x 16 block per wave.  C may
+// not overlap A or B.  Ends synchronized.
+template <bool TA>
+__device__ __forceinline__ void sm_mul(double* C, const double* A, const double* B) {
+  static_assert(kSmallThreads / 64 == SNB * SNB, "one block per wave");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, r16 = lane & 15;
+  const int bi = wave / SNB, bj = wave % SNB;
+  f64x4_t acc{0, 0, 0, 0};
+#pragma unroll
+  for (int k = 0; k < LP; k += 4)
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(TA ? A[(k + q) * P + 16 * bi + r16] : A[(16 * bi + r16) * P + k + q],
+                                               B[(k + q) * P + 16 * bj + r16], acc, 0, 0, 0);
+  block_store<SNB>(C, acc, bi, bj, lane);
   __syncthreads();
 }
 
-__device__ void sm_load(double* A, const double* g) {
-  for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) A[v] = g[v];
+// Zeroes the block below the diagonal blocks (lds_chol_upper leaves it alone).
+__device__ __forceinline__ void sm_upper(double* A) {
+  for (int v = threadIdx.x; v < 256; v += kSmallThreads) A[(16 + v / 16) * P + v % 16] = 0.0;
   __syncthreads();
 }
 
-__device__ void sm_store(double* g, const double* A) {
-  for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) g[v] = A[v];
-  __syncthreads();
-}
-
-// C = op(A) B with op = transpose when ta (n x n), entries outside n x n zero.
-__device__ void sm_mul(double* C, const double* A, const double* B, int n, bool ta) {
-  for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) {
-    const int i = v / LP, j = v % LP;
-    double s = 0.0;
-    if (i < n && j < n)
-      for (int m = 0; m < n; ++m) s += (ta ? A[m * LP + i] : A[i * LP + m]) * B[m * LP + j];
-    C[v] = s;
-  }
-  __syncthreads();
-}
-
-// Upper Cholesky factor R (A = R^T R).  Returns false on breakdown (a pivot
-// that is not positive and finite), the criterion of the host factorization.
-__device__ bool sm_chol(double* R, const double* A, int n, int* flag) {
-  sm_zero(R);
-  if (threadIdx.x == 0) *flag = 1;
-  __syncthreads();
-  for (int j = 0; j < n; ++j) {
-    if (threadIdx.x == 0) {
-      double d = A[j * LP + j];
-      for (int k = 0; k < j; ++k) d -= R[k * LP + j] * R[k * LP + j];
-      if (!(d > 0.0) || !isfinite(d)) {
-        *flag = 0;
-        d = 1.0;
-      }
-      R[j * LP + j] = sqrt(d);
-    }
-    __syncthreads();
-    const double rjj = R[j * LP + j];
-    for (int i = j + 1 + (int)threadIdx.x; i < n; i += kSmallThreads) {
-      double s = A[j * LP + i];
-      for (int k = 0; k < j; ++k) s -= R[k * LP + j] * R[k * LP + i];
-      R[j * LP + i] = s / rjj;
-    }
-    __syncthreads();
-  }
-  const bool ok = *flag != 0;
-  __syncthreads();
-  return ok;
-}
-
-// X = R^-1 for upper triangular R, one column per thread.
+// X = R^-1 for the upper R (zero outside n x n): lane j of wave 0 holds column
+// j; X[i][j] = -(sum_{k = i+1}^{j} R[i][k] X[k][j]) / R[i][i], k ascending.
+// Ends synchronized.
 __device__ void sm_inv_upper(double* X, const double* R, int n) {
-  sm_zero(X);
-  for (int j = threadIdx.x; j < n; j += kSmallThreads) {
-    X[j * LP + j] = 1.0 / R[j * LP + j];
-    for (int i = j - 1; i >= 0; --i) {
-      double s = 0.0;
-      for (int k = i + 1; k <= j; ++k) s += R[i * LP + k] * X[k * LP + j];
-      X[i * LP + j] = -s / R[i * LP + i];
+  if (threadIdx.x < LP) {
+    const int j = threadIdx.x;
+    double x[LP];
+#pragma unroll
+    for (int i = LP - 1; i >= 0; --i) {
+      x[i] = 0.0;
+      if (i < n) {
+        double t = 0.0;
+#pragma unroll
+        for (int k = i + 1; k < LP; ++k) t = fma(R[i * P + k], x[k], t);
+        const double v = (i == j ? 1.0 : -t) / R[i * P + i];
+        x[i] = i <= j && j < n ? v : 0.0;
+      }
     }
+#pragma unroll
+    for (int i = 0; i < LP; ++i) X[i * P + j] = x[i];
   }
   __syncthreads();
 }
+
+// 1 / sqrt(x) for x well inside the FP64 range: the hardware's estimate and
+// two Newton steps y += y (1 - x y^2) / 2.
+__device__ __forceinline__ double rsqrt_newton(double x) {
+  double y = __builtin_amdgcn_rsq(x);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+  return y;
+}
+
+// The rotation (c, s) that zeroes apq: c^2 = (1 + |d| / r) / 2 and s = sign(d) h /
+// (2 r c) with d = aqq - app, h = 2 apq, r = sqrt(d^2 + h^2), i.e. the smaller of
+// the two angles.
+__device__ __forceinline__ void jacobi_rotation(double app, double aqq, double apq, double& c, double& s) {
+  const double d = aqq - app, h = 2.0 * apq;
+  const double r2 = fma(d, d, h * h);
+  if (r2 > 1e-280 && r2 < 1e280) {
+    const double ir = rsqrt_newton(r2);
+    const double c2 = fma(0.5 * fabs(d), ir, 0.5);
+    const double ic = rsqrt_newton(c2);
+    c = c2 * ic;
+    s = copysign(0.5, d) * h * ir * ic;
+  } else {
+    const double tau = d / h, at = fabs(tau);
+    // t = sign(tau) / (|tau| + sqrt(1 + tau^2)), ~ 1 / (2 tau) where tau^2 would overflow
+    const double t = (tau >= 0.0 ? 1.0 : -1.0) / (at > 1e150 ? 2.0 * at : at + sqrt(1.0 + at * at));
+    c = 1.0 / sqrt(1.0 + t * t);
+    s = t * c;
+  }
+}
+
+struct JacobiPairs {
+  double c[LP / 2], s[LP / 2];
+  int p[LP / 2], q[LP / 2];
+};
 
 // Symmetric eigen-decomposition of A (destroyed) by cyclic Jacobi rotations
 // in round-robin order (n/2 disjoint pairs per step); w descending, V columns
-// the eigenvectors in the same order.
-__device__ void sm_sym_eig(double* A, double* V, double* w, double* tmp, int n, double* rot, int* perm) {
-  const int ne = n + (n & 1);  // even number of players; index n (if odd) is a dummy
-  for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) V[v] = (v / LP == v % LP && v / LP < n) ? 1.0 : 0.0;
-  // symmetrize
-  for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) {
+// the eigenvectors in the same order.  Per step one thread per pair of pairs
+// rotates the four entries where they meet from both sides.
+__device__ void sm_sym_eig(double* A, double* V, double* w, double* tmp, int n, JacobiPairs* jp, int* perm,
+                           double* red) {
+  const int tid = threadIdx.x;
+  const int ne = n + (n & 1);  // even number of players; index n (if odd) is a dummy row of zeros
+  const int np = ne / 2;
+  for (int v = tid; v < LP * LP; v += kSmallThreads) {
     const int i = v / LP, j = v % LP;
-    tmp[v] = (i < n && j < n) ? 0.5 * (A[i * LP + j] + A[j * LP + i]) : 0.0;
+    V[i * P + j] = i == j && i < n ? 1.0 : 0.0;
+    tmp[i * P + j] = i < n && j < n ? 0.5 * (A[i * P + j] + A[j * P + i]) : 0.0;
   }
   __syncthreads();
-  for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) A[v] = tmp[v];
+  for (int v = tid; v < LP * LP; v += kSmallThreads) A[v / LP * P + v % LP] = tmp[v / LP * P + v % LP];
   __syncthreads();
-  __shared__ double offn;
   for (int sweep = 0; sweep < 40; ++sweep) {
-    if (threadIdx.x == 0) {
-      double off = 0.0, tot = 0.0;
-      for (int i = 0; i < n; ++i)
-        for (int j = 0; j < n; ++j) {
-          const double x = A[i * LP + j] * A[i * LP + j];
-          tot += x;
-          if (i != j) off += x;
-        }
-      offn = (off <= 1e-30 * tot || tot == 0.0) ? -1.0 : off;  // off-norm <= 1e-15 of the norm
+    double off = 0.0, tot = 0.0;
+#pragma unroll
+    for (int u = 0; u < LP * LP / kSmallThreads; ++u) {
+      const int v = tid + u * kSmallThreads, i = v / LP, j = v % LP;
+      const double x = A[i * P + j] * A[i * P + j];
+      tot += x;
+      off += i != j ? x : 0.0;
     }
+    for (int d = 32; d > 0; d >>= 1) {
+      off += __shfl_xor(off, d);
+      tot += __shfl_xor(tot, d);
+    }
+    if ((tid & 63) == 0) red[tid >> 6] = off, red[4 + (tid >> 6)] = tot;
     __syncthreads();
-    if (offn < 0.0) break;
+    off = (red[0] + red[1]) + (red[2] + red[3]);
+    tot = (red[4] + red[5]) + (red[6] + red[7]);
+    if (off <= 1e-30 * tot || tot == 0.0) break;  // off-norm <= 1e-15 of the norm
     for (int step = 0; step < ne - 1; ++step) {
       // pairs of the round-robin schedule: player 0 fixed, others rotate
-      for (int k = threadIdx.x; k < ne / 2; k += kSmallThreads) {
+      if (tid < np) {
+        const int k = tid;
         int p = k == 0 ? 0 : 1 + (k - 1 + step) % (ne - 1);
         int q = 1 + (ne - 2 - k + step) % (ne - 1);
         if (p > q) {
@@ -657,109 +682,76 @@ __device__ void sm_sym_eig(double* A, double* V, double* w, double* tmp, int n, 
           q = t;
         }
         double c = 1.0, s = 0.0;
-        if (q < n) {
-          const double apq = A[p * LP + q];
-          if (apq != 0.0) {
-            const double tau = (A[q * LP + q] - A[p * LP + p]) / (2.0 * apq);
-            const double at = fabs(tau);
-            // t = sign(tau) / (|tau| + sqrt(1 + tau^2)), ~ 1 / (2 tau) where tau^2 would overflow
-            const double t = (tau >= 0.0 ? 1.0 : -1.0) / (at > 1e150 ? 2.0 * at : at + sqrt(1.0 + at * at));
-            c = 1.0 / sqrt(1.0 + t * t);
-            s = t * c;
-          }
+        const double apq = A[p * P + q];
+        if (q < n && apq != 0.0) jacobi_rotation(A[p * P + p], A[q * P + q], apq, c, s);
+        jp->p[k] = p;
+        jp->q[k] = q;
+        jp->c[k] = c;
+        jp->s[k] = s;
+      }
+      __syncthreads();
+      const int k1 = tid >> 4, k2 = tid & 15;
+      if (k1 < np && k2 < np) {  // A <- J^T A J
+        const int p1 = jp->p[k1], q1 = jp->q[k1], p2 = jp->p[k2], q2 = jp->q[k2];
+        const double c1 = jp->c[k1], s1 = jp->s[k1], c2 = jp->c[k2], s2 = jp->s[k2];
+        const double app = A[p1 * P + p2], apq = A[p1 * P + q2], aqp = A[q1 * P + p2], aqq = A[q1 * P + q2];
+        const double xpp = c2 * app - s2 * apq, xpq = s2 * app + c2 * apq;
+        const double xqp = c2 * aqp - s2 * aqq, xqq = s2 * aqp + c2 * aqq;
+        A[p1 * P + p2] = c1 * xpp - s1 * xqp;
+        A[p1 * P + q2] = c1 * xpq - s1 * xqq;
+        A[q1 * P + p2] = s1 * xpp + c1 * xqp;
+        A[q1 * P + q2] = s1 * xpq + c1 * xqq;
+      }
+      for (int k = k1; k < np; k += 16) {  // V <- V J, rows k2 and k2 + 16
+        const int p = jp->p[k], q = jp->q[k];
+        const double c = jp->c[k], s = jp->s[k];
+#pragma unroll
+        for (int i = k2; i < LP; i += 16) {
+          const double vip = V[i * P + p], viq = V[i * P + q];
+          V[i * P + p] = c * vip - s * viq;
+          V[i * P + q] = s * vip + c * viq;
         }
-        perm[2 * k] = p;
-        perm[2 * k + 1] = q;
-        rot[2 * k] = c;
-        rot[2 * k + 1] = s;
-      }
-      __syncthreads();
-      // A <- A J (column pairs), V <- V J
-      for (int v = threadIdx.x; v < (ne / 2) * n; v += kSmallThreads) {
-        const int k = v / n, i = v % n;
-        const int p = perm[2 * k], q = perm[2 * k + 1];
-        if (q >= n) continue;
-        const double c = rot[2 * k], s = rot[2 * k + 1];
-        const double aip = A[i * LP + p], aiq = A[i * LP + q];
-        A[i * LP + p] = c * aip - s * aiq;
-        A[i * LP + q] = s * aip + c * aiq;
-        const double vip = V[i * LP + p], viq = V[i * LP + q];
-        V[i * LP + p] = c * vip - s * viq;
-        V[i * LP + q] = s * vip + c * viq;
-      }
-      __syncthreads();
-      // A <- J^T A (row pairs)
-      for (int v = threadIdx.x; v < (ne / 2) * n; v += kSmallThreads) {
-        const int k = v / n, j = v % n;
-        const int p = perm[2 * k], q = perm[2 * k + 1];
-        if (q >= n) continue;
-        const double c = rot[2 * k], s = rot[2 * k + 1];
-        const double apj = A[p * LP + j], aqj = A[q * LP + j];
-        A[p * LP + j] = c * apj - s * aqj;
-        A[q * LP + j] = s * apj + c * aqj;
       }
       __syncthreads();
     }
   }
-  // sort descending (stable selection on one thread), permute V's columns
-  if (threadIdx.x == 0) {
-    for (int i = 0; i < n; ++i) perm[i] = i;
-    for (int i = 0; i < n; ++i) {
-      int b = i;
-      for (int j = i + 1; j < n; ++j)
-        if (A[perm[j] * LP + perm[j]] > A[perm[b] * LP + perm[b]]) b = j;
-      const int t = perm[i];
-      perm[i] = perm[b];
-      perm[b] = t;
+  // descending order: an eigenvalue's rank counts the larger ones (and equal ones before it)
+  __syncthreads();
+  if (tid < n) {
+    const double x = A[tid * P + tid];
+    int r = 0;
+    for (int j = 0; j < n; ++j) {
+      const double y = A[j * P + j];
+      r += y > x || (y == x && j < tid) ? 1 : 0;
     }
-    for (int i = 0; i < n; ++i) w[i] = A[perm[i] * LP + perm[i]];
+    perm[r] = tid;
+    w[r] = x;
   }
   __syncthreads();
-  for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) {
+  for (int v = tid; v < LP * LP; v += kSmallThreads) {
     const int i = v / LP, j = v % LP;
-    tmp[v] = (i < n && j < n) ? V[i * LP + perm[j]] : 0.0;
+    tmp[i * P + j] = i < n && j < n ? V[i * P + perm[j]] : 0.0;
   }
   __syncthreads();
-  for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) V[v] = tmp[v];
+  for (int v = tid; v < LP * LP; v += kSmallThreads) V[v / LP * P + v % LP] = tmp[v / LP * P + v % LP];
   __syncthreads();
-}
-
-// Householder-convention column signs of the thin Q whose top n x n block is
-// Y (destroyed): a modified LU without pivoting (Ballard et al., 2014).
-__device__ void sm_householder_signs(double* W, int n, double* s) {
-  for (int i = 0; i < n; ++i) {
-    if (threadIdx.x == 0) {
-      s[i] = W[i * LP + i] >= 0.0 ? -1.0 : 1.0;
-      W[i * LP + i] -= s[i];
-    }
-    __syncthreads();
-    const double piv = W[i * LP + i];
-    for (int r = i + 1 + (int)threadIdx.x; r < n; r += kSmallThreads) {
-      W[r * LP + i] /= piv;
-      const double lr = W[r * LP + i];
-      if (lr == 0.0) continue;
-      for (int c = i + 1; c < n; ++c) W[r * LP + c] -= lr * W[i * LP + c];
-    }
-    __syncthreads();
-  }
 }
 
 __global__ void __launch_bounds__(kSmallThreads) k_b_small(BatchArgs a, int mode, int epoch) {
-  extern __shared__ __align__(16) double smem[];
-  double* M0 = smem;
-  double* M1 = M0 + LP * LP;
-  double* M2 = M1 + LP * LP;
-  double* M3 = M2 + LP * LP;
-  double* M4 = M3 + LP * LP;
-  double* M5 = M4 + LP * LP;
-  double* vec = M5 + LP * LP;   // 2 LP
-  double* rot = vec + 2 * LP;   // LP
-  __shared__ int flag;
-  __shared__ int perm[LP];
+  __shared__ __align__(16) double mats[5][LP * P];
+  __shared__ double vec[LP], red[8], min_pivot;
+  __shared__ JacobiPairs jp;
+  __shared__ int flag, perm[LP];
+  double *M0 = mats[0], *M1 = mats[1], *M2 = mats[2], *M3 = mats[3], *M4 = mats[4];
   const BatchCohort& c = a.coh[blockIdx.x];
   BatchSmall* st = c.st;
   const int state = st->state;
   const int L = a.L, k = a.k;
+  const auto load = [&](double* M, const double* src, bool upper) { lds_load<SNB, kSmallThreads>(M, src, L, upper); };
+  const auto chol = [&](double* M) { return lds_chol_upper<SNB, kSmallThreads, true>(M, L, &min_pivot, &flag); };
+  const auto store = [&](double* dst, const double* M) {
+    for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) dst[v] = M[v / LP * P + v % LP];
+  };
   if (mode == kSmallFinish) {
     if (threadIdx.x == 0 && state == 2) st->state = 0;
     return;
@@ -778,46 +770,53 @@ __global__ void __launch_bounds__(kSmallThreads) k_b_small(BatchArgs a, int mode
   if (state != 1) return;
   if (mode == kSmallEpoch) {
     // R = R2 R1 from the Gram of G~ (CholeskyQR2, second factor on the small side)
-    sm_load(M0, st->gram_a);
-    if (!sm_chol(M1, M0, L, &flag)) {
+    load(M0, st->gram_a, false);
+    load(M1, st->gram_a, true);
+    __syncthreads();
+    if (!chol(M1)) {
       if (threadIdx.x == 0) st->state = -5;
       return;
     }
     sm_inv_upper(M2, M1, L);
-    sm_mul(M3, M0, M2, L, false);  // Ga R1^-1
-    sm_mul(M4, M2, M3, L, true);   // R1^-T Ga R1^-1
-    if (!sm_chol(M3, M4, L, &flag)) {
+    sm_mul<false>(M3, M0, M2);  // Ga R1^-1
+    sm_mul<true>(M4, M2, M3);   // R1^-T Ga R1^-1
+    sm_upper(M4);
+    if (!chol(M4)) {
       if (threadIdx.x == 0) st->state = -5;
       return;
     }
-    sm_mul(M4, M3, M1, L, false);  // R = R2 R1
-    sm_inv_upper(M0, M4, L);       // R^-1
+    sm_mul<false>(M3, M4, M1);  // R = R2 R1
+    sm_inv_upper(M0, M3, L);    // R^-1
     // C = R^-T (H^T H) R^-1
-    sm_load(M1, st->gram_h);
-    sm_mul(M2, M1, M0, L, false);
-    sm_mul(M1, M0, M2, L, true);
-    sm_sym_eig(M1, M2, vec, M3, L, rot, perm);  // M2 = W, vec = eigenvalues (descending)
+    load(M1, st->gram_h, false);
+    __syncthreads();
+    sm_mul<false>(M2, M1, M0);
+    sm_mul<true>(M1, M0, M2);
+    sm_sym_eig(M1, M2, vec, M3, L, &jp, perm, red);  // M2 = W, vec = eigenvalues (descending)
     for (int i = threadIdx.x; i < LP; i += kSmallThreads)
       st->sigma[i] = i < L ? sqrt(vec[i] > 0.0 ? vec[i] : 0.0) : 0.0;
-    sm_mul(M3, M0, M2, L, false);  // R^-1 W
+    sm_mul<false>(M3, M0, M2);  // R^-1 W
     for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) {
       const int i = v / LP, j = v % LP;
-      const double rw = (i < L && j < k) ? M3[v] : 0.0;
+      const double rw = (i < L && j < k) ? M3[i * P + j] : 0.0;
       const double sg = j < L ? sqrt(vec[j] > 0.0 ? vec[j] : 0.0) : 0.0;
       st->tv[v] = rw;
       st->t[v] = sg > 0.0 ? rw / sg : 0.0;
     }
   } else if (mode == kSmallStop) {
+    // 1 - mev(Ucur, Upre), mev = (1/k) sum_i || Ucur^T upre_i ||: one thread per column
+    if (epoch > 0 && (int)threadIdx.x < k) {
+      double s2 = 0.0;
+#pragma unroll 8
+      for (int r = 0; r < k; ++r) s2 += st->gram_a[r * LP + threadIdx.x] * st->gram_a[r * LP + threadIdx.x];
+      vec[threadIdx.x] = sqrt(s2);
+    }
+    __syncthreads();
     if (threadIdx.x == 0) {
       bool stop = false;
       if (epoch > 0) {
-        // 1 - mev(Ucur, Upre), mev = (1/k) sum_i || Ucur^T upre_i ||
         double m = 0.0;
-        for (int i = 0; i < k; ++i) {
-          double s2 = 0.0;
-          for (int r = 0; r < k; ++r) s2 += st->gram_a[r * LP + i] * st->gram_a[r * LP + i];
-          m += sqrt(s2);
-        }
+        for (int i = 0; i < k; ++i) m += vec[i];
         const double diff = 1.0 - m / k;
         if (epoch < kBatchMaxEpochs) st->trace[epoch] = diff;
         stop = diff < a.tol || epoch == a.p;
@@ -833,35 +832,31 @@ __global__ void __launch_bounds__(kSmallThreads) k_b_small(BatchArgs a, int mode
       }
     }
   } else if (mode == kSmallOmega1) {
-    sm_load(M0, st->gram_h);
-    if (!sm_chol(M1, M0, L, &flag)) {
-      if (threadIdx.x == 0) st->state = -5;
-      return;
-    }
-    sm_store(st->r1h, M1);
-    sm_inv_upper(M2, M1, L);
-    sm_store(st->t, M2);
-  } else if (mode == kSmallOmega2) {
-    sm_load(M0, st->gram_a);  // Gram of Q1 = H R1^-1
-    if (!sm_chol(M1, M0, L, &flag)) {
-      if (threadIdx.x == 0) st->state = -5;
-      return;
-    }
-    sm_load(M2, st->r1h);
-    sm_mul(M3, M1, M2, L, false);  // R2 R1
-    sm_inv_upper(M0, M3, L);       // Rinv
-    // top L x L block of Q = H Rinv
-    const double* H = c.mat[kBufH];
-    for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) {
-      const int i = v / LP, j = v % LP;
-      M2[v] = (i < L && j < L) ? H[(uint64_t)i * LP + j] : 0.0;
-    }
+    load(M1, st->gram_h, true);
     __syncthreads();
-    sm_mul(M4, M2, M0, L, false);
-    sm_householder_signs(M4, L, vec);
+    if (!chol(M1)) {
+      if (threadIdx.x == 0) st->state = -5;
+      return;
+    }
+    store(st->r1h, M1);
+    sm_inv_upper(M2, M1, L);
+    store(st->t, M2);
+  } else if (mode == kSmallOmega2) {
+    load(M1, st->gram_a, true);  // Gram of Q1 = H R1^-1
+    load(M2, st->r1h, true);
+    load(M4, c.mat[kBufH], false);  // top L x L block of H
+    __syncthreads();
+    if (!chol(M1)) {
+      if (threadIdx.x == 0) st->state = -5;
+      return;
+    }
+    sm_mul<false>(M3, M1, M2);  // R2 R1
+    sm_inv_upper(M0, M3, L);    // Rinv
+    sm_mul<false>(M2, M4, M0);  // top block of Q = H Rinv
+    lds_householder_signs<SNB, kSmallThreads>(M2, L, vec);
     for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) {
       const int j = v % LP;
-      st->t[v] = j < L ? M0[v] * vec[j] : 0.0;
+      st->t[v] = j < L ? M0[v / LP * P + j] * vec[j] : 0.0;
     }
   } else if (mode == kSmallFlip) {
     for (int l = threadIdx.x; l < LP; l += kSmallThreads)
@@ -874,14 +869,7 @@ unsigned nblocks(uint32_t n) { return n ? n : 1; }
 }  // namespace
 
 void launch_batch_small(const BatchArgs& a, int mode, int epoch, hipStream_t s) {
-  constexpr size_t lds = (6 * LP * LP + 3 * LP) * sizeof(double);
-  static bool attr = false;
-  if (!attr) {
-    PCAONE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_b_small),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    attr = true;
-  }
-  hipLaunchKernelGGL(k_b_small, dim3(a.ncoh), dim3(kSmallThreads), lds, s, a, mode, epoch);
+  hipLaunchKernelGGL(k_b_small, dim3(a.ncoh), dim3(kSmallThreads), 0, s, a, mode, epoch);
   check_launch("batch_small");
 }
 

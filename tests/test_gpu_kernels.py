@@ -197,3 +197,27 @@ def test_batch_row_slices(ctx, form, tol):
         U = ctx.batch_get_u(c)
         # the two structured components, which the passes have converged
         assert np.all(np.abs((U * one.U).sum(0))[:2] >= 1 - tol)
+
+
+@pytest.mark.parametrize("k,os", [(1, 10), (5, 10), (5, 11), (6, 11), (10, 11), (10, 21), (16, 16)])
+def test_batch_small_steps(ctx, k, os):
+    """The batched L x L steps at L = 11 .. 32, odd and even, beside and past the 16-pivot panels: all singular
+    values, U and V of a cohort against the single-matrix FP64 run (host eigen-solver, other L x L kernels)."""
+    L = k + max(k, os)
+    say(f"batch small steps L={L}")
+    rng = np.random.default_rng(L)
+    n, m = 300, 900
+    codes = random_codes(rng, m, n, 0.0)
+    for g in range(5):
+        codes[g::6, g * 50:g * 50 + 50 - 7 * g] = 2 * (g % 2)
+    kw = dict(svd=1, k=k, oversamples=os, maxp=4, tol=0.0, precision="fp64")
+    ctx.batch_upload([(pack(codes), n)])
+    r = ctx.batch_run(want_v=True, **kw)
+    assert r["status"][0] == 0 and r["epochs"][0] == 5
+    ctx.upload_packed(pack(codes), n)
+    one = ctx.run(want_v=True, **kw)
+    # both solve the same L x L problems in FP64; neighbouring noise components are a percent apart
+    np.testing.assert_allclose(r["S"][0], one.S, rtol=1e-11)
+    for x, y in ((ctx.batch_get_u(0), one.U), (ctx.batch_get_v(0), one.V)):
+        np.testing.assert_allclose(np.abs((x * y).sum(0)), 1.0, rtol=1e-9)
+    np.testing.assert_allclose(ctx.batch_trace(0), one.trace, atol=1e-11)
