@@ -682,6 +682,7 @@ int pcaone_packed_gemm(pcaone_ctx* c, int precision, const uint8_t* rows, uint64
     a.k_end = K;
     a.kchunk = K;
     a.lp = lp;
+    a.ncols = (int)L;
     launch_packed_gemm(f, shape, a, x.stream);
     std::vector<unsigned char> h(out.bytes());
     std::vector<double> mul(128, 1.0);

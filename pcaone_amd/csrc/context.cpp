@@ -795,6 +795,7 @@ void Context::sketch(uint64_t j0, uint64_t j1, int hmode) {
   g.k_end = ks_;
   g.kchunk = pg.kchunk;
   g.lp = lp;
+  g.ncols = L;
   require(jl + g.rows <= rows_s_, kErrInternal, "G window exceeds padded rows");
   run_gemm(true, pg.shape, pg.nchunks, g);
   const uint64_t nch_g = pg.nchunks;
@@ -898,6 +899,7 @@ void Context::h_half(uint64_t j0, uint64_t j1, int hmode) {
   h.k_end = klen;
   h.kchunk = ph.kchunk;
   h.lp = lp;
+  h.ncols = L;
   require(h.rows <= rows_t_, kErrInternal, "H rows exceed padding");
   run_gemm(false, ph.shape, ph.nchunks, h);
   const uint64_t nch_h = ph.nchunks;

@@ -84,6 +84,7 @@ struct GemmArgs {
   uint64_t k_end;      // one past the last code (multiple of kKStep)
   uint64_t kchunk;     // codes per chunk (multiple of kKStep)
   int lp;              // padded number of columns (multiple of 16, <= 128)
+  int ncols = 0;       // columns in use (0 = lp); W is zero in the others
 };
 
 // Grouped (batched) form: many independent products in one persistent launch.
@@ -117,6 +118,10 @@ inline int gemm_row_tile(const GemmShape& g) { return g.waves * g.wm * 16; }
 GemmShape gemm_default_shape(Form f, int lp);
 bool gemm_shape_supported(Form f, const GemmShape& g, int lp);
 void launch_packed_gemm(Form f, const GemmShape& g, const GemmArgs& a, hipStream_t s);
+// The FP32 form with the last, short block of columns in groups of 4: false
+// (nothing launched) unless the waves own 64 rows and ncols is 17..28 (lp 32)
+// or 33..40 (lp 48).  With one group less to save (41..44) the fragments spill.
+bool launch_packed_gemm_f32_r4(const GemmShape& g, const GemmArgs& a, hipStream_t s);
 // `grid` workgroups walk the item list (rows of every item are a whole tile of g).
 void launch_grouped_gemm(Form f, const GemmShape& g, int lp, const GroupedGemmArgs& a, unsigned grid,
                          hipStream_t s);

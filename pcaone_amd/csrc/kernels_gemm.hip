@@ -24,6 +24,7 @@
 
 #include "device.hpp"
 #include "gemm.hpp"
+#include "gemm_decode.hpp"
 
 namespace pcaone {
 namespace {
@@ -39,14 +40,8 @@ typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 
 constexpr size_t kLdsMax = 160 * 1024;
 
-// code -> top byte of v in BF16/FP32/FP64: 00 -> +2 (0x40), 01 -> 0, 10 -> 0, 11 -> -2 (0xC0)
-constexpr uint32_t kLutTopByte = 0xC0000040u;
-
 // code -> int8 v/2: 00 -> +1, 01 -> 0, 10 -> 0, 11 -> -1
 constexpr uint32_t kLutI8 = 0xFF000001u;
-
-__device__ __forceinline__ uint32_t spread(uint32_t w, int t) { return (w >> (2 * t)) & 0x03030303u; }
-__device__ __forceinline__ uint32_t top_bytes(uint32_t codes4) { return __builtin_amdgcn_perm(0u, kLutTopByte, codes4); }
 
 // Sixteen int8 values v/2 (codes 0..15 of word w, in order).
 __device__ __forceinline__ i32x4_t decode_i8x16(uint32_t w) {
@@ -66,11 +61,6 @@ __device__ __forceinline__ bf16x8_t decode_bf16x8(uint32_t w, int half) {
   d[2] = __builtin_amdgcn_perm(h1, h1, 0x050C040Cu);
   d[3] = __builtin_amdgcn_perm(h1, h1, 0x070C060Cu);
   return __builtin_bit_cast(bf16x8_t, d);
-}
-
-// Top 32 bits of the FP32/FP64 value of byte e of `tb` (other bytes zero).
-__device__ __forceinline__ uint32_t top_word(uint32_t tb, int e) {
-  return __builtin_amdgcn_perm(tb, tb, ((uint32_t)(4 + e) << 24) | 0x0C0C0Cu);
 }
 
 template <Form F>
@@ -881,7 +871,9 @@ void launch_packed_gemm(Form f, const GemmShape& g, const GemmArgs& a, hipStream
   if (a.rows == 0 || a.k_end <= a.k_begin) return;
   switch (f) {
     case Form::FP64: return launch_shape<Form::FP64>(g, a, s);
-    case Form::FP32: return launch_shape<Form::FP32>(g, a, s);
+    case Form::FP32:
+      if (launch_packed_gemm_f32_r4(g, a, s)) return;
+      return launch_shape<Form::FP32>(g, a, s);
     case Form::BF16: return launch_shape<Form::BF16>(g, a, s);
     case Form::BF16X1: return launch_shape<Form::BF16X1>(g, a, s);
     case Form::FP16: return launch_shape<Form::FP16>(g, a, s);

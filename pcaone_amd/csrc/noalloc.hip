@@ -125,6 +125,7 @@ void packed_gemm_noalloc(Context& x, Form f, const uint8_t* rows, uint64_t nrows
   a.k_end = K;
   a.kchunk = K;
   a.lp = lp;
+  a.ncols = (int)L;
   launch_packed_gemm(f, shape, a, s);
   const int kind = f == Form::FP64 ? 0 : (f == Form::I8 ? 2 : (f == Form::F8 ? 3 : 1));
   hipLaunchKernelGGL(k_gemm_out, dim3(grid_for(nrows * (uint64_t)L)), dim3(256), 0, s, acc, kind, nrows, (int)L, lp,

@@ -221,3 +221,37 @@ def test_batch_small_steps(ctx, k, os):
     for x, y in ((ctx.batch_get_u(0), one.U), (ctx.batch_get_v(0), one.V)):
         np.testing.assert_allclose(np.abs((x * y).sum(0)), 1.0, rtol=1e-9)
     np.testing.assert_allclose(ctx.batch_trace(0), one.trace, atol=1e-11)
+
+
+@pytest.mark.parametrize("L", [17, 20, 21, 28, 29, 33, 36, 40, 41])
+@pytest.mark.parametrize("nrows,ncodes", [(1, 255), (511, 257), (513, 1000)])
+def test_fp32_short_column_blocks(ctx, L, nrows, ncodes):
+    """The FP32 product with its last columns in groups of 4 (L = 17..28, 33..40) and beside that range, exact on
+    values whose products and sums FP32 holds."""
+    say(f"fp32 columns L={L} nrows={nrows} ncodes={ncodes}")
+    rng = np.random.default_rng(nrows + ncodes + L)
+    codes = rng.integers(0, 4, (nrows, ncodes)).astype(np.uint8)
+    W = rng.integers(-64, 64, (ncodes, L)) / 8.0
+    Y = ctx.packed_gemm("fp32", pack(codes), ncodes, W)
+    np.testing.assert_array_equal(Y, np.array([2.0, 0.0, 0.0, -2.0])[codes] @ W)
+
+
+@pytest.mark.parametrize("k", [10, 20])
+def test_fp32_column_groups_same_bits(ctx, k):
+    """The 4-column groups add the same products in the same order as the 16-column blocks: whole runs agree to the
+    bit with workgroup shapes that take the blocks alone (32-row waves), missing genotypes and windows included."""
+    say(f"fp32 column groups k={k}")
+    rng = np.random.default_rng(k)
+    n, m = 700, 3001
+    codes = random_codes(rng, m, n, 0.01)
+    for g in range(3):
+        codes[g::5, g * 200:g * 200 + 150] = 2 * (g % 2)
+    ctx.upload_packed(pack(codes), n)
+    for svd in (1, 2):
+        runs = [ctx.run(svd=svd, k=k, oversamples=10, maxp=3, tol=0.0, bands=4, precision="fp32", want_v=True, wm_g=wm,
+                        wm_h=wm, waves_g=wv, waves_h=wv, kchunk_g=512, kchunk_h=1024)
+                for wm, wv in ((2, 4), (4, 4), (4, 8))]
+        for r in runs[1:]:
+            np.testing.assert_array_equal(r.S, runs[0].S)
+            np.testing.assert_array_equal(r.U, runs[0].U)
+            np.testing.assert_array_equal(r.V, runs[0].V)
