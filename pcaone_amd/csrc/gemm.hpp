@@ -122,6 +122,9 @@ void launch_packed_gemm(Form f, const GemmShape& g, const GemmArgs& a, hipStream
 // (nothing launched) unless the waves own 64 rows and ncols is 17..28 (lp 32)
 // or 33..40 (lp 48).  With one group less to save (41..44) the fragments spill.
 bool launch_packed_gemm_f32_r4(const GemmShape& g, const GemmArgs& a, hipStream_t s);
+// The same for the FP64 form: ncols 17..28, 33..44 or 49..60 (any row tile:
+// 16 rows per wave, and every tile is a multiple of 64 rows).
+bool launch_packed_gemm_f64_r4(const GemmArgs& a, hipStream_t s);
 // `grid` workgroups walk the item list (rows of every item are a whole tile of g).
 void launch_grouped_gemm(Form f, const GemmShape& g, int lp, const GroupedGemmArgs& a, unsigned grid,
                          hipStream_t s);

@@ -870,7 +870,9 @@ void launch_packed_gemm(Form f, const GemmShape& g, const GemmArgs& a, hipStream
   require(f != Form::I8 || a.kchunk <= kI8ChunkCap, kErrArgument, "packed_gemm: I8 chunks are limited to 65536 codes");
   if (a.rows == 0 || a.k_end <= a.k_begin) return;
   switch (f) {
-    case Form::FP64: return launch_shape<Form::FP64>(g, a, s);
+    case Form::FP64:
+      if (launch_packed_gemm_f64_r4(a, s)) return;
+      return launch_shape<Form::FP64>(g, a, s);
     case Form::FP32:
       if (launch_packed_gemm_f32_r4(g, a, s)) return;
       return launch_shape<Form::FP32>(g, a, s);

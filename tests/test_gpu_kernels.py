@@ -223,16 +223,17 @@ def test_batch_small_steps(ctx, k, os):
     np.testing.assert_allclose(ctx.batch_trace(0), one.trace, atol=1e-11)
 
 
-@pytest.mark.parametrize("L", [17, 20, 21, 28, 29, 33, 36, 40, 41])
+@pytest.mark.parametrize("form,L", [(f, L) for f in ("fp32", "fp64") for L in (17, 20, 21, 28, 29, 33, 36, 40, 41)] +
+                         [("fp64", L) for L in (44, 45, 49, 60, 61)])
 @pytest.mark.parametrize("nrows,ncodes", [(1, 255), (511, 257), (513, 1000)])
-def test_fp32_short_column_blocks(ctx, L, nrows, ncodes):
-    """The FP32 product with its last columns in groups of 4 (L = 17..28, 33..40) and beside that range, exact on
-    values whose products and sums FP32 holds."""
-    say(f"fp32 columns L={L} nrows={nrows} ncodes={ncodes}")
+def test_short_column_blocks(ctx, form, L, nrows, ncodes):
+    """The FP32 and FP64 products with their last columns in groups of 4 (L = 17..28, 33..40; FP64 also 41..44 and
+    49..60) and beside those ranges, exact on values whose products and sums FP32 holds."""
+    say(f"{form} columns L={L} nrows={nrows} ncodes={ncodes}")
     rng = np.random.default_rng(nrows + ncodes + L)
     codes = rng.integers(0, 4, (nrows, ncodes)).astype(np.uint8)
     W = rng.integers(-64, 64, (ncodes, L)) / 8.0
-    Y = ctx.packed_gemm("fp32", pack(codes), ncodes, W)
+    Y = ctx.packed_gemm(form, pack(codes), ncodes, W)
     np.testing.assert_array_equal(Y, np.array([2.0, 0.0, 0.0, -2.0])[codes] @ W)
 
 
