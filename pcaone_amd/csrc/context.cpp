@@ -659,7 +659,7 @@ void Context::set_t(const la::Mat& T) {
 
 la::Mat Context::gram_l(const double* X, uint64_t rows, const double* Y, double* dev_out) {
   double* out = dev_out ? dev_out : red_.get() + red_cap_;
-  launch_gram(X, nullptr, Y, rows, lp, red_.get(), red_cap_, out, stream);
+  launch_gram(X, Y, rows, lp, red_.get(), red_cap_, out, stream);
   std::vector<double> h((size_t)lp * lp);
   PCAONE_HIP(hipMemcpyAsync(h.data(), out, h.size() * 8, hipMemcpyDeviceToHost, stream));
   PCAONE_HIP(hipStreamSynchronize(stream));
@@ -1061,12 +1061,17 @@ void Context::zero_h(int which) {
 
 void Context::omega_from(int src, bool flip) {
   require(L > 0, kErrState, "configure() first");
+  const bool deferred = deferred_thinq && deferred_ok();
   if (src == 1) {
-    launch_add(H1_.get(), H2_.get(), H_.get(), H_.size(), stream);
     ++h_version_;
+    if (deferred) {  // H = H1 + H2 on the way into its Gram matrix
+      launch_gram_add(H1_.get(), H2_.get(), H_.get(), N, lp, red_.get(), red_cap_, ldev_.get(), stream);
+      gram_dev_version_ = h_version_;
+    } else {
+      launch_add(H1_.get(), H2_.get(), H_.get(), H_.size(), stream);
+    }
   }
   const double* X = H_.get();
-  const bool deferred = deferred_thinq && deferred_ok();
   if (!deferred && !h_thinq_safe()) {
     // H is (nearly) rank deficient: CholeskyQR2 could break down or lose
     // orthogonality.  The thin Q comes from a Householder QR instead, the
@@ -1082,12 +1087,11 @@ void Context::omega_from(int src, bool flip) {
     double* r1 = g2 + (uint64_t)lp * lp;
     double* dsign = r1 + (uint64_t)lp * lp;
     if (gram_dev_version_ != h_version_) {
-      launch_gram(X, nullptr, nullptr, N, lp, red_.get(), red_cap_, gh, stream);
+      launch_gram(X, nullptr, N, lp, red_.get(), red_cap_, gh, stream);
       gram_dev_version_ = h_version_;
     }
     launch_thinq_first(gh, L, lp, r1, small_.get(), lstatus_.get(), stream, deferred ? kThinqMinPivot : 0.0);
-    launch_apply(X, small_.get(), N, lp, tmp_n_.get(), stream);
-    launch_gram(tmp_n_.get(), nullptr, nullptr, N, lp, red_.get(), red_cap_, g2, stream);
+    launch_gram_apply(X, small_.get(), N, lp, red_.get(), red_cap_, g2, stream);
     launch_thinq_second(g2, r1, X, L, lp, small_.get(), lstatus_.get(), stream);
     if (flip) {  // flipOmg (src/RSVD.hpp:80-89) against Omg2
       launch_apply_flip(X, small_.get(), N, L, lp, omega_c_.get(), omega_.get(), red_.get(), dsign, stream);
@@ -1301,7 +1305,7 @@ void Context::finish_begin() {
   held_ = false;
   // Gram of G~ (first QR of G, src/Halko.cpp:55-60)
   double* gout = red_.get() + red_cap_;
-  launch_gram(gt_.get(), nullptr, nullptr, M, lp, red_.get(), red_cap_, gout, stream);
+  launch_gram(gt_.get(), nullptr, M, lp, red_.get(), red_cap_, gout, stream);
   PCAONE_HIP(hipMemcpyAsync(hp, gout, l2 * 8, hipMemcpyDeviceToHost, stream));
   // Gram of H (B B^T); the device copy serves the next epoch's thin-Q of H
   gram_h_sent_ = gram_version_ != h_version_;
@@ -1309,7 +1313,8 @@ void Context::finish_begin() {
   if (gram_h_sent_) {
     const bool dev = thinq_on_device(lp);
     double* hout = dev ? ldev_.get() : red_.get() + red_cap_ + l2;
-    launch_gram(H_.get(), nullptr, nullptr, N, lp, red_.get(), red_cap_, hout, stream);
+    if (!dev || gram_dev_version_ != h_version_)  // winSVD's last Omega update left it there
+      launch_gram(H_.get(), nullptr, N, lp, red_.get(), red_cap_, hout, stream);
     PCAONE_HIP(hipMemcpyAsync(hp + l2, hout, l2 * 8, hipMemcpyDeviceToHost, stream));
     if (dev) gram_dev_version_ = h_version_;
   }
@@ -1389,7 +1394,7 @@ EpochResult Context::finish_end(int k, bool have_prev) {
   if (have_prev) {
     // mev(Ucur, Upre) = (1/k) sum_i || Ucur^T upre_i ||   (src/Utils.cpp:194-200)
     double* out = red_.get() + red_cap_;
-    launch_gram(ucur_.get(), nullptr, upre_.get(), N, lp, red_.get(), red_cap_, out, stream);
+    launch_gram(ucur_.get(), upre_.get(), N, lp, red_.get(), red_cap_, out, stream);
     std::vector<double> h((size_t)lp * lp);
     PCAONE_HIP(hipMemcpyAsync(h.data(), out, h.size() * 8, hipMemcpyDeviceToHost, stream));
     PCAONE_HIP(hipStreamSynchronize(stream));

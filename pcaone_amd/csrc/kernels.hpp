@@ -82,10 +82,14 @@ void launch_epi_h(Form f, const void* P, uint64_t nchunks, uint64_t chunk_stride
 // Column sums out[l] = sum_{r in [r0,r1)} w_r * X[r][l] (w null = 1), two-stage, deterministic.
 void launch_colsum(const double* X, uint64_t r0, uint64_t r1, int lp, const double* w_sc, const double* w_cf,
                    double* partial, double* out, hipStream_t s);
-// Gram-type reduction: out = (X T)^T (Y) over rows [0, nrows), where Y = Y0 if
-// given else X T; T null = identity.  out is lp x lp row-major.
-void launch_gram(const double* X, const double* T, const double* Y0, uint64_t nrows, int lp, double* partial,
-                 uint64_t partial_cap, double* out, hipStream_t s);
+// Gram matrices over rows [0, nrows), out lp x lp row-major: X^T X, or X^T Y when
+// Y is given; (X + Y)^T (X + Y) with Z = X + Y for those rows; (X T)^T (X T).
+void launch_gram(const double* X, const double* Y, uint64_t nrows, int lp, double* partial, uint64_t partial_cap,
+                 double* out, hipStream_t s);
+void launch_gram_add(const double* X, const double* Y, double* Z, uint64_t nrows, int lp, double* partial,
+                     uint64_t partial_cap, double* out, hipStream_t s);
+void launch_gram_apply(const double* X, const double* T, uint64_t nrows, int lp, double* partial,
+                       uint64_t partial_cap, double* out, hipStream_t s);
 uint64_t gram_partial_elems(uint64_t nrows, int lp);
 // Y = X T (rows x lp) for rows [0, nrows); T lp x lp row-major; rows above nrows untouched.
 void launch_apply(const double* X, const double* T, uint64_t nrows, int lp, double* Y, hipStream_t s);

@@ -525,105 +525,138 @@ inline void sum_partials(double* partial, uint64_t nblocks, uint64_t width, doub
   hipLaunchKernelGGL(k_sum_partials, dim3(gx, 1), dim3(256), 0, s, partial, nblocks, width, (uint64_t)1, nblocks, out);
 }
 
-constexpr int kTileRows = 32;
+// What a Gram kernel multiplies: X^T X, X^T Y, (X + Y)^T (X + Y) with the sum
+// written to Z, or (X T)^T (X T) for an LP x LP T.
+enum GramMode : int { kGramSelf, kGramCross, kGramAdd, kGramApply };
 
-template <int NB>
-constexpr int kSymPerWave = (NB * (NB + 1) / 2 + NB - 1) / NB;
+// Rows staged per step, waves, and the LDS pitch (not a multiple of 32 values:
+// the four rows of one MFMA operand lie in different banks).
+constexpr int gram_tile_rows(int nb, int mode) {
+  return nb <= 2 ? (mode == kGramCross ? 64 : 128) : (nb <= 5 ? (mode == kGramCross ? 32 : 64) : 32);
+}
+constexpr int gram_waves(int nb) { return nb <= 2 ? 4 : 8; }
+constexpr int gram_pitch(int nb) { return 16 * nb + (nb % 2 ? 0 : 16); }
+constexpr size_t gram_lds(int nb, int mode) {
+  return ((size_t)gram_tile_rows(nb, mode) * gram_pitch(nb) * (mode == kGramCross ? 2 : 1) +
+          (mode == kGramApply ? (size_t)256 * nb * nb : 0)) * sizeof(double);
+}
 
 // FP64-MFMA Gram partials: block b sums X[r]^T Y[r] over rows [b*rpb, ...).
-// Cross products: one wave per 16-row block a of the output computes all NB
-// blocks (a, :).  X^T X: the NB (NB + 1) / 2 upper blocks are dealt round
-// robin to the NB waves and each is also stored mirrored (the products are
-// commutative, so the result is exactly symmetric).  Row tiles of X (and Y) are
-// staged in LDS.  v_mfma_f64_16x16x4: A = X^T (lane l: X[k0 + l/16][16i +
+// Cross products: the NB^2 16 x 16 output blocks are dealt round robin to the
+// waves.  X^T X: only the NB (NB + 1) / 2 upper blocks, each also stored
+// mirrored (the products are commutative, so the result is exactly symmetric).
+// Row tiles of X (and Y) are staged in LDS, the next one loaded into
+// registers meanwhile.  v_mfma_f64_16x16x4: A = X^T (lane l: X[k0 + l/16][16i +
 // l%16]), B = Y (lane l: Y[k0 + l/16][16j + l%16]), accumulator lane group q,
 // register r = output row q + 4r.
-template <int NB, bool CROSS>
-__global__ void __launch_bounds__(64 * NB) k_gram_mfma(const double* __restrict__ X, const double* __restrict__ Y,
-                                                       uint64_t nrows, uint64_t rpb, double* __restrict__ partial) {
-  constexpr int LP = NB * 16;
-  __shared__ double xs[kTileRows * LP];
-  __shared__ double ys[CROSS ? kTileRows * LP : 1];
-  const int tid = threadIdx.x, lane = tid & 63, a = tid >> 6;
+// At N of some thousands a block has one or a few tiles and is bound by the
+// latencies in a row: the tiles are as high as LDS and registers allow (one
+// wave per 16 columns with tiles of 32 rows took 11.5 us at 2,000 x 32 and 13.5
+// us at 10,000 x 48, against 5.0 and 6.1 us).  kGramApply forms its tile of X T in
+// LDS and never writes it (8.0 and 11.4 us, against 4.7 + 11.5 and 7.7 + 13.5 us
+// for the product and its Gram); kGramAdd sums H1 + H2 on the way.
+template <int NB, int MODE>
+__global__ void __launch_bounds__(64 * gram_waves(NB)) k_gram(const double* __restrict__ X,
+                                                              const double* __restrict__ Y, uint64_t nrows,
+                                                              uint64_t rpb, double* __restrict__ partial,
+                                                              double* __restrict__ Z) {
+  constexpr int LP = NB * 16, P = gram_pitch(NB), TR = gram_tile_rows(NB, MODE), W = gram_waves(NB), NT = 64 * W;
+  constexpr bool CROSS = MODE == kGramCross, APPLY = MODE == kGramApply;
+  extern __shared__ __align__(16) double gm[];
+  double *xs = gm, *ys = CROSS ? xs + TR * P : xs, *tl = xs + TR * P;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int q = lane >> 4, r16 = lane & 15;
-  f64x4_t acc[NB];
-  for (int b = 0; b < NB; ++b) acc[b] = f64x4_t{0, 0, 0, 0};
-  constexpr int S = kSymPerWave<NB>, NT = NB * (NB + 1) / 2;
-  int ci[S], cj[S];  // this wave's upper blocks in X^T X (unused for cross products)
+  constexpr int NBLK = CROSS ? NB * NB : NB * (NB + 1) / 2, S = (NBLK + W - 1) / W;
+  f64x4_t acc[S];
+  int ci[S], cj[S];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const int t = __builtin_amdgcn_readfirstlane(a + NB * s);
-    ci[s] = t < NT ? 16 * sym_block_i(t, NB) : 0;
-    cj[s] = t < NT ? 16 * sym_block_j(t, NB) : 0;
+    acc[s] = f64x4_t{0, 0, 0, 0};
+    const int t = __builtin_amdgcn_readfirstlane(wave + W * s);
+    ci[s] = t < NBLK ? 16 * (CROSS ? t / NB : sym_block_i(t, NB)) : 0;
+    cj[s] = t < NBLK ? 16 * (CROSS ? t % NB : sym_block_j(t, NB)) : 0;
   }
   const uint64_t rb = (uint64_t)blockIdx.x * rpb;
   const uint64_t re = rb + rpb < nrows ? rb + rpb : nrows;
-  // The next row tile is loaded into registers while the current one is
-  // multiplied; rows past the block's end read as zero.
-  constexpr int PER = kTileRows * LP / (64 * NB);
-  static_assert(PER * 64 * NB == kTileRows * LP, "whole tiles per thread");
-  double px[PER], py[CROSS ? PER : 1];
+  // 16-byte pairs per thread and tile; rows past the block's end read as zero
+  constexpr int PER = (TR * LP / 2 + NT - 1) / NT;
+  constexpr bool EVEN = PER * NT * 2 == TR * LP;
+  double2 px[APPLY ? 1 : PER], py[CROSS || MODE == kGramAdd ? PER : 1];
   auto fetch = [&](uint64_t r0) {
-    const uint64_t nr = re - r0 < (uint64_t)kTileRows ? re - r0 : kTileRows;
+    const int nr = (int)(re - r0 < (uint64_t)TR ? re - r0 : TR);
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
-      const int v = tid + e * 64 * NB;
-      const bool in = (uint64_t)(v / LP) < nr;
-      px[e] = in ? X[r0 * LP + v] : 0.0;
-      if constexpr (CROSS) py[e] = in ? Y[r0 * LP + v] : 0.0;
+      const int v = 2 * (tid + e * NT);
+      const bool in = v / LP < nr;  // nr <= TR: also past a tile that the threads cover unevenly
+      px[e] = in ? *reinterpret_cast<const double2*>(X + r0 * LP + v) : double2{0.0, 0.0};
+      if constexpr (CROSS || MODE == kGramAdd)
+        py[e] = in ? *reinterpret_cast<const double2*>(Y + r0 * LP + v) : double2{0.0, 0.0};
     }
   };
-  fetch(rb);
-  for (uint64_t r0 = rb; r0 < re; r0 += kTileRows) {
+  if constexpr (APPLY) {
+    for (int v = tid; v < LP * LP; v += NT) tl[v] = Y[v];  // Y = T
+  } else {
+    if (rb < re) fetch(rb);
+  }
+  for (uint64_t r0 = rb; r0 < re; r0 += TR) {
     __syncthreads();
+    if constexpr (APPLY) {
+      // xs = X T for this tile: 16-row blocks dealt to the waves, k ascending
+      for (int i = wave; i < TR / 16; i += W) {
+        const uint64_t row = r0 + 16 * i + r16;
+        const bool in = row < re;
+        const double* x = X + row * LP;
+        double av[LP / 4];
 #pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      xs[tid + e * 64 * NB] = px[e];
-      if constexpr (CROSS) ys[tid + e * 64 * NB] = py[e];
-    }
-    __syncthreads();
-    if (r0 + kTileRows < re) fetch(r0 + kTileRows);
-    if constexpr (CROSS) {
+        for (int k = 0; k < LP / 4; ++k) av[k] = in ? x[4 * k + q] : 0.0;
+        f64x4_t y[NB];
 #pragma unroll
-      for (int k0 = 0; k0 < kTileRows; k0 += 4) {
-        const double av = xs[(k0 + q) * LP + 16 * a + r16];
+        for (int b = 0; b < NB; ++b) y[b] = f64x4_t{0, 0, 0, 0};
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          const double bv = ys[(k0 + q) * LP + 16 * b + r16];
-          acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[b], 0, 0, 0);
-        }
+        for (int k = 0; k < LP / 4; ++k)
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+            y[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[k], tl[(4 * k + q) * LP + 16 * b + r16], y[b], 0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) xs[(16 * i + q + 4 * r) * P + 16 * b + r16] = y[b][r];
       }
     } else {
-      // X^T X is symmetric: wave a takes the upper blocks (i <= j) numbered
-      // a, a + NB, a + 2 NB, ... (NB (NB + 1) / 2 blocks over NB waves)
 #pragma unroll
-      for (int k0 = 0; k0 < kTileRows; k0 += 4) {
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-          if (a + NB * s < NT) {
-            const double av = xs[(k0 + q) * LP + ci[s] + r16];
-            const double bv = xs[(k0 + q) * LP + cj[s] + r16];
-            acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[s], 0, 0, 0);
-          }
+      for (int e = 0; e < PER; ++e) {
+        const int v = 2 * (tid + e * NT), at = v / LP * P + v % LP;
+        if (!EVEN && v >= TR * LP) continue;
+        if constexpr (MODE == kGramAdd) {
+          px[e].x += py[e].x, px[e].y += py[e].y;
+          if (r0 + v / LP < re) *reinterpret_cast<double2*>(Z + r0 * LP + v) = px[e];
         }
+        *reinterpret_cast<double2*>(xs + at) = px[e];
+        if constexpr (CROSS) *reinterpret_cast<double2*>(ys + at) = py[e];
+      }
+    }
+    __syncthreads();
+    if constexpr (!APPLY) {
+      if (r0 + TR < re) fetch(r0 + TR);
+    }
+#pragma unroll 8
+    for (int k0 = 0; k0 < TR; k0 += 4) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        if (wave + W * s < NBLK)
+          acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(xs[(k0 + q) * P + ci[s] + r16], ys[(k0 + q) * P + cj[s] + r16],
+                                                        acc[s], 0, 0, 0);
       }
     }
   }
   double* o = partial + (uint64_t)blockIdx.x * LP * LP;
-  if constexpr (CROSS) {
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
+  for (int s = 0; s < S; ++s) {
+    if (wave + W * s < NBLK) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[(16 * a + q + 4 * r) * LP + 16 * b + r16] = acc[b][r];
-  } else {
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      if (a + NB * s < NT) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          o[(ci[s] + q + 4 * r) * LP + cj[s] + r16] = acc[s][r];
-          if (ci[s] != cj[s]) o[(cj[s] + r16) * LP + ci[s] + q + 4 * r] = acc[s][r];  // the mirror block
-        }
+      for (int r = 0; r < 4; ++r) {
+        o[(ci[s] + q + 4 * r) * LP + cj[s] + r16] = acc[s][r];
+        if (!CROSS && ci[s] != cj[s]) o[(cj[s] + r16) * LP + ci[s] + q + 4 * r] = acc[s][r];  // the mirror block
       }
     }
   }
@@ -1510,9 +1543,11 @@ void launch_colsum(const double* X, uint64_t r0, uint64_t r1, int lp, const doub
   check_launch("colsum_sum");
 }
 
+// Rows per Gram partial: about 1,024 of them, a multiple of 32 and at least
+// 128 rows each (the order of the sums is part of the result).
 static uint64_t gram_rpb(uint64_t nrows) {
   uint64_t rpb = (nrows + 1023) / 1024;
-  rpb = (rpb + kTileRows - 1) / kTileRows * kTileRows;
+  rpb = (rpb + 31) / 32 * 32;
   return rpb < 128 ? 128 : rpb;
 }
 
@@ -1522,18 +1557,23 @@ uint64_t gram_partial_elems(uint64_t nrows, int lp) {
   return (nb ? nb : 1) * (uint64_t)lp * lp;
 }
 
-template <int NB>
+template <int NB, int MODE>
 static void gram_nb(const double* X, const double* Y, uint64_t nrows, uint64_t rpb, uint64_t nb, double* partial,
-                    hipStream_t s) {
-  if (Y)
-    hipLaunchKernelGGL((k_gram_mfma<NB, true>), dim3((unsigned)nb), dim3(64 * NB), 0, s, X, Y, nrows, rpb, partial);
-  else
-    hipLaunchKernelGGL((k_gram_mfma<NB, false>), dim3((unsigned)nb), dim3(64 * NB), 0, s, X, X, nrows, rpb, partial);
+                    double* Z, hipStream_t s) {
+  constexpr size_t lds = gram_lds(NB, MODE);
+  static bool attr = false;
+  if (!attr) {
+    PCAONE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gram<NB, MODE>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    attr = true;
+  }
+  hipLaunchKernelGGL((k_gram<NB, MODE>), dim3((unsigned)nb), dim3(64 * gram_waves(NB)), lds, s, X, Y, nrows, rpb,
+                     partial, Z);
 }
 
-void launch_gram(const double* X, const double* T, const double* Y0, uint64_t nrows, int lp, double* partial,
-                 uint64_t partial_cap, double* out, hipStream_t s) {
-  require(T == nullptr, kErrInternal, "gram: apply the transform first");
+template <int MODE>
+static void gram_mode(const double* X, const double* Y, uint64_t nrows, int lp, double* partial, uint64_t partial_cap,
+                      double* Z, double* out, hipStream_t s) {
   require(lp <= 128 && lp % 16 == 0 && lp >= 16, kErrArgument, "gram: bad lp");
   if (nrows == 0) {
     PCAONE_HIP(hipMemsetAsync(out, 0, (size_t)lp * lp * sizeof(double), s));
@@ -1543,19 +1583,39 @@ void launch_gram(const double* X, const double* T, const double* Y0, uint64_t nr
   const uint64_t nb = (nrows + rpb - 1) / rpb;
   require(nb * lp * lp <= partial_cap, kErrInternal, "gram: partial buffer too small");
   switch (lp / 16) {
-    case 1: gram_nb<1>(X, Y0, nrows, rpb, nb, partial, s); break;
-    case 2: gram_nb<2>(X, Y0, nrows, rpb, nb, partial, s); break;
-    case 3: gram_nb<3>(X, Y0, nrows, rpb, nb, partial, s); break;
-    case 4: gram_nb<4>(X, Y0, nrows, rpb, nb, partial, s); break;
-    case 5: gram_nb<5>(X, Y0, nrows, rpb, nb, partial, s); break;
-    case 6: gram_nb<6>(X, Y0, nrows, rpb, nb, partial, s); break;
-    case 7: gram_nb<7>(X, Y0, nrows, rpb, nb, partial, s); break;
-    case 8: gram_nb<8>(X, Y0, nrows, rpb, nb, partial, s); break;
+    case 1: gram_nb<1, MODE>(X, Y, nrows, rpb, nb, partial, Z, s); break;
+    case 2: gram_nb<2, MODE>(X, Y, nrows, rpb, nb, partial, Z, s); break;
+    case 3: gram_nb<3, MODE>(X, Y, nrows, rpb, nb, partial, Z, s); break;
+    case 4: gram_nb<4, MODE>(X, Y, nrows, rpb, nb, partial, Z, s); break;
+    case 5: gram_nb<5, MODE>(X, Y, nrows, rpb, nb, partial, Z, s); break;
+    default:
+      if constexpr (MODE == kGramSelf || MODE == kGramCross) {
+        if (lp == 96) gram_nb<6, MODE>(X, Y, nrows, rpb, nb, partial, Z, s);
+        else if (lp == 112) gram_nb<7, MODE>(X, Y, nrows, rpb, nb, partial, Z, s);
+        else gram_nb<8, MODE>(X, Y, nrows, rpb, nb, partial, Z, s);
+      } else {  // T and the tile share LDS
+        fail(kErrInternal, "gram: the fused forms take at most 80 columns");
+      }
   }
-  check_launch("gram_mfma");
-  const uint64_t w = (uint64_t)lp * lp;
-  sum_partials(partial, nb, w, out, s);
+  check_launch("gram");
+  sum_partials(partial, nb, (uint64_t)lp * lp, out, s);
   check_launch("gram_sum");
+}
+
+void launch_gram(const double* X, const double* Y, uint64_t nrows, int lp, double* partial, uint64_t partial_cap,
+                 double* out, hipStream_t s) {
+  if (Y) gram_mode<kGramCross>(X, Y, nrows, lp, partial, partial_cap, nullptr, out, s);
+  else gram_mode<kGramSelf>(X, nullptr, nrows, lp, partial, partial_cap, nullptr, out, s);
+}
+
+void launch_gram_add(const double* X, const double* Y, double* Z, uint64_t nrows, int lp, double* partial,
+                     uint64_t partial_cap, double* out, hipStream_t s) {
+  gram_mode<kGramAdd>(X, Y, nrows, lp, partial, partial_cap, Z, out, s);
+}
+
+void launch_gram_apply(const double* X, const double* T, uint64_t nrows, int lp, double* partial,
+                       uint64_t partial_cap, double* out, hipStream_t s) {
+  gram_mode<kGramApply>(X, T, nrows, lp, partial, partial_cap, nullptr, out, s);
 }
 
 // Blocks of the product with the flipOmg norms: their partials are summed by
