@@ -1,12 +1,24 @@
-// L x L steps in LDS by one workgroup of NT threads: Cholesky factor, triangular
-// inverse, Householder column signs, 16 x 16 block products.
+// L x L steps in LDS by one workgroup of NT threads: inverse Cholesky factor,
+// Householder column signs, 16 x 16 block products.
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace pcaone {
 namespace {
+
+// f(B), ..., f(E - 1) with constant arguments: registers indexed by nested
+// loops whose bounds depend on each other are not always unrolled, and are then
+// moved through an index register.
+template <int B, int E, class F>
+__device__ __forceinline__ void static_for(const F& f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    static_for<B + 1, E>(f);
+  }
+}
 
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
@@ -26,21 +38,27 @@ __host__ __device__ constexpr int sym_block_j(int t, int nb) {
 template <int NB>
 constexpr int kLP = NB * 16 + 2;
 
-__device__ __forceinline__ double lane_value(double v, int lane) {
+// Lane I of every row of 16 lanes, to the whole row.
+template <int I>
+__device__ __forceinline__ double row_value(double v) {
   const uint64_t u = __builtin_bit_cast(uint64_t, v);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, 0x150 + I, 0xF, 0xF, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), 0x150 + I, 0xF, 0xF, true);
   return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
 
-// Lane S of every group of four lanes, to the whole group.
-template <int S>
-__device__ __forceinline__ double quad_value(double v) {
-  constexpr int ctrl = S * 0x55;
-  const uint64_t u = __builtin_bit_cast(uint64_t, v);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, ctrl, 0xF, 0xF, true);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), ctrl, 0xF, 0xF, true);
-  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+// 1 / sqrt(d) and 1 / x of normal numbers to about one unit in the last place:
+// v_rsq_f64 / v_rcp_f64 (2^-23) and one third-order step.  Half the dependent
+// operations of a correctly rounded root or quotient, and no branch.
+__device__ __forceinline__ double rsqrt_step(double d) {
+  const double y = __builtin_amdgcn_rsq(d);
+  const double e = fma(-(d * y), y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+__device__ __forceinline__ double recip_step(double x) {
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y * e, 1.0 + e, y);
 }
 
 // src (lp x lp in global memory) -> LDS, zero in rows and columns >= n, and
@@ -55,15 +73,18 @@ __device__ __forceinline__ void lds_load(double* M, const double* __restrict__ s
   }
 }
 
-// acc += sign * A[16 bi ..][k] B[k][16 bj ..] for k in [k0, k1), one 16 x 16
-// block per wave (accumulator register r: row q + 4 r, column r16).
-template <int NB>
+// acc += A[16 bi ..][k] B[k][16 bj ..] for k in [k0, k1), one 16 x 16 block per
+// wave (accumulator register r: row q + 4 r, column r16).  TB: B is given as its
+// transpose.
+template <int NB, bool TB = false>
 __device__ __forceinline__ f64x4_t block_product(f64x4_t acc, const double* A, const double* B, int bi, int bj, int k0,
                                                  int k1, int lane) {
   const int q = lane >> 4, r16 = lane & 15;
   for (int k = k0; k < k1; k += 4)
     acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A[(16 * bi + r16) * kLP<NB> + k + q],
-                                               B[(k + q) * kLP<NB> + 16 * bj + r16], acc, 0, 0, 0);
+                                               TB ? B[(16 * bj + r16) * kLP<NB> + k + q]
+                                                  : B[(k + q) * kLP<NB> + 16 * bj + r16],
+                                               acc, 0, 0, 0);
   return acc;
 }
 
@@ -82,75 +103,81 @@ __device__ __forceinline__ void block_store(double* M, const f64x4_t& v, int bi,
 }
 
 // In place: A (n x n, symmetric positive definite, upper blocks used, zero
-// below the diagonal blocks and past n) -> upper R with A = R^T R, zero
-// elsewhere.  Right-looking; DIV: rows divided by the pivot's root, else
-// multiplied by its reciprocal.  Returns false (in every thread) on breakdown;
+// below the diagonal blocks and past n) -> R^-T in the blocks on and below the
+// diagonal (zero above the diagonal within them), where A = R^T R; the blocks
+// above keep R's.  Elimination of [A | 1]: the identity's columns take the rows
+// below the diagonal blocks, which A does not use, and the same row operations,
+// so that the inverse needs no serial steps of its own.  16 pivots at a time
+// run inside a wave: lanes 0..15 hold the diagonal block's columns, the others
+// 48 of the NB 16 columns left and right of it (registers = rows); the rows
+// below follow by MFMA products.  Rows n .. of the last group of four pivots
+// are left as the identity's.  Returns false (in every thread) on breakdown;
 // *min_pivot (thread 0) receives the smallest pivot.
-template <int NB, int NT, bool DIV = false>
-__device__ bool lds_chol_upper(double* A, int n, double* min_pivot, int* flag) {
-  constexpr int P = kLP<NB>;
+template <int NB, int NT>
+__device__ bool lds_chol_inv(double* A, int n, double* min_pivot, int* flag) {
+  constexpr int P = kLP<NB>, LP = NB * 16, NV = (LP + 63) / 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nbn = (n + 15) / 16;
   double dmin = INFINITY;
   if (tid == 0) *flag = 0;
   __syncthreads();
   for (int b = 0; b < nbn; ++b) {
-    const int r0 = 16 * b, m = n - r0 - 16;  // m columns right of the panel's own
-    // lanes 0..15: the diagonal block's columns; the others: 48 columns to the right
-    const bool mine = wave < (m > 48 ? 2 : 1);
-    const int col = lane < 16 ? r0 + lane : r0 + 48 * wave + lane;
-    const bool in = mine && col < NB * 16;
-    double a[16];
+    const int r0 = 16 * b;
+    const int v = 64 * wave + lane;
+    const bool mine = wave < NV, in = v < LP;
+    const bool unit = (v >> 4) == b;  // the identity's columns of this panel
+    double g[16], a[16];
     if (mine) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) a[i] = A[(r0 + i) * P + (in ? col : r0)];
-    }
-    __syncthreads();  // wave 0 writes the diagonal block that both waves read
-    if (mine) {
-      bool ok = true;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        if (ok && r0 + j < n) {
-          const double d = lane_value(a[j], j);
-          if (!(d > 0.0) || !isfinite(d)) {  // the same value in every lane
-            ok = false;
-          } else {
-            dmin = fmin(dmin, d);
-            const double rjj = sqrt(d);
-            double sj;
-            if constexpr (DIV) {
-              sj = a[j] / rjj;
-            } else {
-              const double inv = 1.0 / rjj;
-              sj = a[j] * inv;
-            }
-            a[j] = lane == j ? rjj : sj;
-#pragma unroll
-            for (int i = j + 1; i < 16; ++i) a[i] = fma(-lane_value(sj, i), sj, a[i]);
-          }
-        }
+      for (int i = 0; i < 16; ++i) {
+        g[i] = A[(r0 + i) * P + r0 + (lane & 15)];
+        a[i] = A[(r0 + i) * P + (in ? v : 0)];
+        if (r0 + i >= n) g[i] = (lane & 15) == i ? 1.0 : 0.0;
+        if (unit) a[i] = (lane & 15) == i ? 1.0 : 0.0;
       }
-      if (!ok && tid == 0) *flag = 1;
-      if (in && (lane >= 16 || wave == 0)) {
+    }
+    if constexpr (NV > 1) __syncthreads();  // the diagonal block is read by every wave and written by one
+    if (mine) {
+      bool bad = false;
+      static_for<0, 4>([&](auto q) {
+        if (r0 + 4 * q >= n) return;
+        static_for<4 * q, 4 * q + 4>([&](auto j) {
+          const double d = row_value<j>(g[j]);  // the same value in every lane
+          dmin = r0 + j < n ? fmin(dmin, d) : dmin;
+          bad |= !(d > 0.0 && d < INFINITY);
+          const double inv = rsqrt_step(d);
+          g[j] *= inv;
+          a[j] *= inv;
+          static_for<j + 1, 16>([&](auto i) {
+            g[i] = fma(-row_value<i>(g[j]), g[j], g[i]);
+            a[i] = fma(-row_value<i>(g[j]), a[j], a[i]);
+          });
+        });
+      });
+      if (bad && tid == 0) *flag = 1;
+      if (in) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) A[(r0 + i) * P + col] = (lane >= 16 || i <= lane) && r0 + i < n ? a[i] : 0.0;
+        for (int i = 0; i < 16; ++i) A[(r0 + i) * P + v] = a[i];
       }
     }
     __syncthreads();
     if (*flag) return false;
-    // trailing blocks (bi <= bj): A -= R[panel]^T R[panel]
-    const int t = nbn - b - 1, nt = t * (t + 1) / 2;
-    for (int x = wave; x < nt; x += NT / 64) {
-      int i = 0, y = x;
-      while (y >= t - i) y -= t - i, ++i;
-      const int bi = b + 1 + i, bj = bi + y;
-      f64x4_t acc = block_load<NB>(A, bi, bj, lane);
+    // rows below: A[bi][bj] -= R[b][bi]^T A[b][bj], bj <= b (the inverse) and bj >= bi
+    const int w = b + 1;
+    int x = wave;
+    for (int bi = b + 1; bi < nbn; ++bi) {
+      const int nt = w + nbn - bi;
+      for (; x < nt; x += NT / 64) {
+        const int bj = x < w ? x : bi + x - w;
+        f64x4_t acc = block_load<NB>(A, bi, bj, lane);
 #pragma unroll
-      for (int k = 0; k < 16; k += 4) {
-        const double* row = A + (r0 + k + (lane >> 4)) * P + (lane & 15);
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-row[16 * bi], row[16 * bj], acc, 0, 0, 0);
+        for (int k = 0; k < 16; k += 4) {
+          const double* row = A + (r0 + k + (lane >> 4)) * P + (lane & 15);
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-row[16 * bi], row[16 * bj], acc, 0, 0, 0);
+        }
+        block_store<NB>(A, acc, bi, bj, lane);
       }
-      block_store<NB>(A, acc, bi, bj, lane);
+      x -= nt;
     }
     __syncthreads();
   }
@@ -158,96 +185,60 @@ __device__ bool lds_chol_upper(double* A, int n, double* min_pivot, int* flag) {
   return true;
 }
 
-// X = R^-1 for the upper R in LDS (n x n, zero outside), by rows from the
-// bottom: X[i][c] = (delta_ic - sum_{k > i} R[i][k] X[k][c]) / R[i][i], the sums
-// taken in descending k.  Lane s of four holds the rows 4 m + s of one column
-// c in x[m] (waves 0 .. NB - 1 take 16 columns each; a column's rows below the
-// diagonal stay zero).  rt: scratch of NB 16 x kLP values, which may not
-// overlap R; invd: NB 16 values.  The caller's barrier follows.
-template <int NB, int NT>
-__device__ __forceinline__ void lds_inv_upper(const double* R, double* rt, double* invd, int n, double (&x)[4 * NB]) {
-  constexpr int LP = NB * 16, P = kLP<NB>, L4 = LP / 4;
-  // rt[k][s L4 + m] = R[4 m + s][k]: a lane's factors of one k are contiguous
-  for (int v = threadIdx.x; v < LP * LP; v += NT) {
-    const int i = v / LP, k = v - i * LP;
-    rt[k * P + (i & 3) * L4 + (i >> 2)] = R[i * P + k];
-  }
-  for (int i = threadIdx.x; i < n; i += NT) invd[i] = 1.0 / R[i * P + i];
-#pragma unroll
-  for (int m = 0; m < L4; ++m) x[m] = 0.0;
-  __syncthreads();
-  const int wave = threadIdx.x >> 6, c = threadIdx.x >> 2, s = threadIdx.x & 3;
-  if (wave >= NB) return;
-  const int kmax = 16 * wave + 16 < n ? 16 * wave + 16 : n;
-#pragma unroll
-  for (int kk = L4 - 1; kk >= 0; --kk) {
-    auto row = [&]<int S>() {
-      const int k = 4 * kk + S;
-      if (k >= kmax) return;  // the same in the whole wave
-      double v = ((c == k ? 1.0 : 0.0) - x[kk]) * invd[k];
-      v = c >= k && c < n ? v : 0.0;
-      const double xk = quad_value<S>(v);  // lane S holds row k
-      const double* f = rt + k * P + s * L4;
-#pragma unroll
-      for (int m = 0; m < kk; ++m) x[m] = fma(f[m], xk, x[m]);
-      x[kk] = s == S ? xk : (s < S ? fma(f[kk], xk, x[kk]) : x[kk]);
-    };
-    row.template operator()<3>();
-    row.template operator()<2>();
-    row.template operator()<1>();
-    row.template operator()<0>();
-  }
+// What lds_chol_inv leaves, as R^-1 (upper, zero past n): element (i, c).
+template <int NB>
+__device__ __forceinline__ double inv_upper_at(const double* A, int n, int i, int c) {
+  return i <= c && c < n ? A[c * kLP<NB> + i] : 0.0;
 }
 
 // Householder diagonal signs of the thin QR whose Q has top block W (n x n in
 // LDS, zero past n, destroyed): modified LU, s_i = -sign(u_ii) (Ballard et al.
-// 2014).
+// 2014).  sgn: NB 16 values.
 template <int NB, int NT>
 __device__ void lds_householder_signs(double* W, int n, double* sgn) {
   constexpr int P = kLP<NB>, LP = NB * 16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int nbn = (n + 15) / 16;
   for (int b = 0; b < nbn; ++b) {
-    const int r0 = 16 * b, m = n - r0 - 16;
-    const int nr = m > 48 ? 2 : (m > 0 ? 1 : 0);  // waves for the rows below; the columns right take as many
-    const int nu = nr > 1 ? nr : 1;
-    double a[16];
-    if (wave < nu) {  // lane = column, registers = the panel's rows
-      const int col = lane < 16 ? r0 + lane : r0 + 48 * wave + lane;
-      const bool in = col < LP;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) a[i] = W[(r0 + i) * P + (in ? col : r0)];
+    const int r0 = 16 * b;
+    const bool more = b + 1 < nbn;  // at most 64 columns right and rows below: wave 0 and wave 1
+    if (wave < (more ? 2 : 1)) {
+      const int v = r0 + 16 + lane;
+      const bool in = v < LP, rows = wave == 1;
+      double g[16], a[16];
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        if (r0 + i < n) {
-          const double p = lane_value(a[i], i);
-          const double si = p >= 0.0 ? -1.0 : 1.0, inv = 1.0 / (p - si);
-          if (wave == 0 && lane == i) sgn[r0 + i] = si;
+        g[i] = W[(r0 + i) * P + r0 + (lane & 15)];
+        a[i] = rows ? W[(in ? v : r0) * P + r0 + i] : W[(r0 + i) * P + (in ? v : r0)];
+      }
+      double s = 0.0;
+      const auto panel = [&](auto rows_tag) {
+        static_for<0, 4>([&](auto q) {
+          if (r0 + 4 * q >= n) return;  // rows past n are zero: nothing would change
+          static_for<4 * q, 4 * q + 4>([&](auto i) {
+            const double p = row_value<i>(g[i]);
+            const double si = p >= 0.0 ? -1.0 : 1.0, inv = recip_step(p - si);
+            const double t = g[i] * inv, ta = a[i] * inv;
+            s = (lane & 15) == i ? si : s;
+            static_for<i + 1, 16>([&](auto r) {
+              const double f = -row_value<i>(g[r]);
+              if constexpr (decltype(rows_tag)::value) a[r] = fma(-row_value<r>(g[i]), ta, a[r]);
+              else a[r] = fma(f, ta, a[r]);
+              g[r] = fma(f, t, g[r]);
+            });
+            if constexpr (decltype(rows_tag)::value) a[i] = ta;
+          });
+        });
+      };
+      if (rows) panel(std::true_type{});
+      else panel(std::false_type{});
+      if (!rows && lane < 16) sgn[r0 + lane] = s;
+      if (in && more) {
 #pragma unroll
-          for (int r = i + 1; r < 16; ++r) a[r] = fma(-(lane_value(a[r], i) * inv), a[i], a[r]);
+        for (int i = 0; i < 16; ++i) {
+          if (rows) W[v * P + r0 + i] = a[i];
+          else W[(r0 + i) * P + v] = a[i];
         }
-      }
-      if (in && lane >= 16) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) W[(r0 + i) * P + col] = a[i];
-      }
-    } else if (wave < nu + nr) {  // lane = row, registers = the panel's columns
-      const int row = lane < 16 ? r0 + lane : r0 + 48 * (wave - nu) + lane;
-      const bool in = row < LP;
-#pragma unroll
-      for (int c = 0; c < 16; ++c) a[c] = W[(in ? row : r0) * P + r0 + c];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {  // the rows below exist: the panel is whole
-        const double p = lane_value(a[i], i);
-        const double inv = 1.0 / (p - (p >= 0.0 ? -1.0 : 1.0));
-        const double l = a[i] * inv;
-#pragma unroll
-        for (int c = i + 1; c < 16; ++c) a[c] = fma(-l, lane_value(a[c], i), a[c]);
-        a[i] = l;
-      }
-      if (in && lane >= 16) {
-#pragma unroll
-        for (int c = 0; c < 16; ++c) W[row * P + r0 + c] = a[c];
       }
     }
     __syncthreads();
