@@ -26,6 +26,7 @@ struct BatchSmall {
   int nsv;         // singular values produced (0 when stopped at epoch 0 of --maxp 0)
   double gram_a[kBatchLp * kBatchLp];  // Gram of G~, of Q1, or the cross Gram Ucur^T Upre
   double gram_h[kBatchLp * kBatchLp];  // H^T H
+  double r1h[kBatchLp * kBatchLp];     // R1 of H (CholeskyQR2 of H)
   double t[kBatchLp * kBatchLp];       // transform of the next apply
   double tv[kBatchLp * kBatchLp];      // R^-1 W[:, :k] of the stopping epoch (loadings)
   double sigma[kBatchLp];

@@ -641,7 +641,7 @@ void Context::configure(int prec, int Lr, const GemmTuning& t) {
   h_safe_version_ = ~0ull;
   gram_dev_version_ = ~0ull;
   if (thinq_on_device(lp)) {
-    ldev_.resize(2 * (uint64_t)lp * lp + lp);
+    ldev_.resize(3 * (uint64_t)lp * lp + lp);
     lstatus_.resize(1);
     PCAONE_HIP(hipMemsetAsync(lstatus_.get(), 0, sizeof(int), stream));
   }
@@ -1084,14 +1084,15 @@ void Context::omega_from(int src, bool flip) {
     // every step stream-ordered on the device: no host round trip
     double* gh = ldev_.get();
     double* g2 = gh + (uint64_t)lp * lp;
-    double* dsign = g2 + (uint64_t)lp * lp;
+    double* r1 = g2 + (uint64_t)lp * lp;
+    double* dsign = r1 + (uint64_t)lp * lp;
     if (gram_dev_version_ != h_version_) {
       launch_gram(X, nullptr, N, lp, red_.get(), red_cap_, gh, stream);
       gram_dev_version_ = h_version_;
     }
-    launch_thinq_first(gh, L, lp, small_.get(), lstatus_.get(), stream, deferred ? kThinqMinPivot : 0.0);
+    launch_thinq_first(gh, L, lp, r1, small_.get(), lstatus_.get(), stream, deferred ? kThinqMinPivot : 0.0);
     launch_gram_apply(X, small_.get(), N, lp, red_.get(), red_cap_, g2, stream);
-    launch_thinq_second(g2, X, L, lp, small_.get(), lstatus_.get(), stream);
+    launch_thinq_second(g2, r1, X, L, lp, small_.get(), lstatus_.get(), stream);
     if (flip) {  // flipOmg (src/RSVD.hpp:80-89) against Omg2
       launch_apply_flip(X, small_.get(), N, L, lp, omega_c_.get(), omega_.get(), red_.get(), dsign, stream);
     } else {

@@ -319,7 +319,7 @@ class Context {
   uint64_t h_version_ = 0, gram_version_ = ~0ull;
   la::Mat gram_h_;    // Gram of H (L x L) for h_version_
   // device side of the thin-Q of H (lp <= 80): Gram of H for gram_dev_version_,
-  // second Gram (lp x lp each), column signs (lp); breakdown status
+  // second Gram, R1 (lp x lp each), column signs (lp); breakdown status
   DevBuf<double> res_ut_, res_sv_, res_part_;
   DevBuf<float> res_out_;
   int res_k_ = 0;

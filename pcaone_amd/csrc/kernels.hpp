@@ -103,15 +103,16 @@ void launch_flip_norms(const double* O2, const double* Q, uint64_t nrows, int lp
 // Thin-Q of an N x L matrix X (CholeskyQR2 with Householder column signs) with
 // its L x L steps on the device, for lp <= 80 (thinq_on_device):
 //   first:  R1 = chol(G1 = X^T X), T1 = R1^-1;
-//   second: R2 = chol(G2 = (X T1)^T (X T1)), T1 -> T = T1 R2^-1 diag(s), s the
-//           Householder signs of Xtop T1 R2^-1, Xtop the first n rows of X.
+//   second: R2 = chol(G2 = (X T1)^T (X T1)), T = (R2 R1)^-1 diag(s), s the
+//           Householder signs of Xtop (R2 R1)^-1, Xtop the first n rows of X.
 // A Cholesky breakdown sets *status = 1 (the outputs are then zero).
 bool thinq_on_device(int lp);
 // min_ratio > 0: also set *status = 2 when the smallest Cholesky pivot is at
 // most min_ratio times the largest diagonal entry (H near rank deficient).
-void launch_thinq_first(const double* G1, int n, int lp, double* T1, int* status, hipStream_t s,
+void launch_thinq_first(const double* G1, int n, int lp, double* R1, double* T1, int* status, hipStream_t s,
                         double min_ratio = 0.0);
-void launch_thinq_second(const double* G2, const double* Xtop, int n, int lp, double* T, int* status, hipStream_t s);
+void launch_thinq_second(const double* G2, const double* R1, const double* Xtop, int n, int lp, double* T,
+                         int* status, hipStream_t s);
 // flipOmg's column signs from nb partial blocks of the two norms (2 lp values
 // each; launch_flip_norms leaves one): -1 where a[l] > 2 b[l] (l < n), else 1
 // (lp entries).

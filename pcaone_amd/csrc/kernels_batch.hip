@@ -1,6 +1,7 @@
 // Grouped kernels of the batched randomized SVD: operand pieces, epilogues,
 // reductions and applications over the rows of every cohort, and the
-// per-cohort L x L steps (inverse Cholesky factor, Jacobi eigen-decomposition, Householder signs, stop rule) in one workgroup each.
+// per-cohort L x L steps (Cholesky, triangular inverse, Jacobi
+// eigen-decomposition, Householder signs, stop rule) in one workgroup each.
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
@@ -543,12 +544,12 @@ __global__ void k_b_active(BatchArgs a, int* __restrict__ active) {
 
 // ---------------------------------------------------------------- L x L steps
 // One workgroup per cohort, matrices in LDS with rows of P values, zero outside
-// n x n.  Serial chains of square roots and divisions bound them: the inverse
-// Cholesky factors run in one wave per 16 pivots (small_la.hpp), the products as
-// MFMAs (the same sums in the same order as a loop over k), the Jacobi rotations
-// from two reciprocal roots.  32 cohorts, L = 20: 91 us per launch over all modes
-// as loops over LDS with a thread-0 part in every pivot, sweep and stop test; 34 us
-// with a factor and then an inverse by columns; 27 us now.
+// n x n.  Serial chains of square roots and divisions bound them: the Cholesky
+// factors run in one wave per 16 pivots (small_la.hpp), the inverses one column
+// per lane, the products as MFMAs (the same sums in the same order as a loop
+// over k), the Jacobi rotations from two reciprocal roots.  32 cohorts, L = 20:
+// 91 us per launch over all modes as loops over LDS with a thread-0 part in every
+// pivot, sweep and stop test, against 34 us.
 constexpr int kSmallThreads = 256;
 constexpr int SNB = LP / 16;
 constexpr int P = kLP<SNB>;
@@ -569,9 +570,33 @@ __device__ __forceinline__ void sm_mul(double* C, const double* A, const double*
   __syncthreads();
 }
 
-// Zeroes the block below the diagonal blocks, as lds_chol_inv takes it.
+// Zeroes the block below the diagonal blocks (lds_chol_upper leaves it alone).
 __device__ __forceinline__ void sm_upper(double* A) {
   for (int v = threadIdx.x; v < 256; v += kSmallThreads) A[(16 + v / 16) * P + v % 16] = 0.0;
+  __syncthreads();
+}
+
+// X = R^-1 for the upper R (zero outside n x n): lane j of wave 0 holds column
+// j; X[i][j] = -(sum_{k = i+1}^{j} R[i][k] X[k][j]) / R[i][i], k ascending.
+// Ends synchronized.
+__device__ void sm_inv_upper(double* X, const double* R, int n) {
+  if (threadIdx.x < LP) {
+    const int j = threadIdx.x;
+    double x[LP];
+    static_for<0, LP>([&](auto back) {
+      constexpr int i = LP - 1 - decltype(back)::value;
+      x[i] = 0.0;
+      if (i < n) {
+        const double d = R[i * P + i], inv = 1.0 / d;
+        double t = 0.0;
+        static_for<i + 1, LP>([&](auto k) { t = fma(R[i * P + k], x[k], t); });
+        const double v = quotient(i == j ? 1.0 : -t, d, inv);
+        x[i] = i <= j && j < n ? v : 0.0;
+      }
+    });
+#pragma unroll
+    for (int i = 0; i < LP; ++i) X[i * P + j] = x[i];
+  }
   __syncthreads();
 }
 
@@ -723,13 +748,9 @@ __global__ void __launch_bounds__(kSmallThreads) k_b_small(BatchArgs a, int mode
   const int state = st->state;
   const int L = a.L, k = a.k;
   const auto load = [&](double* M, const double* src, bool upper) { lds_load<SNB, kSmallThreads>(M, src, L, upper); };
-  // M (upper) -> R^-1 in X, for M = R^T R
-  const auto chol_inv = [&](double* X, double* M) {
-    if (!lds_chol_inv<SNB, kSmallThreads>(M, L, &min_pivot, &flag)) return false;
-    for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads)
-      X[v / LP * P + v % LP] = inv_upper_at<SNB>(M, L, v / LP, v % LP);
-    __syncthreads();
-    return true;
+  const auto chol = [&](double* M) { return lds_chol_upper<SNB, kSmallThreads, true>(M, L, &min_pivot, &flag); };
+  const auto store = [&](double* dst, const double* M) {
+    for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) dst[v] = M[v / LP * P + v % LP];
   };
   if (mode == kSmallFinish) {
     if (threadIdx.x == 0 && state == 2) st->state = 0;
@@ -752,18 +773,20 @@ __global__ void __launch_bounds__(kSmallThreads) k_b_small(BatchArgs a, int mode
     load(M0, st->gram_a, false);
     load(M1, st->gram_a, true);
     __syncthreads();
-    if (!chol_inv(M2, M1)) {
+    if (!chol(M1)) {
       if (threadIdx.x == 0) st->state = -5;
       return;
     }
+    sm_inv_upper(M2, M1, L);
     sm_mul<false>(M3, M0, M2);  // Ga R1^-1
     sm_mul<true>(M4, M2, M3);   // R1^-T Ga R1^-1
     sm_upper(M4);
-    if (!chol_inv(M3, M4)) {
+    if (!chol(M4)) {
       if (threadIdx.x == 0) st->state = -5;
       return;
     }
-    sm_mul<false>(M0, M2, M3);  // R^-1 = R1^-1 R2^-1
+    sm_mul<false>(M3, M4, M1);  // R = R2 R1
+    sm_inv_upper(M0, M3, L);    // R^-1
     // C = R^-T (H^T H) R^-1
     load(M1, st->gram_h, false);
     __syncthreads();
@@ -811,21 +834,24 @@ __global__ void __launch_bounds__(kSmallThreads) k_b_small(BatchArgs a, int mode
   } else if (mode == kSmallOmega1) {
     load(M1, st->gram_h, true);
     __syncthreads();
-    if (!chol_inv(M2, M1)) {
+    if (!chol(M1)) {
       if (threadIdx.x == 0) st->state = -5;
       return;
     }
-    for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) st->t[v] = M2[v / LP * P + v % LP];
+    store(st->r1h, M1);
+    sm_inv_upper(M2, M1, L);
+    store(st->t, M2);
   } else if (mode == kSmallOmega2) {
     load(M1, st->gram_a, true);  // Gram of Q1 = H R1^-1
-    load(M2, st->t, true);  // R1^-1
+    load(M2, st->r1h, true);
     load(M4, c.mat[kBufH], false);  // top L x L block of H
     __syncthreads();
-    if (!chol_inv(M3, M1)) {
+    if (!chol(M1)) {
       if (threadIdx.x == 0) st->state = -5;
       return;
     }
-    sm_mul<false>(M0, M2, M3);  // R^-1 = R1^-1 R2^-1
+    sm_mul<false>(M3, M1, M2);  // R2 R1
+    sm_inv_upper(M0, M3, L);    // Rinv
     sm_mul<false>(M2, M4, M0);  // top block of Q = H Rinv
     lds_householder_signs<SNB, kSmallThreads>(M2, L, vec);
     for (int v = threadIdx.x; v < LP * LP; v += kSmallThreads) {

@@ -1138,33 +1138,41 @@ __global__ void __launch_bounds__(256) k_missing_spmm(MissSpmmArgs a) {
 }
 
 // ---- L x L steps of the thin-Q of H on the device (one workgroup each) ----
-// Serial chains: n pivots of an elimination that gives the inverse Cholesky
-// factor at once, n pivots of a modified LU.  What bounds them is one wave's
-// issue and the latency between one pivot and the next (about 300 cycles), so a
-// panel of 16 pivots runs inside one wave with its registers indexed by
-// constants only, roots and quotients take one third-order step, and the 16-row
-// updates between panels and the products are FP64 MFMAs.  T1 R2^-1 in place of
-// (R2 R1)^-1 leaves the first factor out of the second kernel.
-// Factor, then an inverse row by row, correctly rounded roots, registers of the
-// later pivots behind an index register, as before, against this form, first +
-// second kernel: L = 20 13 + 19 -> 7 + 12 us, L = 40 22 + 35 -> 11 + 23 us.
+// Serial chains: n pivots of a Cholesky factorization, n rows of a triangular
+// inverse, n pivots of a modified LU.  What bounds them is one wave's issue and
+// the latency between one pivot and the next, so a panel of 16 pivots runs
+// inside one wave with its registers indexed by constants only (lane = matrix
+// column, registers = the panel's 16 rows, row broadcasts in place of LDS and
+// barriers), a root and its reciprocal come from one approximation, the inverse
+// gives each column of the result to four lanes of one wave and reads the
+// factors of four rows ahead, and the 16-row updates between panels and the
+// products are FP64 MFMAs.  v_mfma_f64_16x16x4 adds its four products to the
+// accumulator one after another in ascending k as fused multiply-adds, so every
+// element of T sees the operations of the unblocked elimination in the same order
+// with the same roundings, and the results are the same bits (a rounding more or
+// less here is a different FP32 Omega, and other signs of U's columns, in one run
+// of six).
+// One element per thread of a 16 x 16 grid and a barrier per pivot, then the
+// panels with the later pivots' registers behind an index register, then this
+// form, first + second kernel: L = 20 17 + 29 -> 13 + 19 -> 10 + 15 us, L = 40
+// 48 + 79 -> 22 + 35 -> 17 + 30 us, L = 80 146 + 259 -> 43 + 77 -> 34 + 66 us.
 constexpr int kThinqThreads = 512;
 constexpr int kThinqMaxNB = 5;  // lp <= 80
 
 template <int NB>
-constexpr size_t thinq_lds(int mats) {
-  return ((size_t)mats * NB * 16 * kLP<NB> + NB * 16 + 2) * sizeof(double);
+constexpr size_t thinq_lds() {
+  return ((size_t)2 * NB * 16 * kLP<NB> + 3 * NB * 16 + 2) * sizeof(double);
 }
 
-// First pass: T1 = R1^-1 for R1 = chol(G1) (lp x lp, zero padded; zero on
+// First pass: R1 = chol(G1), T1 = R1^-1 (lp x lp, zero padded; zero on
 // breakdown).
 template <int NB>
 __global__ void __launch_bounds__(kThinqThreads) k_thinq_first(const double* __restrict__ G1, int n,
-                                                               double* __restrict__ T1, int* __restrict__ status,
-                                                               double min_ratio) {
-  constexpr int LP = NB * 16;
+                                                               double* __restrict__ R1, double* __restrict__ T1,
+                                                               int* __restrict__ status, double min_ratio) {
+  constexpr int LP = NB * 16, P = kLP<NB>;
   extern __shared__ __align__(16) double lm[];
-  double *A = lm, *scal = A + LP * kLP<NB>;
+  double *A = lm, *rt = A + LP * P, *invd = rt + LP * P, *scal = invd + 3 * LP;
   int* flag = reinterpret_cast<int*>(scal + 1);
   const int tid = threadIdx.x;
   lds_load<NB, kThinqThreads>(A, G1, n, true);
@@ -1177,63 +1185,97 @@ __global__ void __launch_bounds__(kThinqThreads) k_thinq_first(const double* __r
   }
   __syncthreads();
   double dmin = 0.0;
-  const bool ok = lds_chol_inv<NB, kThinqThreads>(A, n, &dmin, flag);
+  const bool ok = lds_chol_upper<NB, kThinqThreads>(A, n, &dmin, flag);
+  if (!ok) {
+    if (tid == 0) *status = 1;
+    for (int v = tid; v < LP * LP; v += kThinqThreads) R1[v] = T1[v] = 0.0;
+    return;
+  }
   // the host's safety test of this Gram (smallest pivot / largest diagonal),
   // when the caller defers it to the device: a near rank-deficient H is marked
-  if (tid == 0 && !ok) *status = 1;
-  if (ok && min_ratio > 0.0 && tid == 0 && !(dmin > min_ratio * scal[0])) *status = 2;
-  for (int v = tid; v < LP * LP; v += kThinqThreads) T1[v] = ok ? inv_upper_at<NB>(A, n, v / LP, v % LP) : 0.0;
+  if (min_ratio > 0.0 && tid == 0 && !(dmin > min_ratio * scal[0])) *status = 2;
+  for (int v = tid; v < LP * LP; v += kThinqThreads) R1[v] = A[v / LP * P + v % LP];
+  double x[4 * NB];
+  lds_inv_upper<NB, kThinqThreads>(A, rt, invd, n, x);
+  __syncthreads();  // R has been read: A takes X, so that its rows leave whole
+  if (tid < 4 * LP) {
+#pragma unroll
+    for (int m = 0; m < 4 * NB; ++m) A[(4 * m + (tid & 3)) * P + (tid >> 2)] = x[m];
+  }
+  __syncthreads();
+  for (int v = tid; v < LP * LP; v += kThinqThreads) T1[v] = A[v / LP * P + v % LP];
 }
 
-// Second pass: T1 R2^-1 for R2 = chol(G2), the Householder signs s of
-// Xtop T1 R2^-1 (Xtop = the first n rows of the thinned matrix) and
-// T = T1 R2^-1 diag(s) in place of T1 (lp x lp, zero padded; zero on breakdown).
+// Second pass: R2 = chol(G2), R^-1 = (R2 R1)^-1, the Householder signs s of
+// Xtop R^-1 (Xtop = the first n rows of the thinned matrix) and
+// T = R^-1 diag(s) (lp x lp, zero padded; zero on breakdown).
 template <int NB>
 __global__ void __launch_bounds__(kThinqThreads) k_thinq_second(const double* __restrict__ G2,
+                                                                const double* __restrict__ R1,
                                                                 const double* __restrict__ Xtop, int n,
                                                                 double* __restrict__ T, int* __restrict__ status) {
   constexpr int LP = NB * 16, P = kLP<NB>, NW = kThinqThreads / 64;
   extern __shared__ __align__(16) double lm[];
-  double *A = lm, *B = A + LP * P, *C = B + LP * P, *sgn = C + LP * P;
-  int* flag = reinterpret_cast<int*>(sgn + LP);
+  double *A = lm, *B = A + LP * P, *invd = B + LP * P, *sgn = invd + LP, *scal = invd + 3 * LP;
+  int* flag = reinterpret_cast<int*>(scal + 1);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   lds_load<NB, kThinqThreads>(A, G2, n, true);
-  lds_load<NB, kThinqThreads>(B, T, n, true);
-  lds_load<NB, kThinqThreads>(C, Xtop, n, false);
+  lds_load<NB, kThinqThreads>(B, R1, n, true);
   __syncthreads();
   double dmin;
-  if (!lds_chol_inv<NB, kThinqThreads>(A, n, &dmin, flag)) {  // A: R2^-T
+  if (!lds_chol_upper<NB, kThinqThreads>(A, n, &dmin, flag)) {  // R2
     if (tid == 0) *status = 1;
     for (int v = tid; v < LP * LP; v += kThinqThreads) T[v] = 0.0;
     return;
   }
-  {  // B = T1 R2^-1: the upper blocks
+  {  // A = R2 R1: the upper blocks
     constexpr int NT = NB * (NB + 1) / 2, S = (NT + NW - 1) / NW;
     f64x4_t c[S];
 #pragma unroll
     for (int u = 0; u < S; ++u) {
       const int t = wave + NW * u;
       if (t < NT)
-        c[u] = block_product<NB, true>(f64x4_t{0, 0, 0, 0}, B, A, sym_block_i(t, NB), sym_block_j(t, NB),
-                                       16 * sym_block_i(t, NB), 16 * sym_block_j(t, NB) + 16, lane);
+        c[u] = block_product<NB>(f64x4_t{0, 0, 0, 0}, A, B, sym_block_i(t, NB), sym_block_j(t, NB),
+                                 16 * sym_block_i(t, NB), 16 * sym_block_j(t, NB) + 16, lane);
     }
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < S; ++u) {
       const int t = wave + NW * u;
-      if (t < NT) block_store<NB>(B, c[u], sym_block_i(t, NB), sym_block_j(t, NB), lane);
+      if (t < NT) block_store<NB>(A, c[u], sym_block_i(t, NB), sym_block_j(t, NB), lane);
     }
     __syncthreads();
   }
-  // A = Xtop B (B is upper: k up to the block's last column)
-  for (int t = wave; t < NB * NB; t += NW)
-    block_store<NB>(A, block_product<NB>(f64x4_t{0, 0, 0, 0}, C, B, t / NB, t % NB, 0, 16 * (t % NB) + 16, lane),
-                    t / NB, t % NB, lane);
+  double x[4 * NB];
+  lds_inv_upper<NB, kThinqThreads>(A, B, invd, n, x);
   __syncthreads();
-  lds_householder_signs<NB, kThinqThreads>(A, n, sgn);
+  if (tid < 4 * LP) {  // A = R^-1
+#pragma unroll
+    for (int m = 0; m < 4 * NB; ++m) A[(4 * m + (tid & 3)) * P + (tid >> 2)] = x[m];
+  }
+  lds_load<NB, kThinqThreads>(B, Xtop, n, false);
+  __syncthreads();
+  {  // B = Xtop R^-1 (R^-1 is upper: k up to the block's last column)
+    constexpr int NT = NB * NB, S = (NT + NW - 1) / NW;
+    f64x4_t c[S];
+#pragma unroll
+    for (int u = 0; u < S; ++u) {
+      const int t = wave + NW * u;
+      if (t < NT)
+        c[u] = block_product<NB>(f64x4_t{0, 0, 0, 0}, B, A, t / NB, t % NB, 0, 16 * (t % NB) + 16, lane);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < S; ++u) {
+      const int t = wave + NW * u;
+      if (t < NT) block_store<NB>(B, c[u], t / NB, t % NB, lane);
+    }
+    __syncthreads();
+  }
+  lds_householder_signs<NB, kThinqThreads>(B, n, sgn);
   for (int v = tid; v < LP * LP; v += kThinqThreads) {
     const int c = v % LP;
-    T[v] = c < n ? B[v / LP * P + c] * sgn[c] : 0.0;
+    T[v] = c < n ? A[v / LP * P + c] * sgn[c] : 0.0;
   }
 }
 
@@ -1713,42 +1755,51 @@ void launch_sum_chunks(const double* partial, uint64_t nz, uint64_t nrows, int n
 bool thinq_on_device(int lp) { return lp % 16 == 0 && lp <= 16 * kThinqMaxNB; }
 
 template <int NB>
-void thinq_first_nb(const double* G1, int n, double* T1, int* status, double min_ratio, hipStream_t s) {
-  hipLaunchKernelGGL(k_thinq_first<NB>, dim3(1), dim3(kThinqThreads), thinq_lds<NB>(1), s, G1, n, T1, status,
+void thinq_first_nb(const double* G1, int n, double* R1, double* T1, int* status, double min_ratio, hipStream_t s) {
+  static bool attr = false;
+  if (!attr) {
+    PCAONE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_thinq_first<NB>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)thinq_lds<NB>()));
+    attr = true;
+  }
+  hipLaunchKernelGGL(k_thinq_first<NB>, dim3(1), dim3(kThinqThreads), thinq_lds<NB>(), s, G1, n, R1, T1, status,
                      min_ratio);
 }
 
-void launch_thinq_first(const double* G1, int n, int lp, double* T1, int* status, hipStream_t s, double min_ratio) {
+void launch_thinq_first(const double* G1, int n, int lp, double* R1, double* T1, int* status, hipStream_t s,
+                        double min_ratio) {
   require(thinq_on_device(lp) && n <= lp, kErrInternal, "thinq: lp too large for the device path");
   switch (lp / 16) {
-    case 1: thinq_first_nb<1>(G1, n, T1, status, min_ratio, s); break;
-    case 2: thinq_first_nb<2>(G1, n, T1, status, min_ratio, s); break;
-    case 3: thinq_first_nb<3>(G1, n, T1, status, min_ratio, s); break;
-    case 4: thinq_first_nb<4>(G1, n, T1, status, min_ratio, s); break;
-    default: thinq_first_nb<5>(G1, n, T1, status, min_ratio, s); break;
+    case 1: thinq_first_nb<1>(G1, n, R1, T1, status, min_ratio, s); break;
+    case 2: thinq_first_nb<2>(G1, n, R1, T1, status, min_ratio, s); break;
+    case 3: thinq_first_nb<3>(G1, n, R1, T1, status, min_ratio, s); break;
+    case 4: thinq_first_nb<4>(G1, n, R1, T1, status, min_ratio, s); break;
+    default: thinq_first_nb<5>(G1, n, R1, T1, status, min_ratio, s); break;
   }
   check_launch("thinq_first");
 }
 
 template <int NB>
-void thinq_second_nb(const double* G2, const double* Xtop, int n, double* T, int* status, hipStream_t s) {
+void thinq_second_nb(const double* G2, const double* R1, const double* Xtop, int n, double* T, int* status,
+                     hipStream_t s) {
   static bool attr = false;
   if (!attr) {
     PCAONE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_thinq_second<NB>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)thinq_lds<NB>(3)));
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)thinq_lds<NB>()));
     attr = true;
   }
-  hipLaunchKernelGGL(k_thinq_second<NB>, dim3(1), dim3(kThinqThreads), thinq_lds<NB>(3), s, G2, Xtop, n, T, status);
+  hipLaunchKernelGGL(k_thinq_second<NB>, dim3(1), dim3(kThinqThreads), thinq_lds<NB>(), s, G2, R1, Xtop, n, T, status);
 }
 
-void launch_thinq_second(const double* G2, const double* Xtop, int n, int lp, double* T, int* status, hipStream_t s) {
+void launch_thinq_second(const double* G2, const double* R1, const double* Xtop, int n, int lp, double* T,
+                         int* status, hipStream_t s) {
   require(thinq_on_device(lp) && n <= lp, kErrInternal, "thinq: lp too large for the device path");
   switch (lp / 16) {
-    case 1: thinq_second_nb<1>(G2, Xtop, n, T, status, s); break;
-    case 2: thinq_second_nb<2>(G2, Xtop, n, T, status, s); break;
-    case 3: thinq_second_nb<3>(G2, Xtop, n, T, status, s); break;
-    case 4: thinq_second_nb<4>(G2, Xtop, n, T, status, s); break;
-    default: thinq_second_nb<5>(G2, Xtop, n, T, status, s); break;
+    case 1: thinq_second_nb<1>(G2, R1, Xtop, n, T, status, s); break;
+    case 2: thinq_second_nb<2>(G2, R1, Xtop, n, T, status, s); break;
+    case 3: thinq_second_nb<3>(G2, R1, Xtop, n, T, status, s); break;
+    case 4: thinq_second_nb<4>(G2, R1, Xtop, n, T, status, s); break;
+    default: thinq_second_nb<5>(G2, R1, Xtop, n, T, status, s); break;
   }
   check_launch("thinq_second");
 }

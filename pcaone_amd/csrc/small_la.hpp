@@ -1,5 +1,5 @@
-// L x L steps in LDS by one workgroup of NT threads: inverse Cholesky factor,
-// Householder column signs, 16 x 16 block products.
+// L x L steps in LDS by one workgroup of NT threads: Cholesky factor, triangular
+// inverse, Householder column signs, 16 x 16 block products.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -38,6 +38,9 @@ __host__ __device__ constexpr int sym_block_j(int t, int nb) {
 template <int NB>
 constexpr int kLP = NB * 16 + 2;
 
+// The wave's index in the workgroup, as a scalar: branches on it take no lane masks.
+__device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
+
 // Lane I of every row of 16 lanes, to the whole row.
 template <int I>
 __device__ __forceinline__ double row_value(double v) {
@@ -47,14 +50,33 @@ __device__ __forceinline__ double row_value(double v) {
   return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
 
-// 1 / sqrt(d) and 1 / x of normal numbers to about one unit in the last place:
-// v_rsq_f64 / v_rcp_f64 (2^-23) and one third-order step.  Half the dependent
-// operations of a correctly rounded root or quotient, and no branch.
-__device__ __forceinline__ double rsqrt_step(double d) {
-  const double y = __builtin_amdgcn_rsq(d);
-  const double e = fma(-(d * y), y, 1.0);
-  return fma(y * e, fma(0.375, e, 0.5), y);
+// Lane S of every group of four lanes, to the whole group.
+template <int S>
+__device__ __forceinline__ double quad_value(double v) {
+  constexpr int ctrl = S * 0x55;
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, ctrl, 0xF, 0xF, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), ctrl, 0xF, 0xF, true);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
+
+// sqrt(d) and 1 / sqrt(d), both rounded as the root and the quotient are, without
+// their range checks: v_rsq_f64 (2^-23), one third-order step, and Markstein's
+// corrections of the root and of its reciprocal.
+__device__ __forceinline__ void root_and_inverse(double d, double& r, double& inv) {
+  const double y0 = __builtin_amdgcn_rsq(d);
+  const double e = fma(-(d * y0), y0, 1.0);
+  const double y = fma(y0 * e, fma(0.375, e, 0.5), y0);
+  const double g = d * y;
+  r = fma(fma(-g, g, d), 0.5 * y, g);
+  inv = fma(fma(-r, y, 1.0), y, y);
+}
+// x / d with inv = 1 / d, rounded as the quotient is (Markstein's correction).
+__device__ __forceinline__ double quotient(double x, double d, double inv) {
+  const double q = x * inv;
+  return fma(fma(-q, d, x), inv, q);
+}
+// 1 / x to about one unit in the last place.
 __device__ __forceinline__ double recip_step(double x) {
   const double y = __builtin_amdgcn_rcp(x);
   const double e = fma(-x, y, 1.0);
@@ -74,17 +96,14 @@ __device__ __forceinline__ void lds_load(double* M, const double* __restrict__ s
 }
 
 // acc += A[16 bi ..][k] B[k][16 bj ..] for k in [k0, k1), one 16 x 16 block per
-// wave (accumulator register r: row q + 4 r, column r16).  TB: B is given as its
-// transpose.
-template <int NB, bool TB = false>
+// wave (accumulator register r: row q + 4 r, column r16).
+template <int NB>
 __device__ __forceinline__ f64x4_t block_product(f64x4_t acc, const double* A, const double* B, int bi, int bj, int k0,
                                                  int k1, int lane) {
   const int q = lane >> 4, r16 = lane & 15;
   for (int k = k0; k < k1; k += 4)
     acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A[(16 * bi + r16) * kLP<NB> + k + q],
-                                               TB ? B[(16 * bj + r16) * kLP<NB> + k + q]
-                                                  : B[(k + q) * kLP<NB> + 16 * bj + r16],
-                                               acc, 0, 0, 0);
+                                               B[(k + q) * kLP<NB> + 16 * bj + r16], acc, 0, 0, 0);
   return acc;
 }
 
@@ -103,81 +122,86 @@ __device__ __forceinline__ void block_store(double* M, const f64x4_t& v, int bi,
 }
 
 // In place: A (n x n, symmetric positive definite, upper blocks used, zero
-// below the diagonal blocks and past n) -> R^-T in the blocks on and below the
-// diagonal (zero above the diagonal within them), where A = R^T R; the blocks
-// above keep R's.  Elimination of [A | 1]: the identity's columns take the rows
-// below the diagonal blocks, which A does not use, and the same row operations,
-// so that the inverse needs no serial steps of its own.  16 pivots at a time
-// run inside a wave: lanes 0..15 hold the diagonal block's columns, the others
-// 48 of the NB 16 columns left and right of it (registers = rows); the rows
-// below follow by MFMA products.  Rows n .. of the last group of four pivots
-// are left as the identity's.  Returns false (in every thread) on breakdown;
-// *min_pivot (thread 0) receives the smallest pivot.
-template <int NB, int NT>
-__device__ bool lds_chol_inv(double* A, int n, double* min_pivot, int* flag) {
-  constexpr int P = kLP<NB>, LP = NB * 16, NV = (LP + 63) / 64;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// below the diagonal blocks and past n) -> upper R with A = R^T R, zero
+// elsewhere.  Right-looking; DIV: rows divided by the pivot's root, else
+// multiplied by its reciprocal.  16 pivots at a time run inside wave 0: g holds
+// the diagonal block's columns in every 16 lanes, a the (at most 64) columns to
+// the right, registers = rows, and a row's factor comes as a row broadcast of
+// g; the rows below follow by MFMA products.  Returns false (in every thread) on
+// breakdown; *min_pivot (thread 0) receives the smallest pivot.
+template <int NB, int NT, bool DIV = false>
+__device__ bool lds_chol_upper(double* A, int n, double* min_pivot, int* flag) {
+  constexpr int P = kLP<NB>, LP = NB * 16;
+  static_assert(NB <= 5, "one wave holds the columns right of a panel");
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_index(), l16 = lane & 15;
   const int nbn = (n + 15) / 16;
   double dmin = INFINITY;
   if (tid == 0) *flag = 0;
   __syncthreads();
   for (int b = 0; b < nbn; ++b) {
     const int r0 = 16 * b;
-    const int v = 64 * wave + lane;
-    const bool mine = wave < NV, in = v < LP;
-    const bool unit = (v >> 4) == b;  // the identity's columns of this panel
-    double g[16], a[16];
-    if (mine) {
+    if (wave == 0) {
+      const int v = r0 + 16 + lane;
+      const bool in = v < LP;
+      double g[16], a[16], piv = INFINITY, root = 0.0;  // lane j of 16: pivot j, its root
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        g[i] = A[(r0 + i) * P + r0 + (lane & 15)];
-        a[i] = A[(r0 + i) * P + (in ? v : 0)];
-        if (r0 + i >= n) g[i] = (lane & 15) == i ? 1.0 : 0.0;
-        if (unit) a[i] = (lane & 15) == i ? 1.0 : 0.0;
+        g[i] = A[(r0 + i) * P + r0 + l16];
+        a[i] = A[(r0 + i) * P + (in ? v : r0)];
       }
-    }
-    if constexpr (NV > 1) __syncthreads();  // the diagonal block is read by every wave and written by one
-    if (mine) {
-      bool bad = false;
+      if (r0 + 16 > n) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)  // the rest of a group of four pivots: left as it is
+          if (r0 + i >= n) g[i] = l16 == i ? 1.0 : 0.0;
+      }
       static_for<0, 4>([&](auto q) {
         if (r0 + 4 * q >= n) return;
         static_for<4 * q, 4 * q + 4>([&](auto j) {
           const double d = row_value<j>(g[j]);  // the same value in every lane
-          dmin = r0 + j < n ? fmin(dmin, d) : dmin;
-          bad |= !(d > 0.0 && d < INFINITY);
-          const double inv = rsqrt_step(d);
-          g[j] *= inv;
-          a[j] *= inv;
+          double rjj, inv;
+          root_and_inverse(d, rjj, inv);
+          piv = l16 == j ? d : piv;
+          root = l16 == j ? rjj : root;
+          g[j] = DIV ? quotient(g[j], rjj, inv) : g[j] * inv;
+          a[j] = DIV ? quotient(a[j], rjj, inv) : a[j] * inv;
           static_for<j + 1, 16>([&](auto i) {
-            g[i] = fma(-row_value<i>(g[j]), g[j], g[i]);
-            a[i] = fma(-row_value<i>(g[j]), a[j], a[i]);
+            const double f = -row_value<i>(g[j]);
+            g[i] = fma(f, g[j], g[i]);
+            a[i] = fma(f, a[j], a[i]);
           });
         });
       });
-      if (bad && tid == 0) *flag = 1;
+      const bool past = r0 + l16 >= n;
+      if (__any(!past && !(piv > 0.0 && piv < INFINITY)) && lane == 0) *flag = 1;
+      if (past) piv = INFINITY;
+#pragma unroll
+      for (int d = 1; d < 16; d <<= 1) piv = fmin(piv, __shfl_xor(piv, d));
+      dmin = fmin(dmin, piv);
+      if (lane < 16) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          A[(r0 + i) * P + r0 + lane] = past || i > lane ? 0.0 : (i == lane ? root : g[i]);
+      }
       if (in) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) A[(r0 + i) * P + v] = a[i];
+        for (int i = 0; i < 16; ++i) A[(r0 + i) * P + v] = r0 + i < n ? a[i] : 0.0;
       }
     }
     __syncthreads();
     if (*flag) return false;
-    // rows below: A[bi][bj] -= R[b][bi]^T A[b][bj], bj <= b (the inverse) and bj >= bi
-    const int w = b + 1;
-    int x = wave;
-    for (int bi = b + 1; bi < nbn; ++bi) {
-      const int nt = w + nbn - bi;
-      for (; x < nt; x += NT / 64) {
-        const int bj = x < w ? x : bi + x - w;
-        f64x4_t acc = block_load<NB>(A, bi, bj, lane);
+    // trailing blocks (bi <= bj): A -= R[panel]^T R[panel]
+    const int t = nbn - b - 1, nt = t * (t + 1) / 2;
+    for (int x = wave; x < nt; x += NT / 64) {
+      int i = 0, y = x;
+      while (y >= t - i) y -= t - i, ++i;
+      const int bi = b + 1 + i, bj = bi + y;
+      f64x4_t acc = block_load<NB>(A, bi, bj, lane);
 #pragma unroll
-        for (int k = 0; k < 16; k += 4) {
-          const double* row = A + (r0 + k + (lane >> 4)) * P + (lane & 15);
-          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-row[16 * bi], row[16 * bj], acc, 0, 0, 0);
-        }
-        block_store<NB>(A, acc, bi, bj, lane);
+      for (int k = 0; k < 16; k += 4) {
+        const double* row = A + (r0 + k + (lane >> 4)) * P + (lane & 15);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-row[16 * bi], row[16 * bj], acc, 0, 0, 0);
       }
-      x -= nt;
+      block_store<NB>(A, acc, bi, bj, lane);
     }
     __syncthreads();
   }
@@ -185,10 +209,47 @@ __device__ bool lds_chol_inv(double* A, int n, double* min_pivot, int* flag) {
   return true;
 }
 
-// What lds_chol_inv leaves, as R^-1 (upper, zero past n): element (i, c).
-template <int NB>
-__device__ __forceinline__ double inv_upper_at(const double* A, int n, int i, int c) {
-  return i <= c && c < n ? A[c * kLP<NB> + i] : 0.0;
+// X = R^-1 for the upper R in LDS (n x n, zero outside), by rows from the
+// bottom: X[i][c] = (delta_ic - sum_{k > i} R[i][k] X[k][c]) / R[i][i], the sums
+// taken in descending k.  Lane s of four holds the rows 4 m + s of one column
+// c in x[m] (waves 0 .. NB - 1 take 16 columns each; a column's rows below the
+// diagonal stay zero).  Four rows go without a branch between them, so that their
+// factors are read ahead of the chain.  rt: scratch of NB 16 x kLP values, which
+// may not overlap R; invd: NB 16 values.  The caller's barrier follows.
+template <int NB, int NT>
+__device__ __forceinline__ void lds_inv_upper(const double* R, double* rt, double* invd, int n, double (&x)[4 * NB]) {
+  constexpr int LP = NB * 16, P = kLP<NB>, L4 = LP / 4;
+  // rt[k][s L4 + m] = R[4 m + s][k]: a lane's factors of one k are contiguous
+  for (int v = threadIdx.x; v < LP * LP; v += NT) {
+    const int i = v / LP, k = v - i * LP;
+    rt[k * P + (i & 3) * L4 + (i >> 2)] = R[i * P + k];
+  }
+  for (int i = threadIdx.x; i < LP; i += NT) invd[i] = i < n ? 1.0 / R[i * P + i] : 0.0;
+#pragma unroll
+  for (int m = 0; m < L4; ++m) x[m] = 0.0;
+  __syncthreads();
+  const int wave = wave_index(), c = threadIdx.x >> 2, s = threadIdx.x & 3;
+  if (wave >= NB) return;
+  const int kmax = 16 * wave + 16 < n ? 16 * wave + 16 : n;
+  static_for<0, L4>([&](auto back) {
+    constexpr int kk = L4 - 1 - decltype(back)::value;
+    if (4 * kk >= kmax) return;  // the same in the whole wave; rows past n in the last four give zeros
+    double f[4][kk + 1], id[4];
+    static_for<0, 4>([&](auto S) {
+#pragma unroll
+      for (int m = 0; m <= kk; ++m) f[S][m] = rt[(4 * kk + S) * P + s * L4 + m];
+      id[S] = invd[4 * kk + S];
+    });
+    static_for<0, 4>([&](auto rev) {
+      constexpr int S = 3 - decltype(rev)::value, k = 4 * kk + S;
+      double v = ((c == k ? 1.0 : 0.0) - x[kk]) * id[S];
+      v = c >= k && c < n ? v : 0.0;
+      const double xk = quad_value<S>(v);  // lane S holds row k
+      x[kk] = s == S ? xk : (s < S ? fma(f[S][kk], xk, x[kk]) : x[kk]);
+#pragma unroll
+      for (int m = 0; m < kk; ++m) x[m] = fma(f[S][m], xk, x[m]);
+    });
+  });
 }
 
 // Householder diagonal signs of the thin QR whose Q has top block W (n x n in
@@ -197,7 +258,7 @@ __device__ __forceinline__ double inv_upper_at(const double* A, int n, int i, in
 template <int NB, int NT>
 __device__ void lds_householder_signs(double* W, int n, double* sgn) {
   constexpr int P = kLP<NB>, LP = NB * 16;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = wave_index();
   const int nbn = (n + 15) / 16;
   for (int b = 0; b < nbn; ++b) {
     const int r0 = 16 * b;
@@ -206,10 +267,12 @@ __device__ void lds_householder_signs(double* W, int n, double* sgn) {
       const int v = r0 + 16 + lane;
       const bool in = v < LP, rows = wave == 1;
       double g[16], a[16];
+      const double* from = rows ? W + (in ? v : r0) * P + r0 : W + r0 * P + (in ? v : r0);
+      const int step = rows ? 1 : P;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         g[i] = W[(r0 + i) * P + r0 + (lane & 15)];
-        a[i] = rows ? W[(in ? v : r0) * P + r0 + i] : W[(r0 + i) * P + (in ? v : r0)];
+        a[i] = from[i * step];
       }
       double s = 0.0;
       const auto panel = [&](auto rows_tag) {
@@ -234,11 +297,9 @@ __device__ void lds_householder_signs(double* W, int n, double* sgn) {
       else panel(std::false_type{});
       if (!rows && lane < 16) sgn[r0 + lane] = s;
       if (in && more) {
+        double* to = rows ? W + v * P + r0 : W + r0 * P + v;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          if (rows) W[v * P + r0 + i] = a[i];
-          else W[(r0 + i) * P + v] = a[i];
-        }
+        for (int i = 0; i < 16; ++i) to[i * step] = a[i];
       }
     }
     __syncthreads();
