@@ -777,7 +777,6 @@ void Context::sketch(uint64_t j0, uint64_t j1, int hmode) {
   const uint64_t nwin = j1 - j0;
   const uint64_t jl = j0 - xoff();  // the window's first row in the resident layouts
   const uint64_t wb = bytes_of(form_h);
-  const int P = form_pieces(form_h);
 
   // (1) G[j0:j1] = A Omega : SNP-major rows, K = samples
   const GemmPlan pg = plan_gemm(form_g, shape_g, fixed_g_, lp, nwin, ks_, tuning.kchunk_g, form_kcap(form_g, ks_),
@@ -804,12 +803,11 @@ void Context::sketch(uint64_t j0, uint64_t j1, int hmode) {
   // wh_ (the window's K offset in xt); the K margins around them read as zero.
   const uint64_t off = jl % kKStep;
   const uint64_t klen = round_up(off + nwin, kKStep);
-  launch_zero_ranges(wh_.get(), wh_pitch_ * wb, (uint64_t)P * lp, 0, off * wb, (off + nwin) * wb,
-                     (klen - off - nwin) * wb, stream);
+  const uint32_t right = (uint32_t)(klen - off - nwin);
   if (!lnmiss_ && !form_colscaled(form_g) && !form_colscaled(form_h)) {
     launch_epi_g_fused(form_h, part_.get(), nch_g, g.ychunk, nwin, lp, sc_.get() + j0, cF_.get() + j0,
                        colsum_.get(), gwin, wh_.get() + off * wb, wh_pitch_, (uint64_t)lp * wh_pitch_, red_.get(),
-                       bvec_.get(), stream);
+                       bvec_.get(), (uint32_t)off, right, stream);
   } else {
     launch_epi_g(form_g, part_.get(), nch_g, g.ychunk, nwin, nwin, lp, sc_.get() + j0, cF_.get() + j0,
                  colsum_.get(), gwin, stream, i8_mul(0));
@@ -868,7 +866,7 @@ void Context::sketch(uint64_t j0, uint64_t j1, int hmode) {
       launch_col_scales(form_h, gwin, nwin, lp, sc_.get() + j0, i8max_.get(), i8_scale(1), i8_mul(1), stream);
     launch_make_pieces(form_h, gwin, nwin, nwin, lp, sc_.get() + j0, nullptr, wh_.get() + off * wb, wh_pitch_,
                        (uint64_t)lp * wh_pitch_, gwin, nullptr, stream, i8_scale(1), sc_.get() + j0, cF_.get() + j0,
-                       red_.get(), red_cap_, bvec_.get());
+                       red_.get(), red_cap_, bvec_.get(), (uint32_t)off, right);
   }
 
   h_half(j0, j1, hmode);
@@ -962,12 +960,10 @@ void Context::h_from_g(int hmode) {
   require(L > 0, kErrState, "configure() first");
   require(!form_colscaled(form_h), kErrArgument, "h_from_g: not in the int8 or fp8 form");
   require(!streamed(), kErrArgument, "h_from_g: not with streamed genotypes");
-  const uint64_t wb = bytes_of(form_h);
-  const int P = form_pieces(form_h);
   const uint64_t klen = round_up(M, kKStep);
-  launch_zero_ranges(wh_.get(), wh_pitch_ * wb, (uint64_t)P * lp, 0, 0, M * wb, (klen - M) * wb, stream);
   launch_make_pieces(form_h, gt_.get(), M, M, lp, sc_.get(), nullptr, wh_.get(), wh_pitch_, (uint64_t)lp * wh_pitch_,
-                     gt_.get(), nullptr, stream, nullptr, sc_.get(), cF_.get(), red_.get(), red_cap_, bvec_.get());
+                     gt_.get(), nullptr, stream, nullptr, sc_.get(), cF_.get(), red_.get(), red_cap_, bvec_.get(), 0,
+                     (uint32_t)(klen - M));
   if (lnmiss_) update_missing_weights();
   h_half(0, M, hmode);
 }

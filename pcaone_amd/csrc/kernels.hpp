@@ -50,12 +50,13 @@ void launch_missing_lists(const uint32_t* x, uint64_t pitch, uint64_t nrows, uin
 // The I8 and F8 forms take their column scales from colscale (launch_col_scales).
 // With bvec: bvec[l] = sum_r w_r rounded[r][l], w_r = bsc[r] (1/2 - bcf[r])
 // (1 without bsc), from per-tile partials in bpart (bpart_cap elements; a
-// separate column sum over rounded when they do not fit).
+// separate column sum over rounded when they do not fit).  The `left` elements
+// of every piece row before Wt and the `right` ones after rows_pad are zeroed.
 void launch_make_pieces(Form f, const double* X, uint64_t nreal, uint64_t rows_pad, int lp, const double* rowscale,
                         const double* colsign, void* Wt, uint64_t wpitch, uint64_t wpiece, double* rounded,
                         double* signed_out, hipStream_t s, const double* colscale = nullptr,
                         const double* bsc = nullptr, const double* bcf = nullptr, double* bpart = nullptr,
-                        uint64_t bpart_cap = 0, double* bvec = nullptr);
+                        uint64_t bpart_cap = 0, double* bvec = nullptr, uint32_t left = 0, uint32_t right = 0);
 // Column scales of X for a column-scaled form (rows [0, nreal), each row
 // times rowscale[r], null = 1), from m_l = max_r |X[r][l] rowscale[r]|:
 // I8: scale[l] = m_l / kI8Max, mul[l] = 2 scale[l] (the genotype operand is
@@ -70,12 +71,13 @@ void launch_epi_g(Form f, const void* P, uint64_t nchunks, uint64_t chunk_stride
 // G epilogue fused with the operand split, for data without missing entries
 // (not for I8, whose column scales need the whole window first):
 // gout (nwin x lp) = G~ window, Wt pieces of diag(sc) G~ (window offset
-// already applied), bvec = sum_j sc_j (1/2 - cF_j) G~_j via bpart (scratch of
-// epi_g_fused_partial_elems).
+// already applied; `left` elements before and `right` after the window zeroed),
+// bvec = sum_j sc_j (1/2 - cF_j) G~_j via bpart (scratch of epi_g_fused_partial_elems).
 uint64_t epi_g_fused_partial_elems(uint64_t nwin, int lp);
 void launch_epi_g_fused(Form f, const void* P, uint64_t nchunks, uint64_t stride, uint64_t nwin, int lp,
                         const double* sc, const double* cf, const double* colsum, double* gout, void* Wt,
-                        uint64_t wpitch, uint64_t wpiece, double* bpart, double* bvec, hipStream_t s);
+                        uint64_t wpitch, uint64_t wpiece, double* bpart, double* bvec, uint32_t left, uint32_t right,
+                        hipStream_t s);
 // H epilogue: t = sum_c P[c][i][l] / 4 + b[l]; mode 0: out = t, 1: out += t (i < nreal; rows above = 0 in mode 0).
 void launch_epi_h(Form f, const void* P, uint64_t nchunks, uint64_t chunk_stride, uint64_t nreal, uint64_t rows_pad,
                   int lp, const double* b, double* out, int mode, hipStream_t s, const double* colmul = nullptr);
@@ -117,9 +119,6 @@ void launch_thinq_second(const double* G2, const double* R1, const double* Xtop,
 // each; launch_flip_norms leaves one): -1 where a[l] > 2 b[l] (l < n), else 1
 // (lp entries).
 void launch_flip_signs(const double* partial, int nb, int n, int lp, double* sign, hipStream_t s);
-// Zero bytes [b0, b0 + n0) and [b1, b1 + n1) of each of `rows` rows of `pitch` bytes.
-void launch_zero_ranges(void* base, uint64_t pitch, uint64_t rows, uint64_t b0, uint64_t n0, uint64_t b1, uint64_t n1,
-                        hipStream_t s);
 // flip_UV with V as the base (src/Utils.cpp:118-154) on device-resident
 // V (m x lp) and U (n x lp), row-major: column c < k of both changes sign when
 // V's entry of largest magnitude (the first such) is negative.  partial:

@@ -26,26 +26,27 @@ inline unsigned grid_for(uint64_t n, unsigned block = 256, unsigned cap = 65535u
 
 
 // Operand pieces of one form for each value y = X[r][l] colsign[l] rowscale[r]
-// (F8 and I8 also divided by the column scale), and the value they sum to.
+// (F8 and I8 also divided by the column scale s; is = 1 / s), and the value they
+// sum to.
 template <Form F>
 struct Pieces;
 template <>
 struct Pieces<Form::FP64> {
   using w_t = double;
   static constexpr int P = 1;
-  __device__ static double make(double y, double, w_t* pc) { return pc[0] = y; }
+  __device__ static double make(double y, double, double, w_t* pc) { return pc[0] = y; }
 };
 template <>
 struct Pieces<Form::FP32> {
   using w_t = float;
   static constexpr int P = 1;
-  __device__ static double make(double y, double, w_t* pc) { return (double)(pc[0] = (float)y); }
+  __device__ static double make(double y, double, double, w_t* pc) { return (double)(pc[0] = (float)y); }
 };
 template <>
 struct Pieces<Form::FP16> {
   using w_t = uint16_t;
   static constexpr int P = 1;
-  __device__ static double make(double y, double, w_t* pc) {
+  __device__ static double make(double y, double, double, w_t* pc) {
     pc[0] = fp16_bits(y);
     return fp16_value(pc[0]);
   }
@@ -54,7 +55,7 @@ template <>
 struct Pieces<Form::BF16X1> {
   using w_t = uint16_t;
   static constexpr int P = 1;
-  __device__ static double make(double y, double, w_t* pc) {
+  __device__ static double make(double y, double, double, w_t* pc) {
     pc[0] = bf16_bits((float)y);
     return (double)bf16_value(pc[0]);
   }
@@ -63,7 +64,7 @@ template <>
 struct Pieces<Form::BF16> {
   using w_t = uint16_t;
   static constexpr int P = 2;
-  __device__ static double make(double y, double, w_t* pc) {
+  __device__ static double make(double y, double, double, w_t* pc) {
     pc[0] = bf16_bits((float)y);
     const double back = (double)bf16_value(pc[0]);
     pc[1] = bf16_bits((float)(y - back));
@@ -76,8 +77,8 @@ struct Pieces<Form::F8> {
   static constexpr int P = 3;
   // y / s (exact: s is a power of two, |y / s| <= 448) as three E4M3
   // pieces, each the nearest E4M3 to what the previous ones left
-  __device__ static double make(double y, double s, w_t* pc) {
-    const double x1 = y / s;
+  __device__ static double make(double y, double s, double is, w_t* pc) {
+    const double x1 = y * is;
     double v1, v2, v3;
     pc[0] = e4m3_bits(x1, &v1);
     pc[1] = e4m3_bits(x1 - v1, &v2);
@@ -90,8 +91,8 @@ struct Pieces<Form::I8> {
   using w_t = uint8_t;
   static constexpr int P = 2;
   // q = rint(y / s) within +-kI8Max; q = 256 q_hi + q_lo, q_lo in [-128, 127]
-  __device__ static double make(double y, double s, w_t* pc) {
-    const int q = (int)fmin(fmax(rint(y / s), -(double)kI8Max), (double)kI8Max);
+  __device__ static double make(double y, double s, double is, w_t* pc) {
+    const int q = (int)fmin(fmax(rint(quotient(y, s, is)), -(double)kI8Max), (double)kI8Max);
     const int hi = (q + 128) >> 8, lo = q - 256 * hi;
     pc[0] = (uint8_t)(int8_t)hi;
     pc[1] = (uint8_t)(int8_t)lo;
@@ -103,7 +104,70 @@ struct Pieces<Form::I8> {
 // their transposed pieces (element size wsz bytes): padded so that the
 // column groups of one store land in different banks.
 constexpr int kEpiRows = 64;
-constexpr int epi_pitch(size_t wsz) { return kEpiRows + (wsz == 2 ? 2 : 1); }
+constexpr int kEpiBatch = 4;  // rows a thread loads before it works on them
+constexpr int epi_pitch(size_t wsz) { return kEpiRows + (wsz < 4 ? 4 / (int)wsz : 1); }
+
+// The tile's transposed pieces, LDS -> wt[p][l][r0 + r] for r < nr, in stores of
+// 8 bytes at aligned addresses (one element at a time at the tile's ends, where
+// the window does not start or end on one), and the zeros of the `left` elements
+// before row 0 and the `right` ones from row rows_end, each block a share of the
+// rows.  wpitch and wpiece are multiples of 8 elements.
+template <class w_t>
+__device__ __forceinline__ void store_pieces(const w_t* pt, int np, int lp, w_t* wt, uint64_t wpitch, uint64_t wpiece,
+                                             uint64_t r0, int nr, uint32_t left, uint64_t rows_end, uint32_t right) {
+  constexpr int E = 8 / sizeof(w_t), PITCH = epi_pitch(sizeof(w_t));
+  const auto row_of = [&](int pl) {
+    const int p = (pl >= lp) + (pl >= 2 * lp);
+    return wt + p * wpiece + (pl - p * lp) * wpitch;
+  };
+  if constexpr (E == 1) {
+    for (int v = threadIdx.x; v < np * lp * kEpiRows; v += 256) {
+      const int r = v % kEpiRows, pl = v / kEpiRows;
+      if (r < nr) row_of(pl)[r0 + r] = pt[pl * PITCH + r];
+    }
+  } else {
+    const int sh = (int)(reinterpret_cast<uintptr_t>(wt) / sizeof(w_t) % E);  // r0 is a multiple of E
+    const auto run = [&](auto aligned) {
+      constexpr bool kAligned = decltype(aligned)::value;
+      constexpr int NG = kEpiRows / E + (kAligned ? 0 : 1);
+      for (int v = threadIdx.x; v < np * lp * NG; v += 256) {
+        const int pl = v / NG, r = (v - pl * NG) * E - (kAligned ? 0 : sh);
+        w_t* d = row_of(pl) + r0;
+        const w_t* s = pt + pl * PITCH + r;
+        if (r >= 0 && r + E <= nr) {
+          uint64_t u = 0;
+          if constexpr (kAligned) {
+            const uint32_t* s4 = reinterpret_cast<const uint32_t*>(s);
+            u = (uint64_t)s4[1] << 32 | s4[0];
+          } else {
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+              using bits_t = typename std::conditional<
+                  sizeof(w_t) == 4, uint32_t, typename std::conditional<sizeof(w_t) == 2, uint16_t, uint8_t>::type>::type;
+              u |= (uint64_t)__builtin_bit_cast(bits_t, s[e]) << (8 * sizeof(w_t) * e);
+            }
+          }
+          *reinterpret_cast<uint64_t*>(d + r) = u;
+        } else {
+          for (int e = 0; e < E; ++e)
+            if (r + e >= 0 && r + e < nr) d[r + e] = s[e];
+        }
+      }
+    };
+    if (sh) run(std::false_type{});
+    else run(std::true_type{});
+  }
+  if (left + right) {
+    const uint32_t per = left + right;
+    for (int pl = blockIdx.x; pl < np * lp; pl += gridDim.x) {
+      w_t* d = row_of(pl);
+      for (uint32_t c = threadIdx.x; c < per; c += 256) {
+        if (c < left) (d - left)[c] = w_t(0);
+        else d[rows_end + (c - left)] = w_t(0);
+      }
+    }
+  }
+}
 
 // Operand pieces of X (rows x lp, row-major FP64), transposed to
 // Wt[p][l][r], for a tile of 64 rows per workgroup.  Each thread owns 4
@@ -113,6 +177,10 @@ constexpr int epi_pitch(size_t wsz) { return kEpiRows + (wsz == 2 ? 2 : 1); }
 // pieces' sum / rowscale; in place over X allowed: every element is read and
 // written by the same thread), and the per-tile column sums of
 // w_r rounded[r][l] (w_r = bsc[r] (1/2 - bcf[r]), or 1 without bsc) in bpart.
+// Bound by memory where the rows fill the chip (1,000,000 x 80 as FP8: 469 us,
+// 1.5 GB, against about 580 with a division per value, exponents taken apart by frexp
+// and ldexp and one byte per store) and by a tile's own chain of loads where they
+// do not (10,000 x 40 as BF16: 7.3 us against 10.0 with a row at a time).
 template <Form F>
 __global__ void __launch_bounds__(256) k_make_pieces(const double* X, uint64_t nreal, uint64_t rows_pad, int lp,
                                                      const double* __restrict__ rowscale,
@@ -120,7 +188,7 @@ __global__ void __launch_bounds__(256) k_make_pieces(const double* X, uint64_t n
                                                      uint64_t wpiece, double* rounded, double* __restrict__ signed_out,
                                                      const double* __restrict__ colscale,
                                                      const double* __restrict__ bsc, const double* __restrict__ bcf,
-                                                     double* __restrict__ bpart) {
+                                                     double* __restrict__ bpart, uint32_t left, uint32_t right) {
   using PF = Pieces<F>;
   using w_t = typename PF::w_t;
   constexpr int P = PF::P;
@@ -135,40 +203,58 @@ __global__ void __launch_bounds__(256) k_make_pieces(const double* X, uint64_t n
   const int nr = (int)(rows_pad - r0 < (uint64_t)kEpiRows ? rows_pad - r0 : kEpiRows);
   double b4[4] = {0.0, 0.0, 0.0, 0.0};
   if (act) {
-    double cs[4] = {1.0, 1.0, 1.0, 1.0}, sl[4] = {1.0, 1.0, 1.0, 1.0};
+    double cs[4] = {1.0, 1.0, 1.0, 1.0}, sl[4] = {1.0, 1.0, 1.0, 1.0}, is[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       if (colsign) cs[q] = colsign[4 * cg + q];
       if constexpr (F == Form::F8 || F == Form::I8) sl[q] = colscale[4 * cg + q];
+      is[q] = 1.0 / sl[q];
     }
-    for (int r = rg; r < nr; r += RG) {
-      const uint64_t j = r0 + r;
-      const uint64_t t = j * lp + 4 * cg;
-      double x[4] = {0.0, 0.0, 0.0, 0.0};
-      if (j < nreal) {
-        const double2 a = *reinterpret_cast<const double2*>(X + t);
-        const double2 b = *reinterpret_cast<const double2*>(X + t + 2);
-        x[0] = a.x * cs[0], x[1] = a.y * cs[1], x[2] = b.x * cs[2], x[3] = b.y * cs[3];
-      }
-      if (signed_out) {
-        *reinterpret_cast<double2*>(signed_out + t) = double2{x[0], x[1]};
-        *reinterpret_cast<double2*>(signed_out + t + 2) = double2{x[2], x[3]};
-      }
-      const double rs = rowscale ? rowscale[j] : 1.0;
-      const double w = j < nreal ? (bsc ? bsc[j] * (0.5 - bcf[j]) : 1.0) : 0.0;
-      double rd[4];
+    for (int rb = rg; rb < nr; rb += kEpiBatch * RG) {
+      double x[kEpiBatch][4], rs[kEpiBatch], w[kEpiBatch];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        w_t pc[P];
-        const double back = PF::make(x[q] * rs, sl[q], pc);
-        rd[q] = (j < nreal && rs != 0.0) ? back / rs : 0.0;
-        b4[q] += w * rd[q];
-#pragma unroll
-        for (int p = 0; p < P; ++p) pt[(p * lp + 4 * cg + q) * PITCH + r] = pc[p];
+      for (int u = 0; u < kEpiBatch; ++u) {
+        const uint64_t j = r0 + rb + u * RG;
+        double2 v0{0.0, 0.0}, v1{0.0, 0.0};
+        rs[u] = 1.0, w[u] = 0.0;
+        if (rb + u * RG < nr) {
+          if (j < nreal) {
+            const double* xr = X + j * lp + 4 * cg;
+            v0 = *reinterpret_cast<const double2*>(xr);
+            v1 = *reinterpret_cast<const double2*>(xr + 2);
+            w[u] = bsc ? bsc[j] * (0.5 - bcf[j]) : 1.0;
+          }
+          if (rowscale) rs[u] = rowscale[j];
+        }
+        x[u][0] = v0.x, x[u][1] = v0.y, x[u][2] = v1.x, x[u][3] = v1.y;
       }
-      if (rounded) {
-        *reinterpret_cast<double2*>(rounded + t) = double2{rd[0], rd[1]};
-        *reinterpret_cast<double2*>(rounded + t + 2) = double2{rd[2], rd[3]};
+#pragma unroll
+      for (int u = 0; u < kEpiBatch; ++u) {
+        const int r = rb + u * RG;
+        if (r >= nr) break;
+        const uint64_t j = r0 + r, t = j * lp + 4 * cg;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[u][q] *= cs[q];
+        if (signed_out) {
+          *reinterpret_cast<double2*>(signed_out + t) = double2{x[u][0], x[u][1]};
+          *reinterpret_cast<double2*>(signed_out + t + 2) = double2{x[u][2], x[u][3]};
+        }
+        const bool live = j < nreal && rs[u] != 0.0;
+        const double irs = rowscale ? 1.0 / rs[u] : 1.0;
+        double rd[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          w_t pc[P];
+          const double back = PF::make(x[u][q] * rs[u], sl[q], is[q], pc);
+          rd[q] = live ? (rowscale ? quotient(back, rs[u], irs) : back) : 0.0;
+          b4[q] += w[u] * rd[q];
+#pragma unroll
+          for (int p = 0; p < P; ++p) pt[(p * lp + 4 * cg + q) * PITCH + r] = pc[p];
+        }
+        if (rounded) {
+          *reinterpret_cast<double2*>(rounded + t) = double2{rd[0], rd[1]};
+          *reinterpret_cast<double2*>(rounded + t + 2) = double2{rd[2], rd[3]};
+        }
       }
     }
     if (bpart) {
@@ -177,11 +263,7 @@ __global__ void __launch_bounds__(256) k_make_pieces(const double* X, uint64_t n
     }
   }
   __syncthreads();
-  w_t* wt = static_cast<w_t*>(Wt);
-  for (int v = threadIdx.x; v < P * lp * kEpiRows; v += 256) {
-    const int r = v % kEpiRows, pl = v / kEpiRows, p = pl / lp, l = pl - p * lp;
-    if (r < nr) wt[p * wpiece + l * wpitch + r0 + r] = pt[pl * PITCH + r];
-  }
+  store_pieces(pt, P, lp, static_cast<w_t*>(Wt), wpitch, wpiece, r0, nr, left, rows_pad, right);
   if (bpart) {
     for (int l = threadIdx.x; l < lp; l += 256) {
       double sum = 0.0;
@@ -255,16 +337,21 @@ __global__ void k_epi_g_v4(const PT* __restrict__ part, uint64_t nchunks, uint64
 // column sums of beta_j G~_j with beta_j = sc_j (1/2 - cF_j).  Each thread
 // owns 4 adjacent columns (16-byte partial loads) of every RG-th row; its
 // beta sums stay in registers and are combined across row groups in LDS.
-
+// Bound by reading the partials (all split-K chunks) on long windows and by a
+// tile's chain of loads on short ones, so 16 16-byte loads are in flight: 64
+// windows of 500,000 SNPs, L = 40, 10 chunks each: 24 us on average against 36
+// with a row and a chunk at a time.  The margins cost a kernel of their own (4 to
+// 5 us) before.
 template <Form F, class PT>
 __global__ void __launch_bounds__(256) k_epi_g_fused(const PT* __restrict__ part, uint64_t nchunks, uint64_t stride,
                                                      uint64_t nwin, int lp, const double* __restrict__ sc,
                                                      const double* __restrict__ cf, const double* __restrict__ colsum,
                                                      double* __restrict__ gout, void* Wt, uint64_t wpitch,
-                                                     uint64_t wpiece, double* __restrict__ bpart) {
-  using w_t = typename std::conditional<F == Form::FP64, double,
-                                        typename std::conditional<F == Form::FP32, float, uint16_t>::type>::type;
-  constexpr int P = F == Form::BF16 ? 2 : 1;
+                                                     uint64_t wpiece, double* __restrict__ bpart, uint32_t left,
+                                                     uint32_t right) {
+  using PF = Pieces<F>;
+  using w_t = typename PF::w_t;
+  constexpr int P = PF::P;
   extern __shared__ __align__(16) unsigned char sm[];
   constexpr int PITCH = epi_pitch(sizeof(w_t));
   w_t* pt = reinterpret_cast<w_t*>(sm);  // P x lp rows of PITCH (kEpiRows used)
@@ -276,65 +363,74 @@ __global__ void __launch_bounds__(256) k_epi_g_fused(const PT* __restrict__ part
   const int nr = (int)(nwin - r0 < (uint64_t)kEpiRows ? nwin - r0 : kEpiRows);
   double b4[4] = {0.0, 0.0, 0.0, 0.0};
   if (act) {
-    for (int r = rg; r < nr; r += RG) {
-      const uint64_t j = r0 + r;
-      const uint64_t t = j * lp + 4 * cg;
-      double y[4] = {0.0, 0.0, 0.0, 0.0};
-      for (uint64_t c = 0; c < nchunks; ++c) {
-        const PT* pc4 = part + c * stride + t;
-        if constexpr (sizeof(PT) == 4) {
-          const float4 v = *reinterpret_cast<const float4*>(pc4);
-          y[0] += (double)v.x, y[1] += (double)v.y, y[2] += (double)v.z, y[3] += (double)v.w;
-        } else {
-          const double2 v0 = *reinterpret_cast<const double2*>(pc4);
-          const double2 v1 = *reinterpret_cast<const double2*>(pc4 + 2);
-          y[0] += v0.x, y[1] += v0.y, y[2] += v1.x, y[3] += v1.y;
-        }
-      }
-      const double s = sc[j];
-      const double beta = s * (0.5 - cf[j]);
-      double gr4[4];
+    constexpr int B = 16 / sizeof(PT), NC = B;  // rows and chunks in flight
+    double cs[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int l = 4 * cg + q;
-        const double g = 0.25 * s * y[q] + beta * colsum[l];
-        const double yv = g * s;
-        w_t pc[P];
-        double back;
-        if constexpr (F == Form::FP64) {
-          pc[0] = yv;
-          back = yv;
-        } else if constexpr (F == Form::FP32) {
-          pc[0] = (float)yv;
-          back = (double)pc[0];
-        } else if constexpr (F == Form::FP16) {
-          pc[0] = fp16_bits(yv);
-          back = fp16_value(pc[0]);
-        } else {
-          pc[0] = bf16_bits((float)yv);
-          back = (double)bf16_value(pc[0]);
-          if constexpr (P == 2) {
-            pc[1] = bf16_bits((float)(yv - back));
-            back += (double)bf16_value(pc[1]);
+    for (int q = 0; q < 4; ++q) cs[q] = colsum[4 * cg + q];
+    for (int rb = rg; rb < nr; rb += B * RG) {
+      double y[B][4], sj[B], cj[B];
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const bool in = rb + u * RG < nr;
+        sj[u] = in ? sc[r0 + rb + u * RG] : 0.0;
+        cj[u] = in ? cf[r0 + rb + u * RG] : 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) y[u][q] = 0.0;
+      }
+      // the partials' chunks in order, NC of them in flight at a time
+      const auto take = [&](auto nc_tag, uint64_t c) {
+        constexpr int C = decltype(nc_tag)::value;
+        PT v[C][B][4];
+#pragma unroll
+        for (int i = 0; i < C; ++i)
+#pragma unroll
+          for (int u = 0; u < B; ++u) {
+            const bool in = rb + u * RG < nr;
+            const PT* p = part + (c + i) * stride + (in ? r0 + rb + u * RG : r0) * lp + 4 * cg;
+            if constexpr (sizeof(PT) == 4) {
+              *reinterpret_cast<float4*>(v[i][u]) = *reinterpret_cast<const float4*>(p);
+            } else {
+              *reinterpret_cast<double2*>(v[i][u]) = *reinterpret_cast<const double2*>(p);
+              *reinterpret_cast<double2*>(v[i][u] + 2) = *reinterpret_cast<const double2*>(p + 2);
+            }
           }
-        }
-        gr4[q] = s != 0.0 ? back / s : 0.0;
-        b4[q] += beta * gr4[q];
 #pragma unroll
-        for (int p = 0; p < P; ++p) pt[(p * lp + l) * PITCH + r] = pc[p];
+        for (int i = 0; i < C; ++i)
+#pragma unroll
+          for (int u = 0; u < B; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) y[u][q] += (double)v[i][u][q];
+      };
+      uint64_t c = 0;
+      for (; c + NC <= nchunks; c += NC) take(std::integral_constant<int, NC>{}, c);
+      for (; c < nchunks; ++c) take(std::integral_constant<int, 1>{}, c);
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const int r = rb + u * RG;
+        if (r >= nr) break;
+        const uint64_t t = (r0 + r) * lp + 4 * cg;
+        const double s = sj[u], is = 1.0 / s;
+        const double beta = s * (0.5 - cj[u]);
+        double gr4[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const double g = fma(0.25 * s, y[u][q], beta * cs[q]);
+          w_t pc[P];
+          const double back = PF::make(g * s, 1.0, 1.0, pc);
+          gr4[q] = s != 0.0 ? quotient(back, s, is) : 0.0;
+          b4[q] += beta * gr4[q];
+#pragma unroll
+          for (int p = 0; p < P; ++p) pt[(p * lp + 4 * cg + q) * PITCH + r] = pc[p];
+        }
+        *reinterpret_cast<double2*>(gout + t) = double2{gr4[0], gr4[1]};
+        *reinterpret_cast<double2*>(gout + t + 2) = double2{gr4[2], gr4[3]};
       }
-      *reinterpret_cast<double2*>(gout + t) = double2{gr4[0], gr4[1]};
-      *reinterpret_cast<double2*>(gout + t + 2) = double2{gr4[2], gr4[3]};
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) bred[rg * lp + 4 * cg + q] = b4[q];
   }
   __syncthreads();
-  w_t* w = static_cast<w_t*>(Wt);
-  for (int v = threadIdx.x; v < P * lp * kEpiRows; v += 256) {
-    const int r = v % kEpiRows, pl = v / kEpiRows, p = pl / lp, l = pl - p * lp;
-    if (r < nr) w[p * wpiece + l * wpitch + r0 + r] = pt[pl * PITCH + r];
-  }
+  store_pieces(pt, P, lp, static_cast<w_t*>(Wt), wpitch, wpiece, r0, nr, left, nwin, right);
   for (int l = threadIdx.x; l < lp; l += 256) {
     double sum = 0.0;
     for (int q = 0; q < RG; ++q) sum += bred[q * lp + l];
@@ -786,16 +882,6 @@ __global__ void __launch_bounds__(256) k_rows_to_colmajor(const double* __restri
   for (int v = threadIdx.x; v < 32 * k; v += 256) {
     const int j = v >> 5, r = v & 31;
     if (r < nr) dst[(uint64_t)j * n + (place ? place[r0 + r] : r0 + r)] = tile[r * (lp + 1) + j];
-  }
-}
-
-// Zero bytes [b0, b0 + n0) and [b1, b1 + n1) of each of `rows` rows (pitch bytes).
-__global__ void k_zero_ranges(unsigned char* __restrict__ base, uint64_t pitch, uint64_t rows, uint64_t b0,
-                              uint64_t n0, uint64_t b1, uint64_t n1) {
-  const uint64_t per = n0 + n1;
-  GRID_STRIDE(t, rows * per) {
-    const uint64_t r = t / per, c = t - r * per;
-    base[r * pitch + (c < n0 ? b0 + c : b1 + (c - n0))] = 0;
   }
 }
 
@@ -1323,14 +1409,6 @@ void launch_colmajor_to_rows(const double* src, uint64_t n, int L, int lp, uint6
   check_launch("colmajor_to_rows");
 }
 
-void launch_zero_ranges(void* base, uint64_t pitch, uint64_t rows, uint64_t b0, uint64_t n0, uint64_t b1, uint64_t n1,
-                        hipStream_t s) {
-  if (!rows || n0 + n1 == 0) return;
-  hipLaunchKernelGGL(k_zero_ranges, dim3(grid_for(rows * (n0 + n1))), dim3(256), 0, s,
-                     static_cast<unsigned char*>(base), pitch, rows, b0, n0, b1, n1);
-  check_launch("zero_ranges");
-}
-
 void launch_flip_cols_by_max(double* V, uint64_t m, double* U, uint64_t n, int lp, int k, double* partial,
                              double* sign, hipStream_t s) {
   require(k >= 1 && k <= lp && lp <= 128, kErrArgument, "flip_cols_by_max: bad column count");
@@ -1381,7 +1459,7 @@ template <Form F>
 static void make_pieces_t(const double* X, uint64_t nreal, uint64_t rows_pad, int lp, const double* rowscale,
                           const double* colsign, void* Wt, uint64_t wpitch, uint64_t wpiece, double* rounded,
                           double* signed_out, const double* colscale, const double* bsc, const double* bcf,
-                          double* bpart, hipStream_t s) {
+                          double* bpart, uint32_t left, uint32_t right, hipStream_t s) {
   using w_t = typename Pieces<F>::w_t;
   constexpr int P = Pieces<F>::P;
   const auto lds_for = [](int l) {
@@ -1395,14 +1473,16 @@ static void make_pieces_t(const double* X, uint64_t nreal, uint64_t rows_pad, in
   }
   const uint64_t nb = (rows_pad + kEpiRows - 1) / kEpiRows;
   hipLaunchKernelGGL(k_make_pieces<F>, dim3((unsigned)nb), dim3(256), lds_for(lp), s, X, nreal, rows_pad, lp, rowscale,
-                     colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bpart);
+                     colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bpart, left, right);
 }
 
 void launch_make_pieces(Form f, const double* X, uint64_t nreal, uint64_t rows_pad, int lp, const double* rowscale,
                         const double* colsign, void* Wt, uint64_t wpitch, uint64_t wpiece, double* rounded,
                         double* signed_out, hipStream_t s, const double* colscale, const double* bsc,
-                        const double* bcf, double* bpart, uint64_t bpart_cap, double* bvec) {
+                        const double* bcf, double* bpart, uint64_t bpart_cap, double* bvec, uint32_t left,
+                        uint32_t right) {
   require(!form_colscaled(f) || colscale, kErrInternal, "make_pieces: this form needs column scales");
+  require(wpitch % 8 == 0 && wpiece % 8 == 0, kErrInternal, "make_pieces: bad pitch");
   require(lp >= 16 && lp <= 128 && lp % 4 == 0, kErrArgument, "make_pieces: bad lp");
   if (!rows_pad) return;
   const uint64_t nb = (rows_pad + kEpiRows - 1) / kEpiRows;
@@ -1410,13 +1490,13 @@ void launch_make_pieces(Form f, const double* X, uint64_t nreal, uint64_t rows_p
   const bool fuse = bvec && bpart && nb * (uint64_t)lp <= bpart_cap;
   double* bp = fuse ? bpart : nullptr;
   switch (f) {
-    case Form::FP64: make_pieces_t<Form::FP64>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, s); break;
-    case Form::FP32: make_pieces_t<Form::FP32>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, s); break;
-    case Form::BF16: make_pieces_t<Form::BF16>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, s); break;
-    case Form::BF16X1: make_pieces_t<Form::BF16X1>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, s); break;
-    case Form::FP16: make_pieces_t<Form::FP16>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, s); break;
-    case Form::I8: make_pieces_t<Form::I8>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, s); break;
-    case Form::F8: make_pieces_t<Form::F8>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, s); break;
+    case Form::FP64: make_pieces_t<Form::FP64>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, left, right, s); break;
+    case Form::FP32: make_pieces_t<Form::FP32>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, left, right, s); break;
+    case Form::BF16: make_pieces_t<Form::BF16>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, left, right, s); break;
+    case Form::BF16X1: make_pieces_t<Form::BF16X1>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, left, right, s); break;
+    case Form::FP16: make_pieces_t<Form::FP16>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, left, right, s); break;
+    case Form::I8: make_pieces_t<Form::I8>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, left, right, s); break;
+    case Form::F8: make_pieces_t<Form::F8>(X, nreal, rows_pad, lp, rowscale, colsign, Wt, wpitch, wpiece, rounded, signed_out, colscale, bsc, bcf, bp, left, right, s); break;
   }
   check_launch("make_pieces");
   if (!bvec) return;
@@ -1471,9 +1551,9 @@ uint64_t epi_g_fused_partial_elems(uint64_t nwin, int lp) { return (nwin + kEpiR
 template <Form F, class PT>
 static void epi_fused_t(const void* P, uint64_t nchunks, uint64_t stride, uint64_t nwin, int lp, const double* sc,
                         const double* cf, const double* colsum, double* gout, void* Wt, uint64_t wpitch,
-                        uint64_t wpiece, double* bpart, hipStream_t s) {
-  constexpr int NP = F == Form::BF16 ? 2 : 1;
-  constexpr size_t wsz = F == Form::FP64 ? 8 : (F == Form::FP32 ? 4 : 2);
+                        uint64_t wpiece, double* bpart, uint32_t left, uint32_t right, hipStream_t s) {
+  constexpr int NP = Pieces<F>::P;
+  constexpr size_t wsz = sizeof(typename Pieces<F>::w_t);
   // pieces (transposed) + the row groups' beta sums (256 / (lp / 4) groups x lp)
   const auto lds_for = [](int l) { return ((size_t)epi_pitch(wsz) * l * NP * wsz + 15) / 16 * 16 + (size_t)1024 * 8; };
   const size_t lds = lds_for(lp);
@@ -1486,20 +1566,22 @@ static void epi_fused_t(const void* P, uint64_t nchunks, uint64_t stride, uint64
   }
   const uint64_t nb = (nwin + kEpiRows - 1) / kEpiRows;
   hipLaunchKernelGGL((k_epi_g_fused<F, PT>), dim3((unsigned)nb), dim3(256), lds, s, static_cast<const PT*>(P), nchunks,
-                     stride, nwin, lp, sc, cf, colsum, gout, Wt, wpitch, wpiece, bpart);
+                     stride, nwin, lp, sc, cf, colsum, gout, Wt, wpitch, wpiece, bpart, left, right);
 }
 
 void launch_epi_g_fused(Form f, const void* P, uint64_t nchunks, uint64_t stride, uint64_t nwin, int lp,
                         const double* sc, const double* cf, const double* colsum, double* gout, void* Wt,
-                        uint64_t wpitch, uint64_t wpiece, double* bpart, double* bvec, hipStream_t s) {
+                        uint64_t wpitch, uint64_t wpiece, double* bpart, double* bvec, uint32_t left, uint32_t right,
+                        hipStream_t s) {
   if (!nwin) return;
   require(lp >= 16 && lp <= 128, kErrArgument, "epi_g_fused: bad lp");
+  require(wpitch % 8 == 0 && wpiece % 8 == 0, kErrInternal, "epi_g_fused: bad pitch");
   switch (f) {
-    case Form::FP64: epi_fused_t<Form::FP64, double>(P, nchunks, stride, nwin, lp, sc, cf, colsum, gout, Wt, wpitch, wpiece, bpart, s); break;
-    case Form::FP32: epi_fused_t<Form::FP32, float>(P, nchunks, stride, nwin, lp, sc, cf, colsum, gout, Wt, wpitch, wpiece, bpart, s); break;
-    case Form::BF16: epi_fused_t<Form::BF16, float>(P, nchunks, stride, nwin, lp, sc, cf, colsum, gout, Wt, wpitch, wpiece, bpart, s); break;
-    case Form::BF16X1: epi_fused_t<Form::BF16X1, float>(P, nchunks, stride, nwin, lp, sc, cf, colsum, gout, Wt, wpitch, wpiece, bpart, s); break;
-    case Form::FP16: epi_fused_t<Form::FP16, float>(P, nchunks, stride, nwin, lp, sc, cf, colsum, gout, Wt, wpitch, wpiece, bpart, s); break;
+    case Form::FP64: epi_fused_t<Form::FP64, double>(P, nchunks, stride, nwin, lp, sc, cf, colsum, gout, Wt, wpitch, wpiece, bpart, left, right, s); break;
+    case Form::FP32: epi_fused_t<Form::FP32, float>(P, nchunks, stride, nwin, lp, sc, cf, colsum, gout, Wt, wpitch, wpiece, bpart, left, right, s); break;
+    case Form::BF16: epi_fused_t<Form::BF16, float>(P, nchunks, stride, nwin, lp, sc, cf, colsum, gout, Wt, wpitch, wpiece, bpart, left, right, s); break;
+    case Form::BF16X1: epi_fused_t<Form::BF16X1, float>(P, nchunks, stride, nwin, lp, sc, cf, colsum, gout, Wt, wpitch, wpiece, bpart, left, right, s); break;
+    case Form::FP16: epi_fused_t<Form::FP16, float>(P, nchunks, stride, nwin, lp, sc, cf, colsum, gout, Wt, wpitch, wpiece, bpart, left, right, s); break;
     case Form::I8:
     case Form::F8: fail(kErrInternal, "epi_g_fused: the column-scaled forms take the unfused epilogue");
   }

@@ -80,6 +80,31 @@ def test_missing_lists(ctx, n, m, miss):
     assert (np.abs(ctx.get_h(0, L) - H) / h_bound).max() <= 1.0
 
 
+@pytest.mark.parametrize("form", ["fp32", "bf16", "fp16", "fp8", "int8"])
+@pytest.mark.parametrize("miss", [0.0, 0.1])
+def test_cut_windows_match_whole_ones(ctx, form, miss):
+    """H of a window that starts and ends between the pieces' aligned stores (every offset of 8 bytes, one and two
+    64-row tiles, one row) after a longer window has filled the same buffer: the same operand pieces, hence the same
+    G, and zeros around them, hence H as from that window's matrix alone."""
+    say(f"cut windows {form} miss={miss}")
+    rng = np.random.default_rng(7)
+    n, m, L = 130, 700, 20
+    codes = random_codes(rng, m, n, miss)
+    ctx.upload_packed(pack(codes), n)
+    ctx.standardize()
+    ctx.configure(form, L)
+    ctx.set_omega(rng.standard_normal((n, L)))
+    A, sc = standardized(codes)
+    for j0, j1 in ((1, 64), (2, 130), (3, 68), (4, 5), (261, 389), (262, 330), (263, 520), (519, 700), (5, 690)):
+        ctx.sketch(0, m, 0)
+        ctx.sketch(j0, j1, 0)
+        G, H = ctx.get_g(j0, j1, L), ctx.get_h(0, L)
+        # H = A^T G in 32-bit sums over j1 - j0 rows: each step rounds sums of at most sc (1/2 + 1/2) |G|, and one
+        # product more for the centering; FP8 and INT8 give G as the sum of its pieces, so that H's operand is G
+        bound = (j1 - j0 + 2) * 2.0**-23 * (1.5 * sc[j0:j1] @ np.abs(G))
+        assert (np.abs(H - A[j0:j1].T @ G) / bound).max() <= 1.0, (j0, j1)
+
+
 @pytest.mark.parametrize("n,m,L", [(18, 200, 16), (65, 300, 20), (1023, 1200, 40), (1030, 700, 64), (4097, 500, 80),
                                    (20011, 300, 33), (130, 400, 100)])
 def test_omega_update(ctx, n, m, L):
