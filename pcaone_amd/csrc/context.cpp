@@ -598,6 +598,7 @@ void Context::configure(int prec, int Lr, const GemmTuning& t) {
   upre_.resize(nrows_n * lp);
   for (auto* b : {&H_, &H1_, &H2_, &gt_})
     PCAONE_HIP(hipMemsetAsync(b->get(), 0, b->bytes(), stream));
+  h_zero_[1] = h_zero_[2] = false;
   small_.resize(2 * 128 * 128);
   red_cap_ = std::max<uint64_t>({gram_partial_elems(std::max<uint64_t>(M, N), lp), 2048 * 256,
                                  epi_g_fused_partial_elems(rows_s_, lp)});
@@ -903,8 +904,10 @@ void Context::h_half(uint64_t j0, uint64_t j1, int hmode) {
   const uint64_t nch_h = ph.nchunks;
   // hmode 0: H = ..., 1: H1 += ..., 2: H2 += ..., 3: H += ... (blocks of one pass)
   double* target = (hmode == 0 || hmode == 3) ? H_.get() : (hmode == 1 ? H1_.get() : H2_.get());
-  launch_epi_h(form_h, part_.get(), nch_h, h.ychunk, N, rows_t_, lp, bvec_.get(), target, hmode == 0 ? 0 : 1, stream,
+  const bool fresh = hmode == 0 || ((hmode == 1 || hmode == 2) && h_zero_[hmode]);
+  launch_epi_h(form_h, part_.get(), nch_h, h.ychunk, N, rows_t_, lp, bvec_.get(), target, fresh ? 0 : 1, stream,
                i8_mul(1));
+  if (hmode == 1 || hmode == 2) h_zero_[hmode] = false;
   if (lnmiss_ && miss_tiled_) {
     launch_compact_rows(gwin, nwin, lp, L, cpitch_, true, csh_.get(), stream);
     MissTiledSpmmArgs m{};
@@ -1050,15 +1053,27 @@ void Context::update_missing_weights() {
 }
 
 void Context::zero_h(int which) {
-  DevBuf<double>& b = which == 0 ? H_ : (which == 1 ? H1_ : H2_);
+  if (which != 0) {
+    h_zero_[which] = true;
+    return;
+  }
+  PCAONE_HIP(hipMemsetAsync(H_.get(), 0, H_.bytes(), stream));
+  ++h_version_;
+}
+
+void Context::settle_h(int which) {
+  if (!h_zero_[which]) return;
+  DevBuf<double>& b = which == 1 ? H1_ : H2_;
   PCAONE_HIP(hipMemsetAsync(b.get(), 0, b.bytes(), stream));
-  if (which == 0) ++h_version_;
+  h_zero_[which] = false;
 }
 
 void Context::omega_from(int src, bool flip) {
   require(L > 0, kErrState, "configure() first");
   const bool deferred = deferred_thinq && deferred_ok();
   if (src == 1) {
+    settle_h(1);
+    settle_h(2);
     ++h_version_;
     if (deferred) {  // H = H1 + H2 on the way into its Gram matrix
       launch_gram_add(H1_.get(), H2_.get(), H_.get(), N, lp, red_.get(), red_cap_, ldev_.get(), stream);
@@ -1150,8 +1165,9 @@ void restore_dev(DevBuf<T>& dst, const DevBuf<T>& src, hipStream_t s) {
 }  // namespace
 
 void Context::epoch_checkpoint() {
-  copy_dev(ck_H1_, H1_, stream);
-  copy_dev(ck_H2_, H2_, stream);
+  std::copy(h_zero_, h_zero_ + 3, ck_zero_);
+  if (!h_zero_[1]) copy_dev(ck_H1_, H1_, stream);
+  if (!h_zero_[2]) copy_dev(ck_H2_, H2_, stream);
   copy_dev(ck_omega_, omega_, stream);
   copy_dev(ck_omega_r_, omega_r_, stream);
   copy_dev(ck_colsum_, colsum_, stream);
@@ -1168,8 +1184,9 @@ bool Context::epoch_thinq_failed() {
 }
 
 void Context::epoch_rollback() {
-  restore_dev(H1_, ck_H1_, stream);
-  restore_dev(H2_, ck_H2_, stream);
+  std::copy(ck_zero_, ck_zero_ + 3, h_zero_);
+  if (!h_zero_[1]) restore_dev(H1_, ck_H1_, stream);
+  if (!h_zero_[2]) restore_dev(H2_, ck_H2_, stream);
   restore_dev(omega_, ck_omega_, stream);
   restore_dev(omega_r_, ck_omega_r_, stream);
   restore_dev(colsum_, ck_colsum_, stream);
@@ -1420,6 +1437,7 @@ void Context::download_g(uint64_t j0, uint64_t j1, double* G) {
 void Context::download_h(int which, double* H) {
   require(L > 0, kErrState, "configure() first");
   require(which >= 0 && which <= 2, kErrArgument, "get_h: which must be 0 (H), 1 (H1) or 2 (H2)");
+  if (which) settle_h(which);
   download_cols(which == 0 ? H_.get() : (which == 1 ? H1_.get() : H2_.get()), N, lp, L, tmp_n_.get(), H);
 }
 

@@ -326,6 +326,10 @@ class Context {
   bool res_as_read_ = false;
   DevBuf<double> ldev_;
   DevBuf<int> lstatus_;
+  // H1 / H2 stand for zero until something is added: the first product writes
+  // them instead of adding to zeros that a launch of its own put there
+  bool h_zero_[3] = {false, false, false}, ck_zero_[3] = {false, false, false};  // [1], [2]
+  void settle_h(int which);
   DevBuf<double> ck_H1_, ck_H2_, ck_omega_, ck_omega_r_, ck_colsum_, ck_i8s_;  // epoch checkpoint
   DevBuf<unsigned char> ck_wg_;
   uint64_t gram_dev_version_ = ~0ull;

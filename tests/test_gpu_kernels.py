@@ -105,6 +105,37 @@ def test_cut_windows_match_whole_ones(ctx, form, miss):
         assert (np.abs(H - A[j0:j1].T @ G) / bound).max() <= 1.0, (j0, j1)
 
 
+@pytest.mark.parametrize("miss", [0.0, 0.1])
+def test_zeroed_h1_and_h2(ctx, miss):
+    """H1 and H2 after zero_h: read back as zeros, the first window written, the second added, also when the zeroed
+    one is summed into H untouched."""
+    say(f"zeroed H1, H2 miss={miss}")
+    rng = np.random.default_rng(3)
+    n, m, L = 70, 300, 12
+    ctx.upload_packed(pack(random_codes(rng, m, n, miss)), n)
+    ctx.standardize()
+    ctx.configure("fp64", L)
+    ctx.set_omega(rng.standard_normal((n, L)))
+    ctx.sketch(0, 130, 0)
+    a = ctx.get_h(0, L)
+    ctx.sketch(130, m, 0)
+    b = ctx.get_h(0, L)
+    for which in (1, 2):
+        ctx.sketch(0, m, which)  # what zeroing has to undo
+        ctx.zero_h(which)
+        assert not ctx.get_h(which, L).any()
+        ctx.zero_h(which)
+        ctx.sketch(0, 130, which)
+        np.testing.assert_array_equal(ctx.get_h(which, L), a)
+        ctx.sketch(130, m, which)
+        if not miss:  # a window's correction is a sum of its own: (a + dense part) + correction
+            np.testing.assert_array_equal(ctx.get_h(which, L), a + b)
+        ctx.zero_h(which)
+    ctx.sketch(0, 130, 1)
+    ctx.update_omega(1)  # H = H1 + H2
+    np.testing.assert_array_equal(ctx.get_h(0, L), a)
+
+
 @pytest.mark.parametrize("n,m,L", [(18, 200, 16), (65, 300, 20), (1023, 1200, 40), (1030, 700, 64), (4097, 500, 80),
                                    (20011, 300, 33), (130, 400, 100)])
 def test_omega_update(ctx, n, m, L):
