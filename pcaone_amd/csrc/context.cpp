@@ -805,13 +805,16 @@ void Context::sketch(uint64_t j0, uint64_t j1, int hmode) {
   const uint64_t off = jl % kKStep;
   const uint64_t klen = round_up(off + nwin, kKStep);
   const uint32_t right = (uint32_t)(klen - off - nwin);
+  bool maxima = false;
   if (!lnmiss_ && !form_colscaled(form_g) && !form_colscaled(form_h)) {
     launch_epi_g_fused(form_h, part_.get(), nch_g, g.ychunk, nwin, lp, sc_.get() + j0, cF_.get() + j0,
                        colsum_.get(), gwin, wh_.get() + off * wb, wh_pitch_, (uint64_t)lp * wh_pitch_, red_.get(),
                        bvec_.get(), (uint32_t)off, right, stream);
   } else {
-    launch_epi_g(form_g, part_.get(), nch_g, g.ychunk, nwin, nwin, lp, sc_.get() + j0, cF_.get() + j0,
-                 colsum_.get(), gwin, stream, i8_mul(0));
+    // the column maxima of diag(sc) G~ with it, where nothing is added to G~ afterwards
+    maxima = launch_epi_g(form_g, part_.get(), nch_g, g.ychunk, nwin, nwin, lp, sc_.get() + j0, cF_.get() + j0,
+                          colsum_.get(), gwin, stream, i8_mul(0),
+                          !lnmiss_ && form_colscaled(form_h) ? i8max_.get() : nullptr);
   }
   if (lnmiss_ && miss_tiled_) {
     update_missing_weights();
@@ -864,7 +867,8 @@ void Context::sketch(uint64_t j0, uint64_t j1, int hmode) {
   }
   if (lnmiss_ || form_colscaled(form_g) || form_colscaled(form_h)) {
     if (form_colscaled(form_h))
-      launch_col_scales(form_h, gwin, nwin, lp, sc_.get() + j0, i8max_.get(), i8_scale(1), i8_mul(1), stream);
+      launch_col_scales(form_h, maxima ? nullptr : gwin, nwin, lp, sc_.get() + j0, i8max_.get(), i8_scale(1),
+                        i8_mul(1), stream);
     launch_make_pieces(form_h, gwin, nwin, nwin, lp, sc_.get() + j0, nullptr, wh_.get() + off * wb, wh_pitch_,
                        (uint64_t)lp * wh_pitch_, gwin, nullptr, stream, i8_scale(1), sc_.get() + j0, cF_.get() + j0,
                        red_.get(), red_cap_, bvec_.get(), (uint32_t)off, right);

@@ -62,12 +62,13 @@ void launch_make_pieces(Form f, const double* X, uint64_t nreal, uint64_t rows_p
 // I8: scale[l] = m_l / kI8Max, mul[l] = 2 scale[l] (the genotype operand is
 // v/2); F8: scale[l] = the power of two that brings m_l into (224, 448],
 // mul[l] = scale[l].  An all-zero column has scale 1.  maxbits: lp words of
-// scratch.
+// scratch; X null: they hold the m_l already (launch_epi_g with maxbits returned
+// true, rowscale = sc).
 void launch_col_scales(Form f, const double* X, uint64_t nreal, int lp, const double* rowscale,
                        unsigned long long* maxbits, double* scale, double* mul, hipStream_t s);
-void launch_epi_g(Form f, const void* P, uint64_t nchunks, uint64_t chunk_stride, uint64_t nreal, uint64_t rows_pad,
+bool launch_epi_g(Form f, const void* P, uint64_t nchunks, uint64_t chunk_stride, uint64_t nreal, uint64_t rows_pad,
                   int lp, const double* sc, const double* cf, const double* colsum, double* out, hipStream_t s,
-                  const double* colmul = nullptr);
+                  const double* colmul = nullptr, unsigned long long* maxbits = nullptr);
 // G epilogue fused with the operand split, for data without missing entries
 // (not for I8, whose column scales need the whole window first):
 // gout (nwin x lp) = G~ window, Wt pieces of diag(sc) G~ (window offset
