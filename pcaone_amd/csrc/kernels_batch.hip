@@ -715,17 +715,11 @@ __device__ void sm_sym_eig(double* A, double* V, double* w, double* tmp, int n, 
       __syncthreads();
     }
   }
-  // descending order: an eigenvalue's rank counts the larger ones (and equal ones before it)
   __syncthreads();
   if (tid < n) {
-    const double x = A[tid * P + tid];
-    int r = 0;
-    for (int j = 0; j < n; ++j) {
-      const double y = A[j * P + j];
-      r += y > x || (y == x && j < tid) ? 1 : 0;
-    }
+    const int r = place_descending(A, P + 1, n, tid);
     perm[r] = tid;
-    w[r] = x;
+    w[r] = A[tid * P + tid];
   }
   __syncthreads();
   for (int v = tid; v < LP * LP; v += kSmallThreads) {

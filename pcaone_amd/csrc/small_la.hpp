@@ -76,6 +76,19 @@ __device__ __forceinline__ double quotient(double x, double d, double inv) {
   const double q = x * inv;
   return fma(fma(-q, d, x), inv, q);
 }
+// Place of x[i stride] among the n values x[0], x[stride], ... in descending order,
+// NaNs after the numbers and equal ones by index: a total order, so that the n
+// places are a permutation whatever the values.
+__host__ __device__ __forceinline__ int place_descending(const double* x, int stride, int n, int i) {
+  const double v = x[i * stride];
+  int place = 0;
+  for (int j = 0; j < n; ++j) {
+    const double y = x[j * stride];
+    const bool ahead = v != v ? y == y || j < i : y > v || (y == v && j < i);
+    place += ahead ? 1 : 0;
+  }
+  return place;
+}
 // 1 / x to about one unit in the last place.
 __device__ __forceinline__ double recip_step(double x) {
   const double y = __builtin_amdgcn_rcp(x);
