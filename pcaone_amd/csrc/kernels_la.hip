@@ -26,27 +26,26 @@ inline unsigned grid_for(uint64_t n, unsigned block = 256, unsigned cap = 65535u
 
 
 // Operand pieces of one form for each value y = X[r][l] colsign[l] rowscale[r]
-// (F8 and I8 also divided by the column scale s; is = 1 / s), and the value they
-// sum to.
+// (F8 and I8: y / s, s the column scale), and the value they sum to (times s).
 template <Form F>
 struct Pieces;
 template <>
 struct Pieces<Form::FP64> {
   using w_t = double;
   static constexpr int P = 1;
-  __device__ static double make(double y, double, double, w_t* pc) { return pc[0] = y; }
+  __device__ static double make(double y, double, w_t* pc) { return pc[0] = y; }
 };
 template <>
 struct Pieces<Form::FP32> {
   using w_t = float;
   static constexpr int P = 1;
-  __device__ static double make(double y, double, double, w_t* pc) { return (double)(pc[0] = (float)y); }
+  __device__ static double make(double y, double, w_t* pc) { return (double)(pc[0] = (float)y); }
 };
 template <>
 struct Pieces<Form::FP16> {
   using w_t = uint16_t;
   static constexpr int P = 1;
-  __device__ static double make(double y, double, double, w_t* pc) {
+  __device__ static double make(double y, double, w_t* pc) {
     pc[0] = fp16_bits(y);
     return fp16_value(pc[0]);
   }
@@ -55,7 +54,7 @@ template <>
 struct Pieces<Form::BF16X1> {
   using w_t = uint16_t;
   static constexpr int P = 1;
-  __device__ static double make(double y, double, double, w_t* pc) {
+  __device__ static double make(double y, double, w_t* pc) {
     pc[0] = bf16_bits((float)y);
     return (double)bf16_value(pc[0]);
   }
@@ -64,7 +63,7 @@ template <>
 struct Pieces<Form::BF16> {
   using w_t = uint16_t;
   static constexpr int P = 2;
-  __device__ static double make(double y, double, double, w_t* pc) {
+  __device__ static double make(double y, double, w_t* pc) {
     pc[0] = bf16_bits((float)y);
     const double back = (double)bf16_value(pc[0]);
     pc[1] = bf16_bits((float)(y - back));
@@ -75,10 +74,9 @@ template <>
 struct Pieces<Form::F8> {
   using w_t = uint8_t;
   static constexpr int P = 3;
-  // y / s (exact: s is a power of two, |y / s| <= 448) as three E4M3
+  // x1 = y / s (exact: s is a power of two, |y / s| <= 448) as three E4M3
   // pieces, each the nearest E4M3 to what the previous ones left
-  __device__ static double make(double y, double s, double is, w_t* pc) {
-    const double x1 = y * is;
+  __device__ static double make(double x1, double s, w_t* pc) {
     double v1, v2, v3;
     pc[0] = e4m3_bits(x1, &v1);
     pc[1] = e4m3_bits(x1 - v1, &v2);
@@ -91,8 +89,8 @@ struct Pieces<Form::I8> {
   using w_t = uint8_t;
   static constexpr int P = 2;
   // q = rint(y / s) within +-kI8Max; q = 256 q_hi + q_lo, q_lo in [-128, 127]
-  __device__ static double make(double y, double s, double is, w_t* pc) {
-    const int q = (int)fmin(fmax(rint(quotient(y, s, is)), -(double)kI8Max), (double)kI8Max);
+  __device__ static double make(double ys, double s, w_t* pc) {
+    const int q = (int)fmin(fmax(rint(ys), -(double)kI8Max), (double)kI8Max);
     const int hi = (q + 128) >> 8, lo = q - 256 * hi;
     pc[0] = (uint8_t)(int8_t)hi;
     pc[1] = (uint8_t)(int8_t)lo;
@@ -244,9 +242,12 @@ __global__ void __launch_bounds__(256) k_make_pieces(const double* X, uint64_t n
         double rd[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
+          double y = x[u][q] * rs[u];
+          if constexpr (F == Form::F8) y *= is[q];
+          if constexpr (F == Form::I8) y = quotient(y, sl[q], is[q]);
           w_t pc[P];
-          const double back = PF::make(x[u][q] * rs[u], sl[q], is[q], pc);
-          rd[q] = live ? (rowscale ? quotient(back, rs[u], irs) : back) : 0.0;
+          const double back = PF::make(y, sl[q], pc);
+          rd[q] = live ? (rowscale ? quotient_any(back, rs[u], irs) : back) : 0.0;
           b4[q] += w[u] * rd[q];
 #pragma unroll
           for (int p = 0; p < P; ++p) pt[(p * lp + 4 * cg + q) * PITCH + r] = pc[p];
@@ -480,8 +481,8 @@ __global__ void __launch_bounds__(256) k_epi_g_fused(const PT* __restrict__ part
         for (int q = 0; q < 4; ++q) {
           const double g = fma(0.25 * s, y[u][q], beta * cs[q]);
           w_t pc[P];
-          const double back = PF::make(g * s, 1.0, 1.0, pc);
-          gr4[q] = s != 0.0 ? quotient(back, s, is) : 0.0;
+          const double back = PF::make(g * s, 1.0, pc);
+          gr4[q] = s != 0.0 ? quotient_any(back, s, is) : 0.0;
           b4[q] += beta * gr4[q];
 #pragma unroll
           for (int p = 0; p < P; ++p) pt[(p * lp + 4 * cg + q) * PITCH + r] = pc[p];

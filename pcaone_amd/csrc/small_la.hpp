@@ -71,10 +71,17 @@ __device__ __forceinline__ void root_and_inverse(double d, double& r, double& in
   r = fma(fma(-g, g, d), 0.5 * y, g);
   inv = fma(fma(-r, y, 1.0), y, y);
 }
-// x / d with inv = 1 / d, rounded as the quotient is (Markstein's correction).
-__device__ __forceinline__ double quotient(double x, double d, double inv) {
+// x / d with inv = 1 / d, rounded as the quotient is (Markstein's correction), for
+// finite d and inv and a finite x that is 0 or at least 2^-960 in size (the residual
+// x - q d is exact), without overflow.
+__host__ __device__ __forceinline__ double quotient(double x, double d, double inv) {
   const double q = x * inv;
   return fma(fma(-q, d, x), inv, q);
+}
+// The same where x may be infinite or NaN or the quotient overflow: as the division.
+__host__ __device__ __forceinline__ double quotient_any(double x, double d, double inv) {
+  const double q = x * inv;
+  return fabs(q) < INFINITY ? fma(fma(-q, d, x), inv, q) : q;
 }
 // Place of x[i stride] among the n values x[0], x[stride], ... in descending order,
 // NaNs after the numbers and equal ones by index: a total order, so that the n

@@ -16,6 +16,9 @@ extern "C" {
 void places(const double* x, int stride, int n, int* out) {
   for (int i = 0; i < n; ++i) out[i] = place_descending(x, stride, n, i);
 }
+void divisions(const double* x, const double* d, int n, double* out) {
+  for (int i = 0; i < n; ++i) out[i] = quotient_any(x[i], d[i], 1.0 / d[i]);
+}
 }
 '''
 
@@ -50,3 +53,30 @@ def test_descending_places_are_a_permutation(host, values):
     numbers = ordered[~np.isnan(ordered)]
     assert not np.isnan(ordered[:len(numbers)]).any()
     assert np.all(numbers[:-1] >= numbers[1:])
+
+
+def divisions(host, x, d):
+    x, d = np.ascontiguousarray(x, dtype=np.float64), np.ascontiguousarray(d, dtype=np.float64)
+    out = np.empty_like(x)
+    host.divisions(dptr(x), dptr(d), len(x), dptr(out))
+    return out
+
+
+def test_divisions_round_as_the_quotient(host):
+    """Random significands and exponents (and quotients next to ties and to 1): the very bits of x / d."""
+    rng = np.random.default_rng(1)
+    n = 200000
+    x = np.ldexp(1 + rng.random(n), rng.integers(-400, 400, n)) * rng.choice([-1, 1], n)
+    d = np.ldexp(1 + rng.random(n), rng.integers(-400, 400, n))
+    near = 1 + rng.integers(0, 64, n) * 2.0**-52
+    for a, b in ((x, d), (d * near, d), (near, 1 + rng.integers(0, 64, n) * 2.0**-52), (x, np.sqrt(d))):
+        np.testing.assert_array_equal(divisions(host, a, b), a / b)
+
+
+def test_divisions_of_infinities_and_zeros(host):
+    """Dividends that are zero, infinite, NaN or the smallest that the residual allows, and overflow."""
+    x = np.array([0.0, -0.0, 1.0, -3.0, np.inf, -np.inf, np.nan, 1e308, -1.7e308, 2.0**-960, -3 * 2.0**-959])
+    x, d = (a.ravel() for a in np.meshgrid(x, [1.0, 3.0, 1.4142135e9, 0.125, 1e-4]))
+    with np.errstate(all="ignore"):
+        ref = x / d
+    np.testing.assert_array_equal(divisions(host, x, d), ref)

@@ -312,3 +312,28 @@ def test_fp32_column_groups_same_bits(ctx, k):
             np.testing.assert_array_equal(r.S, runs[0].S)
             np.testing.assert_array_equal(r.U, runs[0].U)
             np.testing.assert_array_equal(r.V, runs[0].V)
+
+
+@pytest.mark.parametrize("miss", [0.0, 0.05])
+def test_overflowing_pieces_stay_infinite(ctx, miss):
+    """FP16 pieces of diag(sc) G beyond 65,504 are infinite, and so is G, with its sign, as the piece divided by sc."""
+    say(f"overflowing pieces miss={miss}")
+    rng = np.random.default_rng(9)
+    n, m, L = 130, 300, 20
+    codes = random_codes(rng, m, n, miss)
+    ctx.upload_packed(pack(codes), n)
+    ctx.standardize()
+    ctx.configure("fp16", L)
+    omega = 1500 * rng.standard_normal((n, L))
+    ctx.set_omega(omega)
+    ctx.sketch(0, m, 0)
+    A, sc = standardized(codes)
+    exact = A @ omega
+    G = ctx.get_g(0, m, L)
+    # Omega's FP16 rounding moves sc G by at most 2^-11 sc |A| |Omega| <= a few units of 1,000: 10,000 apart
+    size = np.abs(sc[:, None] * exact)
+    over, under = size > 75000, size < 55000
+    assert over.any() and under.any()
+    np.testing.assert_array_equal(G[over], np.copysign(np.inf, exact[over]))
+    bound = 2.0**-10 * (np.abs(A) @ np.abs(omega))
+    assert (np.abs(G - exact) / bound)[under].max() <= 1.0
