@@ -202,11 +202,13 @@ __global__ void __launch_bounds__(256) k_make_pieces(const double* X, uint64_t n
   double b4[4] = {0.0, 0.0, 0.0, 0.0};
   if (act) {
     double cs[4] = {1.0, 1.0, 1.0, 1.0}, sl[4] = {1.0, 1.0, 1.0, 1.0}, is[4];
+    bool plain = true;  // the scales' reciprocals serve (a column near the ends of the FP64 range is divided)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       if (colsign) cs[q] = colsign[4 * cg + q];
       if constexpr (F == Form::F8 || F == Form::I8) sl[q] = colscale[4 * cg + q];
       is[q] = 1.0 / sl[q];
+      plain = plain && sl[q] >= 0x1p-900 && sl[q] <= 0x1p900;
     }
     for (int rb = rg; rb < nr; rb += kEpiBatch * RG) {
       double x[kEpiBatch][4], rs[kEpiBatch], w[kEpiBatch];
@@ -243,8 +245,8 @@ __global__ void __launch_bounds__(256) k_make_pieces(const double* X, uint64_t n
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           double y = x[u][q] * rs[u];
-          if constexpr (F == Form::F8) y *= is[q];
-          if constexpr (F == Form::I8) y = quotient(y, sl[q], is[q]);
+          if constexpr (F == Form::F8) y = plain ? y * is[q] : y / sl[q];
+          if constexpr (F == Form::I8) y = plain ? quotient(y, sl[q], is[q]) : y / sl[q];
           w_t pc[P];
           const double back = PF::make(y, sl[q], pc);
           rd[q] = live ? (rowscale ? quotient_any(back, rs[u], irs) : back) : 0.0;

@@ -337,3 +337,30 @@ def test_overflowing_pieces_stay_infinite(ctx, miss):
     np.testing.assert_array_equal(G[over], np.copysign(np.inf, exact[over]))
     bound = 2.0**-10 * (np.abs(A) @ np.abs(omega))
     assert (np.abs(G - exact) / bound)[under].max() <= 1.0
+
+
+@pytest.mark.parametrize("form", ["fp8", "int8"])
+def test_tiny_columns_keep_their_digits(ctx, form):
+    """Column scales whose reciprocal overflows: a column of Omega near the smallest FP64 numbers gives the G of the
+    same column at an ordinary size, scaled."""
+    say(f"tiny columns {form}")
+    rng = np.random.default_rng(10)
+    n, m, L = 130, 300, 20
+    codes = random_codes(rng, m, n, 0.0)
+    ctx.upload_packed(pack(codes), n)
+    ctx.standardize()
+    ctx.configure(form, L)
+    omega = rng.standard_normal((n, L))
+    ctx.set_omega(omega)
+    ctx.sketch(0, m, 0)
+    G = ctx.get_g(0, m, L)
+    small = omega.copy()
+    small[:, 3] *= 2.0**-1020
+    ctx.set_omega(small)
+    ctx.sketch(0, m, 0)
+    T = ctx.get_g(0, m, L)
+    np.testing.assert_array_equal(np.delete(T, 3, 1), np.delete(G, 3, 1))
+    # the scale itself has 2^-1074 steps there: 2^-40 of its size at the least, and G's a few dozen more
+    A, _ = standardized(codes)
+    bound = 2.0**-12 * (np.abs(A) @ np.abs(omega[:, 3]))
+    assert (np.abs(np.ldexp(T[:, 3], 1020) - G[:, 3]) / bound).max() <= 1.0
