@@ -495,15 +495,15 @@ void Batch::run(const Param& p, bool want_v, bool use_graph, BatchResult& out) {
 void Batch::get_u(uint32_t c, double* U) {
   require(c < size() && c < stop_epoch_.size(), kErrState, "batch: no result for this cohort");
   const int buf = (stop_epoch_[c] & 1) ? kBufU1 : kBufU0;
-  cols_.resize((uint64_t)*std::max_element(N_.begin(), N_.end()) * last_k_);  // one allocation serves every cohort
-  ctx_.download_cols(host_coh_[c].mat[buf], N_[c], LP, last_k_, cols_.get(), U);
+  // between runs the cohort's H R^-1 is scratch (N x LP; every run writes it before it reads it)
+  ctx_.download_cols(host_coh_[c].mat[buf], N_[c], LP, last_k_, host_coh_[c].mat[kBufTmpN], U);
 }
 
 void Batch::get_v(uint32_t c, double* V) {
   require(c < size() && c < stop_epoch_.size(), kErrState, "batch: no result for this cohort");
   require(layout_.want_v && host_coh_[c].mat[kBufV], kErrState, "batch: run with loadings first");
-  cols_.resize(*std::max_element(M_.begin(), M_.end()) * (uint64_t)last_k_);
-  ctx_.download_cols(host_coh_[c].mat[kBufV], M_[c], LP, last_k_, cols_.get(), V);
+  // and so is its G~ (M x LP)
+  ctx_.download_cols(host_coh_[c].mat[kBufV], M_[c], LP, last_k_, host_coh_[c].mat[kBufG], V);
 }
 
 }  // namespace pcaone

@@ -87,7 +87,7 @@ class Batch {
              g.wm == o.g.wm && g.waves == o.g.waves && h.wm == o.h.wm && h.waves == o.h.waves;
     }
   } layout_;
-  DevBuf<double> mats_, scf_, vecs_, partial_, cols_;
+  DevBuf<double> mats_, scf_, vecs_, partial_;
   DevBuf<unsigned char> pieces_, part_;
   DevBuf<BatchSmall> small_;
   DevBuf<BatchCohort> coh_;

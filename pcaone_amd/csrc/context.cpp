@@ -714,9 +714,8 @@ void Context::stage_out(const double* dev, uint64_t count, double* host) {
   }
 }
 
-void Context::download_cols(const double* src, uint64_t rows, int pitch, int k, double* tmp, double* out,
-                            const uint32_t* place) {
-  launch_rows_to_colmajor(src, rows, pitch, k, tmp, stream, place);
+void Context::download_cols(const double* src, uint64_t rows, int pitch, int k, double* tmp, double* out) {
+  launch_rows_to_colmajor(src, rows, pitch, k, tmp, rows, stream);
   stage_out(tmp, rows * (uint64_t)k, out);
 }
 
@@ -1510,11 +1509,17 @@ void Context::download_v(int k, double* V) { download_cols(vbuf_.get(), M, lp, k
 
 void Context::download_v_original(int k, double* V) {
   if (perm_identity_) return download_v(k, V);
-  // column i of the device order is SNP perm[i]
+  // column i of the device order is SNP perm[i]; the positions go through the
+  // reductions' scratch, as many at a time as it holds (over a million)
   static_assert(sizeof(int) == sizeof(uint32_t));
-  place_.resize(M);
-  PCAONE_HIP(hipMemcpyAsync(place_.get(), perm.data(), M * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
-  download_cols(vbuf_.get(), M, lp, k, tmp_m_.get(), V, place_.get());
+  uint32_t* place = reinterpret_cast<uint32_t*>(red_.get());
+  const uint64_t cap = red_.bytes() / sizeof(uint32_t);
+  for (uint64_t r0 = 0; r0 < M; r0 += cap) {
+    const uint64_t n = std::min(cap, M - r0);
+    PCAONE_HIP(hipMemcpyAsync(place, perm.data() + r0, n * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
+    launch_rows_to_colmajor(vbuf_.get() + r0 * lp, n, lp, k, tmp_m_.get(), M, stream, place);
+  }
+  stage_out(tmp_m_.get(), M * (uint64_t)k, V);
 }
 
 }  // namespace pcaone

@@ -174,9 +174,8 @@ class Context {
   void download_v(int k, double* V);
   void download_v_original(int k, double* V);  // the same in the original SNP order
   // The first k columns of src (rows x pitch on the device, row-major) to out
-  // (rows x k, column-major; row r at place[r] when given); tmp: rows x k.
-  void download_cols(const double* src, uint64_t rows, int pitch, int k, double* tmp, double* out,
-                     const uint32_t* place = nullptr);
+  // (rows x k, column-major); tmp: rows x k.
+  void download_cols(const double* src, uint64_t rows, int pitch, int k, double* tmp, double* out);
   // G of the last sketches, rows [j0, j1) (current column order), and H / H1 / H2:
   // column-major FP64 with L columns.
   void download_g(uint64_t j0, uint64_t j1, double* G);
@@ -308,7 +307,6 @@ class Context {
   DevBuf<unsigned char> wg_, wh_;
   uint64_t wg_pitch_ = 0, wh_pitch_ = 0;
   DevBuf<double> gt_, H_, H1_, H2_, tmp_n_, tmp_m_, ucur_, upre_, vbuf_, vpre_;
-  DevBuf<uint32_t> place_;  // original position of every column (loadings of a permuted run)
   DevBuf<unsigned char> part_;
   DevBuf<double> small_, red_;
   uint64_t red_cap_ = 0;

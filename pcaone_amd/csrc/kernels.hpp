@@ -173,9 +173,10 @@ void launch_gather_f64(const double* src, const uint32_t* idx, uint64_t n, doubl
 // Column-major n x L (leading dimension n) -> row-major rows_pad x lp (zero padded).
 void launch_colmajor_to_rows(const double* src, uint64_t n, int L, int lp, uint64_t rows_pad, double* dst,
                              hipStream_t s);
-// Row-major n x lp -> column-major n x k.
-void launch_rows_to_colmajor(const double* src, uint64_t n, int lp, int k, double* dst, hipStream_t s,
-                             const uint32_t* place = nullptr);
+// Row-major n x lp -> k columns of col_len values, row r at position r (place[r]
+// when given).
+void launch_rows_to_colmajor(const double* src, uint64_t n, int lp, int k, double* dst, uint64_t col_len,
+                             hipStream_t s, const uint32_t* place = nullptr);
 // Y = X + Z elementwise (n elements).
 void launch_add(const double* X, const double* Z, double* Y, uint64_t n, hipStream_t s);
 // Missing-entry corrections, in two steps.

@@ -932,12 +932,12 @@ __global__ void k_colmajor_to_rows(const double* __restrict__ src, uint64_t n, i
   }
 }
 
-// Row-major n x lp -> column-major n x k (row r at place[r] when given), 32 rows per workgroup through LDS:
-// whole rows read, 256-byte runs of each column written (one thread per output
+// Row-major n x lp -> k columns of col_len values (row r at place[r] when given, else at r), 32 rows per workgroup
+// through LDS: whole rows read, 256-byte runs of each column written (one thread per output
 // value would read 8 bytes of every row line it touched).  Bound by HBM: 27 us
 // for 100,003 x 40 from lp = 48.
 __global__ void __launch_bounds__(256) k_rows_to_colmajor(const double* __restrict__ src, uint64_t n, int lp, int k,
-                                                          double* __restrict__ dst,
+                                                          double* __restrict__ dst, uint64_t col_len,
                                                           const uint32_t* __restrict__ place) {
   extern __shared__ double tile[];  // 32 rows of lp + 1
   const uint64_t r0 = (uint64_t)blockIdx.x * 32;
@@ -949,7 +949,7 @@ __global__ void __launch_bounds__(256) k_rows_to_colmajor(const double* __restri
   __syncthreads();
   for (int v = threadIdx.x; v < 32 * k; v += 256) {
     const int j = v >> 5, r = v & 31;
-    if (r < nr) dst[(uint64_t)j * n + (place ? place[r0 + r] : r0 + r)] = tile[r * (lp + 1) + j];
+    if (r < nr) dst[(uint64_t)j * col_len + (place ? place[r0 + r] : r0 + r)] = tile[r * (lp + 1) + j];
   }
 }
 
@@ -1514,12 +1514,12 @@ void launch_gather_f64(const double* src, const uint32_t* idx, uint64_t n, doubl
   check_launch("gather_f64");
 }
 
-void launch_rows_to_colmajor(const double* src, uint64_t n, int lp, int k, double* dst, hipStream_t s,
-                             const uint32_t* place) {
+void launch_rows_to_colmajor(const double* src, uint64_t n, int lp, int k, double* dst, uint64_t col_len,
+                             hipStream_t s, const uint32_t* place) {
   if (!n || !k) return;
   require(lp >= 1 && lp <= 128 && k <= lp, kErrArgument, "rows_to_colmajor: bad column count");
   hipLaunchKernelGGL(k_rows_to_colmajor, dim3((unsigned)((n + 31) / 32)), dim3(256), 32 * (lp + 1) * sizeof(double), s,
-                     src, n, lp, k, dst, place);
+                     src, n, lp, k, dst, col_len, place);
   check_launch("rows_to_colmajor");
 }
 

@@ -1,8 +1,10 @@
 """Single kernels of the device path at the sizes where their tiles, remainders and scans can go wrong."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from pcaone_amd import api
+from pcaone_amd import _lib, api
 
 pytestmark = pytest.mark.gpu
 
@@ -364,3 +366,57 @@ def test_tiny_columns_keep_their_digits(ctx, form):
     A, _ = standardized(codes)
     bound = 2.0**-12 * (np.abs(A) @ np.abs(omega[:, 3]))
     assert (np.abs(np.ldexp(T[:, 3], 1020) - G[:, 3]) / bound).max() <= 1.0
+
+
+def free_memory():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert _lib.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0  # of the runtime that the library has loaded
+    return free.value
+
+
+def test_batch_read_back_takes_no_device_memory(ctx):
+    """U and V of every cohort, twice, in any order, in the memory that the run left: the device's free memory stays,
+    and so do the results and those of the next run."""
+    say("batch read back in place")
+    rng = np.random.default_rng(12)
+    k = 16
+    kw = dict(svd=1, k=k, oversamples=10, maxp=2, tol=0.0, precision="fp32", kchunk_g=4096, kchunk_h=8192)
+    ctx.batch_upload([(pack(random_codes(rng, m, n, 0.0)), n) for n, m in [(60, 100000), (40000, 50), (300, 700)]])
+    first = ctx.batch_run(want_v=True, **kw)
+    assert np.all(first["status"] == 0)
+    before = free_memory()
+    got = [(ctx.batch_get_u(c), ctx.batch_get_v(c)) for c in range(3)]
+    assert free_memory() == before
+    for c in (2, 0, 1):
+        np.testing.assert_array_equal(ctx.batch_get_v(c), got[c][1])
+        np.testing.assert_array_equal(ctx.batch_get_u(c), got[c][0])
+    again = ctx.batch_run(want_v=True, **kw)
+    np.testing.assert_array_equal(again["S"], first["S"])
+    for c in range(3):
+        np.testing.assert_array_equal(ctx.batch_get_u(c), got[c][0])
+        np.testing.assert_array_equal(ctx.batch_get_v(c), got[c][1])
+        assert np.abs(got[c][1].T @ got[c][1] - np.eye(k)).max() < 1e-4  # whole columns of whole matrices
+
+
+def test_permuted_loadings_take_no_device_memory():
+    """Loadings of a shuffled run of more SNPs than one part of the positions holds (2 (2,048 256 + 2 128^2)): in
+    the memory of the run without them, every SNP in its place."""
+    n, m, k = 24, 1150000, 2
+    say(f"permuted loadings m={m}")
+    rng = np.random.default_rng(13)
+    codes = random_codes(rng, m, n, 0.0)
+    codes[::2, : n // 2] = 0
+    codes[1::3, n // 2:] = 3
+    kw = dict(svd=2, k=k, oversamples=10, maxp=6, tol=0.0, bands=4, precision="fp64")
+    with api.Context(0) as ctx:
+        ctx.upload_packed(pack(codes), n)
+        ctx.run(**kw)
+        before = free_memory()
+        r = ctx.run(want_v=True, **kw)
+        assert free_memory() == before
+    A, _ = standardized(codes)
+    proj = A @ r.U
+    for c in range(k):
+        assert np.dot(r.V[:, c], proj[:, c]) / np.linalg.norm(proj[:, c]) >= 0.999
+        tail = slice(m - 30000, m)  # past the first part
+        assert np.corrcoef(r.V[tail, c], proj[tail, c])[0, 1] >= 0.99
