@@ -24,7 +24,7 @@ constexpr int LP = kBatchLp;
 // X T 53 -> 15 us, Omega's pieces 83 -> 20 us.  The reductions keep whole items:
 // their order is part of the result.
 constexpr uint32_t kSliceRows = 128;
-constexpr unsigned kSlices = kBatchRowsPerItem / kSliceRows;
+constexpr unsigned kSlices = (kBatchRowsPerItem + kSliceRows - 1) / kSliceRows;  // the last may be short or empty
 
 template <Form F>
 using piece_t = typename std::conditional<
@@ -194,6 +194,7 @@ __global__ void __launch_bounds__(FLIP ? 1024 : 256) k_b_rowsum(BatchArgs a, con
 enum SumDest : int { kDestColsum = 0, kDestBvec, kDestGramA, kDestGramH, kDestAb };
 enum ItemList : int { kListM = 0, kListN, kListE };
 constexpr int kSumItems = 128;
+static_assert(LP % 32 == 0, "the widths LP, 2 LP and LP LP are whole groups of 32 values");
 
 __global__ void __launch_bounds__(1024) k_b_sum_items(BatchArgs a, const double* __restrict__ partial, int width,
                                                       int list, int dest, int state_req) {
