@@ -136,12 +136,8 @@ void RsvdOpData::fit_with_pi() {
   // EMU branch only runs with --emu; the device recomputes the imputed values
   // inside every product from (U S, V).
   if (!params_.emu) return;
-  require(!S.empty(), kErrState, "fit_with_pi before the first decomposition");
-  if (device_uv) {
-    ctx_.set_impute_device(S.data(), (int)S.size());
-    return;
-  }
-  fail(kErrInternal, "fit_with_pi: U and V are not on the device");
+  require(v_ready, kErrState, "fit_with_pi before the first decomposition");
+  ctx_.set_impute_device(S.data(), (int)S.size());  // computeUSV left U and V in the context
 }
 
 void RsvdOpData::computeUSV(int p, double tol) {
