@@ -24,7 +24,7 @@ __device__ __forceinline__ double fp16_value(uint16_t b) { return (double)__buil
 // 8 steps of 2^(E-3); below 2^-6 the step stays 2^-9.  Adding and taking off
 // 1.5 2^52 steps rounds to whole steps, ties to even; the exponent and the
 // three leading fraction bits of the result are the E4M3 bits.
-__device__ __forceinline__ uint8_t e4m3_bits(double y, double* val) {
+__host__ __device__ __forceinline__ uint8_t e4m3_bits(double y, double* val) {
   const double a = fmin(fmax(fabs(y), 0.0), 448.0);
   const uint32_t ex = (uint32_t)(__builtin_bit_cast(uint64_t, a) >> 52);
   const uint32_t em = ex < 1017u ? 1017u : ex;  // E = em - 1023 >= -6

@@ -60,16 +60,19 @@ __device__ __forceinline__ double quad_value(double v) {
   return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
 
-// sqrt(d) and 1 / sqrt(d), both rounded as the root and the quotient are, without
-// their range checks: v_rsq_f64 (2^-23), one third-order step, and Markstein's
-// corrections of the root and of its reciprocal.
-__device__ __forceinline__ void root_and_inverse(double d, double& r, double& inv) {
-  const double y0 = __builtin_amdgcn_rsq(d);
+// r = sqrt(d) and inv = 1 / r, both rounded as the root and the quotient are, without
+// their range checks, from y0 = 1 / sqrt(d) to 2^-23: one third-order step and
+// Markstein's corrections of the root and of its reciprocal.  (The one significand
+// that the latter does not cover, r of all ones, gives inv one unit low.)
+__host__ __device__ __forceinline__ void refine_root(double d, double y0, double& r, double& inv) {
   const double e = fma(-(d * y0), y0, 1.0);
   const double y = fma(y0 * e, fma(0.375, e, 0.5), y0);
   const double g = d * y;
   r = fma(fma(-g, g, d), 0.5 * y, g);
   inv = fma(fma(-r, y, 1.0), y, y);
+}
+__device__ __forceinline__ void root_and_inverse(double d, double& r, double& inv) {
+  refine_root(d, __builtin_amdgcn_rsq(d), r, inv);  // v_rsq_f64
 }
 // x / d with inv = 1 / d, rounded as the quotient is (Markstein's correction), for
 // finite d and inv and a finite x that is 0 or at least 2^-960 in size (the residual

@@ -316,6 +316,21 @@ def test_fp32_column_groups_same_bits(ctx, k):
             np.testing.assert_array_equal(r.V, runs[0].V)
 
 
+@pytest.mark.parametrize("form,L,wide", [("fp64", 17, 32), ("fp64", 20, 32), ("fp64", 28, 32), ("fp64", 36, 48),
+                                         ("fp64", 44, 48), ("fp64", 52, 64), ("fp64", 60, 64), ("fp32", 20, 32),
+                                         ("fp32", 25, 32), ("fp32", 40, 48)])
+def test_column_groups_same_bits_as_whole_blocks(ctx, form, L, wide):
+    """A product of L columns (the last ones in groups of 4) and the same W with more columns (16-column blocks
+    alone): the first L columns are the same bits, on values whose sums round at every step."""
+    say(f"{form} columns {L} of {wide}")
+    rng = np.random.default_rng(L)
+    nrows, ncodes = 513, 1000
+    rows = pack(rng.integers(0, 4, (nrows, ncodes)).astype(np.uint8))
+    W = rng.standard_normal((ncodes, wide)) * np.exp(3 * rng.standard_normal((ncodes, 1)))
+    whole = ctx.packed_gemm(form, rows, ncodes, W)
+    np.testing.assert_array_equal(ctx.packed_gemm(form, rows, ncodes, np.ascontiguousarray(W[:, :L])), whole[:, :L])
+
+
 @pytest.mark.parametrize("miss", [0.0, 0.05])
 def test_overflowing_pieces_stay_infinite(ctx, miss):
     """FP16 pieces of diag(sc) G beyond 65,504 are infinite, and so is G, with its sign, as the piece divided by sc."""
