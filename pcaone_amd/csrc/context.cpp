@@ -692,29 +692,54 @@ void Context::stage_out(const double* dev, uint64_t count, double* host) {
   // whole powers of two: a sequence of slightly larger reads does not pin memory anew each time
   pinned_.resize(std::bit_ceil(std::max<uint64_t>((n > 1 ? 2 : 1) * slot * 8, 256 << 10)));
   double* st = reinterpret_cast<double*>(pinned_.get());
+  // 256 KB and less by this thread alone: waking the others takes up to 50 us
+  const auto copy = [&](const double* from, uint64_t m, double* to) {
+    const int64_t pieces = 16;
+#pragma omp parallel for schedule(static) if (m > 32768)
+    for (int64_t q = 0; q < pieces; ++q) {
+      const uint64_t b0 = m * q / pieces, b1 = m * (q + 1) / pieces;
+      std::memcpy(to + b0, from + b0, (b1 - b0) * 8);
+    }
+  };
+  if (n <= 1) {  // no second slot, no events
+    PCAONE_HIP(hipMemcpyAsync(st, dev, count * 8, hipMemcpyDeviceToHost, stream));
+    PCAONE_HIP(hipStreamSynchronize(stream));
+    return copy(st, count, host);
+  }
   Event done[2];
   const auto send = [&](uint64_t c) {
     const uint64_t m = std::min(kSlot, count - c * kSlot);
     PCAONE_HIP(hipMemcpyAsync(st + (c & 1) * slot, dev + c * kSlot, m * 8, hipMemcpyDeviceToHost, stream));
     PCAONE_HIP(hipEventRecord(done[c & 1].get(), stream));
   };
-  if (n) send(0);
+  send(0);
   for (uint64_t c = 0; c < n; ++c) {
     if (c + 1 < n) send(c + 1);  // its slot was copied out in the step before
     PCAONE_HIP(hipEventSynchronize(done[c & 1].get()));
     const uint64_t m = std::min(kSlot, count - c * kSlot);
-    const double* from = st + (c & 1) * slot;
-    double* to = host + c * kSlot;
-    const int64_t pieces = 16;
-#pragma omp parallel for schedule(static)
-    for (int64_t q = 0; q < pieces; ++q) {
-      const uint64_t b0 = m * q / pieces, b1 = m * (q + 1) / pieces;
-      std::memcpy(to + b0, from + b0, (b1 - b0) * 8);
-    }
+    copy(st + (c & 1) * slot, m, host + c * kSlot);
   }
 }
 
+bool Context::download_rows(const double* src, uint64_t rows, int pitch, int k, double* out, const int* place) {
+  // A value over the link costs about a quarter of one transposed here; past
+  // 131,072 such units the transpose kernel's launch is the cheaper part: 512 x 32
+  // 15.5 us against 27 with the kernel, 2,048 x 16 35 against 32, 1,024 x 20 (of
+  // 32) 27 against 29.
+  constexpr uint64_t kDirect = 128 << 10;
+  if (rows * (uint64_t)(pitch + 4 * k) > kDirect) return false;
+  const uint64_t count = rows * (uint64_t)pitch;
+  pinned_.resize(std::bit_ceil(std::max<uint64_t>(count * 8, 256 << 10)));
+  const double* st = reinterpret_cast<const double*>(pinned_.get());
+  PCAONE_HIP(hipMemcpyAsync(pinned_.get(), src, count * 8, hipMemcpyDeviceToHost, stream));
+  PCAONE_HIP(hipStreamSynchronize(stream));
+  for (int j = 0; j < k; ++j)
+    for (uint64_t i = 0; i < rows; ++i) out[j * rows + (place ? place[i] : i)] = st[i * pitch + j];
+  return true;
+}
+
 void Context::download_cols(const double* src, uint64_t rows, int pitch, int k, double* tmp, double* out) {
+  if (download_rows(src, rows, pitch, k, out)) return;
   launch_rows_to_colmajor(src, rows, pitch, k, tmp, rows, stream);
   stage_out(tmp, rows * (uint64_t)k, out);
 }
@@ -1509,6 +1534,7 @@ void Context::download_v(int k, double* V) { download_cols(vbuf_.get(), M, lp, k
 
 void Context::download_v_original(int k, double* V) {
   if (perm_identity_) return download_v(k, V);
+  if (download_rows(vbuf_.get(), M, lp, k, V, perm.data())) return;
   // column i of the device order is SNP perm[i]; the positions go through the
   // reductions' scratch, as many at a time as it holds (over a million)
   static_assert(sizeof(int) == sizeof(uint32_t));

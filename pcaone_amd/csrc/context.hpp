@@ -176,6 +176,8 @@ class Context {
   // The first k columns of src (rows x pitch on the device, row-major) to out
   // (rows x k, column-major); tmp: rows x k.
   void download_cols(const double* src, uint64_t rows, int pitch, int k, double* tmp, double* out);
+  // The same for a few rows, false (nothing done) for more.
+  bool download_rows(const double* src, uint64_t rows, int pitch, int k, double* out, const int* place = nullptr);
   // G of the last sketches, rows [j0, j1) (current column order), and H / H1 / H2:
   // column-major FP64 with L columns.
   void download_g(uint64_t j0, uint64_t j1, double* G);

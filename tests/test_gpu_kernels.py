@@ -435,3 +435,36 @@ def test_permuted_loadings_take_no_device_memory():
         assert np.dot(r.V[:, c], proj[:, c]) / np.linalg.norm(proj[:, c]) >= 0.999
         tail = slice(m - 30000, m)  # past the first part
         assert np.corrcoef(r.V[tail, c], proj[tail, c])[0, 1] >= 0.99
+
+
+@pytest.mark.parametrize("L,rows", [(1, 6553), (1, 6554), (16, 1638), (16, 1639), (20, 1170), (20, 1171), (100, 256),
+                                    (100, 257)])
+def test_read_back_on_both_sides_of_the_direct_rows(ctx, L, rows):
+    """Reads of as many rows as are still transposed on the host, and of one more (rows (pitch + 4 k) about 131,072):
+    the same values as in a read of all."""
+    say(f"read back L={L} rows={rows}")
+    rng = np.random.default_rng(rows)
+    n, m = 150, 8000
+    ctx.upload_packed(pack(random_codes(rng, m, n, 0.0)), n)
+    ctx.standardize()
+    ctx.configure("fp64", L)
+    ctx.set_omega(rng.standard_normal((n, L)))
+    ctx.sketch(0, m, 0)
+    G = ctx.get_g(0, m, L)
+    np.testing.assert_array_equal(ctx.get_g(0, rows, L), G[:rows])
+    np.testing.assert_array_equal(ctx.get_g(m - rows, m, L), G[m - rows:])
+
+
+@pytest.mark.parametrize("m", [3640, 3641])
+def test_shuffled_loadings_on_both_sides_of_the_direct_rows(ctx, m):
+    """Loadings of a shuffled run, placed on the host (m (32 + 4) <= 131,072) and on the device."""
+    say(f"shuffled loadings m={m}")
+    n, k = 120, 1
+    rng = np.random.default_rng(m)
+    codes = random_codes(rng, m, n, 0.0)
+    codes[::2, : n // 3] = 0
+    ctx.upload_packed(pack(codes), n)
+    r = ctx.run(svd=2, k=k, oversamples=19, maxp=20, tol=1e-12, bands=8, precision="fp64", want_v=True)
+    A, _ = standardized(codes)
+    proj = A @ r.U
+    assert np.corrcoef(r.V[:, 0], proj[:, 0])[0, 1] >= 0.999
