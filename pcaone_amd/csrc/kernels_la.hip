@@ -201,14 +201,21 @@ __global__ void __launch_bounds__(256) k_make_pieces(const double* X, uint64_t n
   const int nr = (int)(rows_pad - r0 < (uint64_t)kEpiRows ? rows_pad - r0 : kEpiRows);
   double b4[4] = {0.0, 0.0, 0.0, 0.0};
   if (act) {
+    // F8: sl = the column's scale 2^se.  I8: the scale is sl 2^se, is = 1 / sl.  The
+    // exponents go through ldexp: the reciprocal of a whole scale may overflow.
     double cs[4] = {1.0, 1.0, 1.0, 1.0}, sl[4] = {1.0, 1.0, 1.0, 1.0}, is[4];
-    bool plain = true;  // the scales' reciprocals serve (a column near the ends of the FP64 range is divided)
+    int se[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       if (colsign) cs[q] = colsign[4 * cg + q];
-      if constexpr (F == Form::F8 || F == Form::I8) sl[q] = colscale[4 * cg + q];
-      is[q] = 1.0 / sl[q];
-      plain = plain && sl[q] >= 0x1p-900 && sl[q] <= 0x1p900;
+      if constexpr (F == Form::F8) {
+        sl[q] = colscale[4 * cg + q];
+        (void)frexp(sl[q], &se[q]);
+        --se[q];
+      } else if constexpr (F == Form::I8) {
+        sl[q] = frexp(colscale[4 * cg + q], &se[q]);
+        is[q] = 1.0 / sl[q];
+      }
     }
     for (int rb = rg; rb < nr; rb += kEpiBatch * RG) {
       double x[kEpiBatch][4], rs[kEpiBatch], w[kEpiBatch];
@@ -245,10 +252,11 @@ __global__ void __launch_bounds__(256) k_make_pieces(const double* X, uint64_t n
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           double y = x[u][q] * rs[u];
-          if constexpr (F == Form::F8) y = plain ? y * is[q] : y / sl[q];
-          if constexpr (F == Form::I8) y = plain ? quotient(y, sl[q], is[q]) : y / sl[q];
+          if constexpr (F == Form::F8) y = ldexp(y, -se[q]);
+          if constexpr (F == Form::I8) y = quotient(ldexp(y, -se[q]), sl[q], is[q]);
           w_t pc[P];
-          const double back = PF::make(y, sl[q], pc);
+          double back = PF::make(y, sl[q], pc);
+          if constexpr (F == Form::I8) back = ldexp(back, se[q]);
           rd[q] = live ? (rowscale ? quotient_any(back, rs[u], irs) : back) : 0.0;
           b4[q] += w[u] * rd[q];
 #pragma unroll
