@@ -121,6 +121,9 @@ void launch_packed_gemm(Form f, const GemmShape& g, const GemmArgs& a, hipStream
 // The FP32 form with the last, short block of columns in groups of 4: false
 // (nothing launched) unless the waves own 64 rows and ncols is 17..28 (lp 32)
 // or 33..40 (lp 48).  With one group less to save (41..44) the fragments spill.
+// plan_gemm knows neither this kernel nor the next: its row tiles, chunks and
+// occupancy are the padded kernel's, so that a product keeps its chunks, and with
+// them the order of its sums and its bits, whichever kernel takes it.
 bool launch_packed_gemm_f32_r4(const GemmShape& g, const GemmArgs& a, hipStream_t s);
 // The same for the FP64 form: ncols 17..28, 33..44 or 49..60 (any row tile:
 // 16 rows per wave, and every tile is a multiple of 64 rows).

@@ -127,9 +127,11 @@ __global__ void k_gather_rows(const uint32_t* __restrict__ in, uint64_t pitch, c
 
 // The code-01 entries of every row, in code order: one wave per row, 64 words
 // (1,024 codes) per step, each lane's place from an exclusive scan of the
-// lanes' counts.  Bound by the row reads (N M / 4 bytes).  One thread per row had
-// every load of a wave on 64 different rows: 6.67 ms per list of 20,011 x 200,003
-// codes, 1 % missing, against 0.62 ms now.
+// lanes' counts.  20,011 x 200,003 codes, 1 % missing: 0.62 ms per list, 1.6 TB/s of
+// row reads, a third of a copy's rate: each step's scan (six dependent lane
+// exchanges) and the lanes' scattered 4-byte stores stand between its load and the
+// next one's.  One thread per row had every load of a wave on 64 different rows:
+// 6.67 ms.
 __global__ void __launch_bounds__(256) k_missing_lists(const uint32_t* __restrict__ x, uint64_t pitch, uint64_t nrows,
                                                        uint64_t ncodes, const uint64_t* __restrict__ rp,
                                                        uint32_t* __restrict__ ix) {

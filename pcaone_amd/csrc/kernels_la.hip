@@ -175,10 +175,11 @@ __device__ __forceinline__ void store_pieces(const w_t* pt, int np, int lp, w_t*
 // pieces' sum / rowscale; in place over X allowed: every element is read and
 // written by the same thread), and the per-tile column sums of
 // w_r rounded[r][l] (w_r = bsc[r] (1/2 - bcf[r]), or 1 without bsc) in bpart.
-// Bound by memory where the rows fill the chip (1,000,000 x 80 as FP8: 469 us,
-// 1.5 GB, against about 580 with a division per value, exponents taken apart by frexp
-// and ldexp and one byte per store) and by a tile's own chain of loads where they
-// do not (10,000 x 40 as BF16: 7.3 us against 10.0 with a row at a time).
+// Bound by the conversions where the rows fill the chip (as FP8 about 150 VALU
+// instructions a value: 1,000,000 x 80 take 469 us, 1.5 GB at 3.2 TB/s, two thirds of
+// a copy's rate, against about 580 with a division per value, exponents taken apart
+// by frexp and ldexp and one byte per store) and by a tile's own chain of loads
+// where they do not (10,000 x 40 as BF16: 7.3 us against 10.0 with a row at a time).
 template <Form F>
 __global__ void __launch_bounds__(256) k_make_pieces(const double* X, uint64_t nreal, uint64_t rows_pad, int lp,
                                                      const double* __restrict__ rowscale,
@@ -940,10 +941,11 @@ __global__ void k_colmajor_to_rows(const double* __restrict__ src, uint64_t n, i
   }
 }
 
-// Row-major n x lp -> k columns of col_len values (row r at place[r] when given, else at r), 32 rows per workgroup
-// through LDS: whole rows read, 256-byte runs of each column written (one thread per output
-// value would read 8 bytes of every row line it touched).  Bound by HBM: 27 us
-// for 100,003 x 40 from lp = 48.
+// Row-major n x lp -> k columns of col_len values (row r at place[r] when given,
+// else at r), 32 rows per workgroup through LDS: whole rows read, 256-byte runs of
+// each column written (one thread per output value would read 8 bytes of every row
+// line it touched).  100,003 x 40 from lp = 48: 27 us, 2.6 TB/s read and written,
+// half of a copy's rate: a workgroup reads, waits, and writes 12 KB once.
 __global__ void __launch_bounds__(256) k_rows_to_colmajor(const double* __restrict__ src, uint64_t n, int lp, int k,
                                                           double* __restrict__ dst, uint64_t col_len,
                                                           const uint32_t* __restrict__ place) {
