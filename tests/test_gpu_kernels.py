@@ -401,7 +401,7 @@ def test_batch_read_back_takes_no_device_memory(ctx):
     assert np.all(first["status"] == 0)
     before = free_memory()
     got = [(ctx.batch_get_u(c), ctx.batch_get_v(c)) for c in range(3)]
-    assert free_memory() == before
+    assert free_memory() >= before
     for c in (2, 0, 1):
         np.testing.assert_array_equal(ctx.batch_get_v(c), got[c][1])
         np.testing.assert_array_equal(ctx.batch_get_u(c), got[c][0])
@@ -428,7 +428,7 @@ def test_permuted_loadings_take_no_device_memory():
         ctx.run(**kw)
         before = free_memory()
         r = ctx.run(want_v=True, **kw)
-        assert free_memory() == before
+        assert free_memory() >= before
     A, _ = standardized(codes)
     proj = A @ r.U
     for c in range(k):
